@@ -3,11 +3,11 @@
 // (loadcontrol.inl:55-57) / secant (pathfollowingfunctions.hh:188-195) displacement predictor, and
 // NewtonRaphson still has to reach the same ||R|| tolerance from the predicted state.
 //
-// Training products run through one tiled GEMM on v_mfma_f32_16x16x16bf16_1k: operands are rounded to BF16
-// (round to nearest even) while staged into LDS, accumulation is FP32, parameters keep an FP32 master copy
-// updated by Adam. Strided operand access covers every product of training: Z = A W^T + b (forward),
-// dW = dZ^T A (weight gradient, split over the batch), dA = dZ W (back-propagation). The prediction inside the
-// load loop runs in one fused kernel (features, four layers, update of u) on the same instruction and rounding.
+// Products run on the BF16 matrix instructions: operands rounded to BF16 (round to nearest even), FP32 accumulation,
+// parameters with an FP32 master copy updated by Adam. Training takes three launches per step: forward and backward of
+// the activations (mlpRows), the weight and bias gradients per batch slice (mlpWeightGrad), and their sum over the
+// slices with the Adam update (mlpFold). The prediction inside the load loop runs in one fused kernel (features, four
+// layers, update of u).
 //
 // Features of node v for the step n -> n+1 (load increment dlam, velocities v_n = du_n / dlam):
 //   [ X_v / L (3), t / 40 (3), lam_{n+1}, 40 dlam, v_n / 0.1 (3), v_{n-1} / 0.1 (3) ]
@@ -40,132 +40,299 @@ __device__ inline uint16_t toBf16(float f) { return __builtin_bit_cast(uint16_t,
 __device__ inline float sigmoid(float z) { return __builtin_amdgcn_rcpf(1.f + __expf(-z)); }
 __device__ inline float silu(float z) { return z * sigmoid(z); }
 
-// EPI_SILU_ONLY: C = silu(A B + bias), the pre-activation is not kept (inference)
-// EPI_PARTIAL: slice z of a K split stores its partial product at C + z * M * ldc (summed later in z order)
-enum { EPI_STORE = 0, EPI_PARTIAL = 1, EPI_BIAS_SILU = 2, EPI_BIAS = 3, EPI_SILU_ONLY = 4 };
+// ---- training and batched forward -----------------------------------------------------------------------------
+// One wavefront = 16 rows at a time, weights in LDS as BF16, every activation and every
+// pre-activation of a row in registers from the features to the loss gradient and back. Each layer is computed
+// transposed, out^T (outputs x 16 rows) = W act^T, with W as the MFMA A operand: lane (n, kq) = (lane & 15,
+// lane >> 4) then holds outputs 16 t + 4 kq + r of row n (C fragment of tile t), which is the B fragment of K step t
+// of the next layer on v_mfma_f32_16x16x16bf16_1k, in the natural order of the inputs, so no value moves between
+// lanes. The backward products dA^T = W^T dZ^T run the same way on a transposed copy of the weights. Operands are
+// rounded to BF16 (nearest even), K runs in steps of 16 in increasing order with FP32 accumulation, then the bias.
+// Bound: a batch of 8192 rows is 3.5 GFLOP over 512 wavefronts (half of one per SIMD), so latency (LDS fragment ->
+// MFMA -> SiLU chains) and the staging of the weights, not the matrix rate. Layer by layer through memory, the
+// forward and backward products, SiLU' and loss kernels of that batch took 11 launches and 116 us; this kernel takes
+// 24 us (26 with 4 wavefronts per workgroup in training: 8 stage the 140 KB of parameters faster).
+constexpr int kWr = kHid + 8;  // padded row of 128 BF16 values (68 dwords): the 16 rows of a fragment read spread over
+                               // the banks
+// LDS layout (BF16 values): W1 [128][16], W2, W3 [128][kWr], W4 [16][kWr] (rows past the 3 outputs zero), and for the
+// backward pass W2^T, W3^T [128][kWr], W4^T [128][16] (columns past 3 zero)
+constexpr int lW1 = 0, lW2 = lW1 + kHid * 16, lW3 = lW2 + kHid * kWr, lW4 = lW3 + kHid * kWr, lEndF = lW4 + 16 * kWr,
+              lT2 = lEndF, lT3 = lT2 + kHid * kWr, lT4 = lT3 + kHid * kWr, lEndB = lT4 + kHid * 16;
+static_assert(lEndB * 2 + (3 * kHid + 16) * 4 + 64 <= 160 * 1024, "weights and their transposes fit the LDS of a CU");
 
-// C[i][j] = sum_k A(i,k) B(k,j) with A(i,k) = A[i*sai + k*sak], B(k,j) = B[k*sbk + j*sbj].
-// 256 threads, 64x64 block tile, 4 waves of 32x32 (2x2 MFMA tiles), K in steps of 16.
-// gridDim.z splits K into chunks of kChunk (EPI_PARTIAL: one partial product per chunk).
-template <int EPI>
-__global__ __launch_bounds__(256) void gemmBf16(int M, int N, int K, const float* __restrict__ A, int64_t sai,
-                                                int64_t sak, const float* __restrict__ B, int64_t sbk, int64_t sbj,
-                                                float* __restrict__ C, int64_t ldc, const float* __restrict__ bias,
-                                                float* __restrict__ act, int kChunk) {
-  __shared__ uint16_t As[64][20];  // row i, k (padded)
-  __shared__ uint16_t Bs[16][68];  // k, col j (padded)
+__device__ inline bf16x4 pack4(float a, float b, float c, float d) {
+  return bf16x4{(short)toBf16(a), (short)toBf16(b), (short)toBf16(c), (short)toBf16(d)};
+}
+// four consecutive BF16 values of a weight row in LDS (8-byte aligned): a 16x16x16 A fragment
+__device__ inline bf16x4 wfrag(const uint16_t* w) { return *reinterpret_cast<const bf16x4*>(w); }
+
+// acc[t] = tile t of W act^T for T output tiles: W rows of `ld` values in LDS, KS steps of 16 inputs
+template <int T, int KS>
+__device__ inline void layerT(const uint16_t* W, int ld, int n, int kq, const bf16x4* act, f32x4* acc) {
+  // keeps the fragment reads here (hoisted out of the row loop they would spill hundreds of registers)
+  asm volatile("" ::: "memory");
+#pragma unroll
+  for (int t = 0; t < T; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int s = 0; s < KS; ++s)
+#pragma unroll
+    for (int t = 0; t < T; ++t)
+      acc[t] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(wfrag(W + (16 * t + n) * ld + 16 * s + 4 * kq), act[s], acc[t],
+                                                         0, 0, 0);
+}
+
+// BACK: the hidden activations A[l] and the gradients dZ[l] (n x 128) and dY (n x 3) go to memory for the weight
+// gradients, with the workgroup's sum of (y - t)^2 in partial[blockIdx.x]. Otherwise only the outputs y (n x 3).
+template <bool BACK>
+__global__ __launch_bounds__(BACK ? 512 : 256) void mlpRows(const float* __restrict__ P, const float* __restrict__ X,
+                                                             const float* __restrict__ Tg, int64_t n, float scale,
+                                                             float* __restrict__ Y, float* __restrict__ A0,
+                                                             float* __restrict__ A1, float* __restrict__ A2,
+                                                             float* __restrict__ D0, float* __restrict__ D1,
+                                                             float* __restrict__ D2, float* __restrict__ dY,
+                                                             double* __restrict__ partial) {
+  constexpr int BS = BACK ? 512 : 256;
+  __shared__ __align__(16) uint16_t sW[BACK ? lEndB : lEndF];
+  __shared__ float sB[3 * kHid + 16];
+  __shared__ double red[BS / 64];
+  const int tid = threadIdx.x;
+  for (int i = tid; i < kHid * 16; i += BS) {
+    const int j = i >> 4, k = i & 15;
+    sW[lW1 + i] = toBf16(k < kIn ? P[oW1 + j * kIn + k] : 0.f);
+    if constexpr (BACK) sW[lT4 + i] = toBf16(k < kOut ? P[oW4 + k * kHid + j] : 0.f);
+  }
+  for (int i = tid; i < 16 * kHid; i += BS) {
+    const int j = i >> 7, k = i & 127;
+    sW[lW4 + j * kWr + k] = toBf16(j < kOut ? P[oW4 + j * kHid + k] : 0.f);
+  }
+#pragma unroll 4
+  for (int i = tid; i < kHid * kHid / 4; i += BS) {  // four inputs of one output at a time
+    const int j = i >> 5, k = 4 * (i & 31);
+    const float* w2 = P + oW2 + j * kHid + k;
+    const float* w3 = P + oW3 + j * kHid + k;
+    *reinterpret_cast<bf16x4*>(&sW[lW2 + j * kWr + k]) = pack4(w2[0], w2[1], w2[2], w2[3]);
+    *reinterpret_cast<bf16x4*>(&sW[lW3 + j * kWr + k]) = pack4(w3[0], w3[1], w3[2], w3[3]);
+  }
+  if constexpr (BACK) {
+#pragma unroll 4
+    for (int i = tid; i < kHid * kHid / 4; i += BS) {  // four outputs of one input, for the transposes
+      const int k = i & 127, j = 4 * (i >> 7);
+      const float* w2 = P + oW2 + j * kHid + k;
+      const float* w3 = P + oW3 + j * kHid + k;
+      *reinterpret_cast<bf16x4*>(&sW[lT2 + k * kWr + j]) = pack4(w2[0], w2[kHid], w2[2 * kHid], w2[3 * kHid]);
+      *reinterpret_cast<bf16x4*>(&sW[lT3 + k * kWr + j]) = pack4(w3[0], w3[kHid], w3[2 * kHid], w3[3 * kHid]);
+    }
+  }
+  for (int i = tid; i < 3 * kHid + 16; i += BS) {
+    float v = 0.f;
+    if (i < kHid) v = P[oB1 + i];
+    else if (i < 2 * kHid) v = P[oB2 + i - kHid];
+    else if (i < 3 * kHid) v = P[oB3 + i - 2 * kHid];
+    else if (i - 3 * kHid < kOut) v = P[oB4 + i - 3 * kHid];
+    sB[i] = v;
+  }
+  __syncthreads();
+  const int lane = tid & 63, nl = lane & 15, kq = lane >> 4;
+  double sq = 0.0;
+  for (int64_t r0 = ((int64_t)blockIdx.x + (int64_t)gridDim.x * (tid >> 6)) * 16; r0 < n;
+       r0 += (int64_t)gridDim.x * (BS / 4)) {
+    const int64_t v  = r0 + nl;
+    const bool valid = v < n;
+    float f[4] = {0.f, 0.f, 0.f, 0.f};
+    if (valid)
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        if (4 * kq + q < kIn) f[q] = X[v * kIn + 4 * kq + q];
+    bf16x4 act[8];
+    f32x4 Z[3][8], acc[8];
+    act[0] = pack4(f[0], f[1], f[2], f[3]);
+    // pre-activation, SiLU, the next layer's B fragments (and the activations to memory)
+    auto activate = [&](int l, float* Al) {
+#pragma unroll
+      for (int t = 0; t < 8; ++t) {
+        f32x4 a;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          Z[l][t][r] = acc[t][r] + sB[l * kHid + 16 * t + 4 * kq + r];
+          a[r]       = silu(Z[l][t][r]);
+        }
+        act[t] = pack4(a[0], a[1], a[2], a[3]);
+        if constexpr (BACK)
+          if (valid) *reinterpret_cast<f32x4*>(&Al[v * kHid + 16 * t + 4 * kq]) = a;
+      }
+    };
+    layerT<8, 1>(sW + lW1, 16, nl, kq, act, acc);
+    activate(0, A0);
+    layerT<8, 8>(sW + lW2, kWr, nl, kq, act, acc);
+    activate(1, A1);
+    layerT<8, 8>(sW + lW3, kWr, nl, kq, act, acc);
+    activate(2, A2);
+    layerT<1, 8>(sW + lW4, kWr, nl, kq, act, acc);
+    // lanes kq = 0 hold the outputs 0..2 of row n
+    const bool out = valid && kq == 0;
+    float g[3] = {0.f, 0.f, 0.f};
+    if (out) {
+#pragma unroll
+      for (int k = 0; k < kOut; ++k) {
+        const float y = acc[0][k] + sB[3 * kHid + k];
+        if constexpr (BACK) {
+          const float d = y - Tg[v * kOut + k];
+          g[k]          = 2.f * d * scale;
+          sq += (double)d * d;
+          dY[v * kOut + k] = g[k];
+        } else {
+          Y[v * kOut + k] = y;
+        }
+      }
+    }
+    if constexpr (BACK) {
+      act[0] = pack4(g[0], g[1], g[2], 0.f);
+      // dZ = dA silu'(Z), the B fragments of the next product (and dZ to memory)
+      auto gradient = [&](int l, float* Dl) {
+#pragma unroll
+        for (int t = 0; t < 8; ++t) {
+          f32x4 d;
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const float z = Z[l][t][r], sg = sigmoid(z);
+            d[r]          = acc[t][r] * sg * (1.f + z * (1.f - sg));
+          }
+          act[t] = pack4(d[0], d[1], d[2], d[3]);
+          if (valid) *reinterpret_cast<f32x4*>(&Dl[v * kHid + 16 * t + 4 * kq]) = d;
+        }
+      };
+      layerT<8, 1>(sW + lT4, 16, nl, kq, act, acc);
+      gradient(2, D2);
+      layerT<8, 8>(sW + lT3, kWr, nl, kq, act, acc);
+      gradient(1, D1);
+      layerT<8, 8>(sW + lT2, kWr, nl, kq, act, acc);
+      gradient(0, D0);
+    }
+  }
+  if constexpr (BACK) {
+    for (int o = 32; o > 0; o >>= 1) sq += __shfl_xor(sq, o, 64);
+    if (lane == 0) red[tid >> 6] = sq;
+    __syncthreads();
+    if (tid == 0) {
+      double t = red[0];
+#pragma unroll
+      for (int w = 1; w < BS / 64; ++w) t += red[w];
+      partial[blockIdx.x] = t;
+    }
+  }
+}
+
+// Weight and bias gradients of all four layers over one slice of the batch: dW_l = dZ_l^T A_{l-1}, db_l = column sums
+// of dZ_l, into slice blockIdx.y of part (kParams values, laid out as the parameters). blockIdx.x = one 64 x 64 tile of
+// one product (kGradTiles of them): 4 wavefronts of 32 x 32. kRowsStep rows of both operands (64 columns each) are
+// loaded at once (lanes along the columns, four rows per thread and step), rounded to BF16 and stored row-packed, so
+// that an MFMA fragment (four rows of one column) is one 8-byte LDS read. Bound by the latency of those loads: 12 x 32
+// workgroups for 8192 rows, two load rounds each, 12 us for
+// 8192 rows (27 with every load guarded; 318 for the products and column sums of one launch per layer before).
+constexpr int kGradTiles = 12;    // 128x128 (W3, W2): 4 each; 3x128 (W4), 128x14 (W1): 2 each
+constexpr int kRowsStep  = 128;
+constexpr int kGs = kRowsStep + 4;  // padded column (66 dwords)
+__global__ __launch_bounds__(256) void mlpWeightGrad(const float* __restrict__ X, const float* __restrict__ A0,
+                                                     const float* __restrict__ A1, const float* __restrict__ A2,
+                                                     const float* __restrict__ D0, const float* __restrict__ D1,
+                                                     const float* __restrict__ D2, const float* __restrict__ dY,
+                                                     int64_t n, int64_t chunk, float* __restrict__ part) {
+  __shared__ __align__(16) uint16_t As[64 * kGs], Bs[64 * kGs];
+  __shared__ float sb[4][64];
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  const int wm = w >> 1, wn = w & 1;
-  const int i0 = blockIdx.y * 64, j0 = blockIdx.x * 64;
-  const int kb = blockIdx.z * kChunk, ke = min(K, kb + kChunk);
+  const int tile = blockIdx.x;
+  const float *D, *A;
+  int M, N, i0, j0;
+  int64_t oW, oB;
+  if (tile < 4) {
+    D = D2, A = A1, M = kHid, N = kHid, i0 = 64 * (tile >> 1), j0 = 64 * (tile & 1), oW = oW3, oB = oB3;
+  } else if (tile < 8) {
+    D = D1, A = A0, M = kHid, N = kHid, i0 = 64 * ((tile - 4) >> 1), j0 = 64 * (tile & 1), oW = oW2, oB = oB2;
+  } else if (tile < 10) {
+    D = dY, A = A2, M = kOut, N = kHid, i0 = 0, j0 = 64 * (tile & 1), oW = oW4, oB = oB4;
+  } else {
+    D = D0, A = X, M = kHid, N = kIn, i0 = 64 * (tile & 1), j0 = 0, oW = oW1, oB = oB1;
+  }
+  const int64_t k0 = (int64_t)blockIdx.y * chunk, k1 = k0 + chunk < n ? k0 + chunk : n;
+  const bool ci = i0 + lane < M, cj = j0 + lane < N;
   f32x4 acc[2][2];
 #pragma unroll
   for (int a = 0; a < 2; ++a)
 #pragma unroll
     for (int b = 0; b < 2; ++b) acc[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
-  for (int k0 = kb; k0 < ke; k0 += 16) {
+  const int wm = w >> 1, wn = w & 1;
+  float bsum = 0.f;
+  for (int64_t kb = k0; kb < k1; kb += kRowsStep) {
+    // wavefront w loads rows 4 (4 q + w) .. + 3 of column `lane` of both operands
+    float va[kRowsStep / 16][4], vb[kRowsStep / 16][4];
+    const float* d = D + (kb + 4 * w) * M + i0 + lane;
+    const float* a = A + (kb + 4 * w) * N + j0 + lane;
+    auto load = [&](auto guarded) {
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int e = tid * 4 + q;
-      const int r = e >> 4, kk = e & 15;
-      const int gi = i0 + r, gk = k0 + kk;
-      As[r][kk] = toBf16((gi < M && gk < ke) ? A[(int64_t)gi * sai + (int64_t)gk * sak] : 0.f);
-      const int kb2 = e >> 6, cc = e & 63;
-      const int gk2 = k0 + kb2, gj = j0 + cc;
-      Bs[kb2][cc] = toBf16((gj < N && gk2 < ke) ? B[(int64_t)gk2 * sbk + (int64_t)gj * sbj] : 0.f);
+      for (int q = 0; q < kRowsStep / 16; ++q)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const bool in = !decltype(guarded)::value || kb + 4 * w + 16 * q + r < k1;
+          va[q][r]      = (!decltype(guarded)::value || (ci && in)) ? d[(16 * q + r) * M] : 0.f;
+          vb[q][r]      = (!decltype(guarded)::value || (cj && in)) ? a[(16 * q + r) * N] : 0.f;
+        }
+    };
+    if (tile < 8 && kb + kRowsStep <= k1)  // whole tiles of the 128x128 products
+      load(std::false_type{});
+    else
+      load(std::true_type{});
+    if (kb > k0) __syncthreads();  // the previous step's fragments have been read
+#pragma unroll
+    for (int q = 0; q < kRowsStep / 16; ++q) {
+      *reinterpret_cast<bf16x4*>(&As[lane * kGs + 4 * (4 * q + w)]) = pack4(va[q][0], va[q][1], va[q][2], va[q][3]);
+      *reinterpret_cast<bf16x4*>(&Bs[lane * kGs + 4 * (4 * q + w)]) = pack4(vb[q][0], vb[q][1], vb[q][2], vb[q][3]);
+      bsum += (va[q][0] + va[q][1]) + (va[q][2] + va[q][3]);
     }
     __syncthreads();
 #pragma unroll
-    for (int mi = 0; mi < 2; ++mi) {
-      bf16x4 av;
-      const int ar = wm * 32 + mi * 16 + (lane & 15);
+    for (int s = 0; s < kRowsStep / 16; ++s) {
+      bf16x4 a[2], b[2];
 #pragma unroll
-      for (int q = 0; q < 4; ++q) av[q] = (short)As[ar][4 * (lane >> 4) + q];
-#pragma unroll
-      for (int nj = 0; nj < 2; ++nj) {
-        bf16x4 bv;
-        const int bc = wn * 32 + nj * 16 + (lane & 15);
-#pragma unroll
-        for (int q = 0; q < 4; ++q) bv[q] = (short)Bs[4 * (lane >> 4) + q][bc];
-        acc[mi][nj] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(av, bv, acc[mi][nj], 0, 0, 0);
+      for (int m = 0; m < 2; ++m) {
+        a[m] = wfrag(&As[(32 * wm + 16 * m + (lane & 15)) * kGs + 16 * s + 4 * (lane >> 4)]);
+        b[m] = wfrag(&Bs[(32 * wn + 16 * m + (lane & 15)) * kGs + 16 * s + 4 * (lane >> 4)]);
       }
+#pragma unroll
+      for (int m = 0; m < 2; ++m)
+#pragma unroll
+        for (int q = 0; q < 2; ++q) acc[m][q] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a[m], b[q], acc[m][q], 0, 0, 0);
     }
-    __syncthreads();
   }
+  float* out = part + (int64_t)blockIdx.y * kParams;
 #pragma unroll
-  for (int mi = 0; mi < 2; ++mi)
+  for (int m = 0; m < 2; ++m)
 #pragma unroll
-    for (int nj = 0; nj < 2; ++nj)
+    for (int q = 0; q < 2; ++q)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const int i = i0 + wm * 32 + mi * 16 + 4 * (lane >> 4) + r;
-        const int j = j0 + wn * 32 + nj * 16 + (lane & 15);
-        if (i >= M || j >= N) continue;
-        float v = acc[mi][nj][r];
-        if constexpr (EPI == EPI_PARTIAL) {
-          C[(int64_t)blockIdx.z * M * ldc + (int64_t)i * ldc + j] = v;
-        } else {
-          if constexpr (EPI == EPI_BIAS_SILU || EPI == EPI_BIAS || EPI == EPI_SILU_ONLY) v += bias[j];
-          if constexpr (EPI == EPI_SILU_ONLY) {
-            C[(int64_t)i * ldc + j] = silu(v);
-          } else {
-            C[(int64_t)i * ldc + j] = v;
-          }
-          if constexpr (EPI == EPI_BIAS_SILU) act[(int64_t)i * ldc + j] = silu(v);
-        }
+        const int i = i0 + 32 * wm + 16 * m + 4 * (lane >> 4) + r, j = j0 + 32 * wn + 16 * q + (lane & 15);
+        if (i < M && j < N) out[oW + (int64_t)i * N + j] = acc[m][q][r];
       }
-}
-
-// dZ = dA * silu'(Z)
-__global__ void siluBackward(const float* __restrict__ dA, const float* __restrict__ Z, float* __restrict__ dZ,
-                             int64_t n) {
-  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) {
-    const float z = Z[i], sg = sigmoid(z);
-    dZ[i]         = dA[i] * sg * (1.f + z * (1.f - sg));
+  if (j0 == 0) {  // the tiles of the first columns also own the bias gradient of their rows
+    sb[w][lane] = bsum;
+    __syncthreads();
+    if (w == 0 && ci) out[oB + i0 + lane] = ((sb[0][lane] + sb[1][lane]) + sb[2][lane]) + sb[3][lane];
   }
 }
 
-// dY = 2 (Y - T) / (3 n); per-block partial sums of (Y - T)^2
-__global__ void mseGrad(const float* __restrict__ Y, const float* __restrict__ T, int64_t n3, float scale,
-                        float* __restrict__ dY, double* __restrict__ partial) {
-  __shared__ double red[4];
-  double s = 0.0;
-  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n3; i += (int64_t)gridDim.x * 256) {
-    const float d = Y[i] - T[i];
-    dY[i]         = 2.f * d * scale;
-    s += (double)d * d;
-  }
-  for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
-  __syncthreads();
-  if (threadIdx.x == 0) partial[blockIdx.x] = red[0] + red[1] + red[2] + red[3];
-}
-
-// db[j] += sum over rows of dZ (one block per 256-row slab, one thread per column)
-// column sums of 256-row slices of dZ: part[slice * cols + j]
-__global__ void biasGrad(const float* __restrict__ dZ, int64_t n, int cols, float* __restrict__ part) {
-  const int j = threadIdx.x;
-  if (j >= cols) return;
-  const int64_t r0 = (int64_t)blockIdx.x * 256, r1 = min<int64_t>(n, r0 + 256);
-  float s = 0.f;
-  for (int64_t r = r0; r < r1; ++r) s += dZ[r * cols + j];
-  part[(int64_t)blockIdx.x * cols + j] = s;
-}
-
-// out[i] = sum over z = 0 .. nz-1 of part[z * len + i], in that order: the gradients do not depend on scheduling
-__global__ void foldSlices(const float* __restrict__ part, int nz, int64_t len, float* __restrict__ out) {
-  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < len; i += (int64_t)gridDim.x * 256) {
-    float s = 0.f;
-    for (int z = 0; z < nz; ++z) s += part[(int64_t)z * len + i];
-    out[i] = s;
-  }
-}
-
-__global__ void adamKernel(float* __restrict__ p, const float* __restrict__ g, float* __restrict__ m,
-                           float* __restrict__ v, int64_t n, float lr, float b1, float b2, float eps, float c1,
-                           float c2) {
-  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) {
-    const float gi = g[i];
+// g[i] = sum over the slices z = 0 .. nz-1 of part[z * kParams + i], in that order (the gradients do not depend on
+// scheduling); ADAM: then one Adam step on the parameters
+template <bool ADAM>
+__global__ __launch_bounds__(256) void mlpFold(const float* __restrict__ part, int nz, float* __restrict__ g,
+                                               float* __restrict__ p, float* __restrict__ m, float* __restrict__ v,
+                                               float lr, float b1, float b2, float eps, float c1, float c2) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= kParams) return;
+  float gi = 0.f;
+#pragma unroll 8
+  for (int z = 0; z < nz; ++z) gi += part[(int64_t)z * kParams + i];
+  g[i] = gi;
+  if constexpr (ADAM) {
     const float mi = b1 * m[i] + (1.f - b1) * gi;
     const float vi = b2 * v[i] + (1.f - b2) * gi * gi;
     m[i]           = mi;
@@ -209,8 +376,7 @@ __global__ void packBf16Weights(const float* __restrict__ P, uint16_t* __restric
   Wb[i] = toBf16(v);
 }
 
-// four (eight) consecutive BF16 values of a weight row in LDS, 8- (16-) byte aligned: an MFMA A fragment
-__device__ inline bf16x4 wfrag(const uint16_t* w) { return *reinterpret_cast<const bf16x4*>(w); }
+// eight consecutive BF16 values of a weight row in LDS (16-byte aligned): a 16x16x32 A fragment
 __device__ inline bf16x8 wfrag8(const uint16_t* w) { return *reinterpret_cast<const bf16x8*>(w); }
 // the 16x16x32 B fragment of K step s: this lane's outputs of tiles 2 s and 2 s + 1
 __device__ inline bf16x8 actPair(bf16x4 lo, bf16x4 hi) {
@@ -226,7 +392,7 @@ __device__ inline bf16x8 actPair(bf16x4 lo, bf16x4 hi) {
 // step s takes from this lane exactly its outputs of tiles 2 s and 2 s + 1 (the weight columns are stored in
 // that order): no data moves between lanes from layer to layer. The 8 output tiles of a layer are independent
 // accumulation chains, interleaved per K step. Same operand rounding (BF16, round to nearest even), FP32
-// accumulation, bias and SiLU as the layer-by-layer GEMMs (within a 32-input step the summation order differs).
+// accumulation, bias and SiLU as mlpRows (within a 32-input step the summation order differs).
 __global__ __launch_bounds__(256) void mlpPredictFused(const uint16_t* __restrict__ Wb, const float* __restrict__ P,
                                                        const double* __restrict__ X, const double* __restrict__ duN,
                                                        const double* __restrict__ duN1, int64_t nn, double invL,
@@ -337,8 +503,8 @@ inline unsigned g1(int64_t n) { return (unsigned)std::min<int64_t>(std::max<int6
 struct Mlp {
   hipStream_t s = nullptr;
   int64_t maxBatch = 0;
-  DevBuf<float> P, G, Mo, Vo;          // params (fp32 master), grads, Adam moments
-  DevBuf<float> Z[3], Aa[3], Y, dY, dA, dZ, Xin, Tin;
+  DevBuf<float> P, G, Mo, Vo;      // params (fp32 master), grads, Adam moments
+  DevBuf<float> Aa[3], dZ[3], Y, dY, Xin, Tin;
   DevBuf<float> Gpart;  // per-slice partial gradients, folded in a fixed order
   DevBuf<uint16_t> Wb;  // BF16 weights of the fused predictor (packed when the parameters are set)
   DevBuf<double> partial;
@@ -350,92 +516,51 @@ struct Mlp {
     if (n <= maxBatch) return;
     maxBatch = n;
     for (int l = 0; l < 3; ++l) {
-      Z[l].ensure(n * kHid);
       Aa[l].ensure(n * kHid);
+      dZ[l].ensure(n * kHid);
     }
     Y.ensure(n * kOut);
     dY.ensure(n * kOut);
-    dA.ensure(n * kHid);
-    dZ.ensure(n * kHid);
     Xin.ensure(n * kIn);
     Tin.ensure(n * kOut);
   }
 
-  // returns the number of K slices (gridDim.z)
-  template <int EPI>
-  int gemm(int M, int N, int K, const float* A, int64_t sai, int64_t sak, const float* B, int64_t sbk, int64_t sbj,
-           float* C, int64_t ldc, const float* bias, float* act, int splitK = 1) {
-    const int kChunk = splitK > 1 ? ((K + splitK - 1) / splitK + 15) / 16 * 16 : K;
-    const int nz     = splitK > 1 ? (K + kChunk - 1) / kChunk : 1;
-    dim3 grid((N + 63) / 64, (M + 63) / 64, nz);
-    hipLaunchKernelGGL((gemmBf16<EPI>), grid, dim3(256), 0, s, M, N, K, A, sai, sak, B, sbk, sbj, C, ldc, bias, act,
-                       kChunk);
-    return nz;
+  // y (n x 3) = the network on x (n x 14); nothing is kept and nothing is allocated
+  void forward(const float* x, int64_t n, float* y) {
+    const unsigned grid = (unsigned)std::min<int64_t>((n + 63) / 64, 512);  // 2 workgroups of 80 KB LDS per CU
+    hipLaunchKernelGGL((mlpRows<false>), dim3(grid), dim3(256), 0, s, P.p, x, nullptr, n, 0.f, y, nullptr, nullptr,
+                       nullptr, nullptr, nullptr, nullptr, nullptr, nullptr);
   }
 
-  // forward on x (n x 14) -> Y (n x 3), keeping Z/A for the backward pass
-  void forward(const float* x, int64_t n) {
-    const float* P0 = P.p;
-    gemm<EPI_BIAS_SILU>((int)n, kHid, kIn, x, kIn, 1, P0 + oW1, 1, kIn, Z[0].p, kHid, P0 + oB1, Aa[0].p);
-    gemm<EPI_BIAS_SILU>((int)n, kHid, kHid, Aa[0].p, kHid, 1, P0 + oW2, 1, kHid, Z[1].p, kHid, P0 + oB2, Aa[1].p);
-    gemm<EPI_BIAS_SILU>((int)n, kHid, kHid, Aa[1].p, kHid, 1, P0 + oW3, 1, kHid, Z[2].p, kHid, P0 + oB3, Aa[2].p);
-    gemm<EPI_BIAS>((int)n, kOut, kHid, Aa[2].p, kHid, 1, P0 + oW4, 1, kHid, Y.p, kOut, P0 + oB4, nullptr);
-  }
-
-  // the same forward through caller-provided buffers: hidden activations ping-pong between a and b (n x 128
-  // each), the output goes to y (n x 3); no pre-activations are kept and nothing is allocated
-  void forwardInto(const float* x, int64_t n, float* a, float* b, float* y) {
-    const float* P0 = P.p;
-    gemm<EPI_SILU_ONLY>((int)n, kHid, kIn, x, kIn, 1, P0 + oW1, 1, kIn, a, kHid, P0 + oB1, nullptr);
-    gemm<EPI_SILU_ONLY>((int)n, kHid, kHid, a, kHid, 1, P0 + oW2, 1, kHid, b, kHid, P0 + oB2, nullptr);
-    gemm<EPI_SILU_ONLY>((int)n, kHid, kHid, b, kHid, 1, P0 + oW3, 1, kHid, a, kHid, P0 + oB3, nullptr);
-    gemm<EPI_BIAS>((int)n, kOut, kHid, a, kHid, 1, P0 + oW4, 1, kHid, y, kOut, P0 + oB4, nullptr);
-  }
-
-  // mean-squared-error loss and its gradient w.r.t. all parameters (into G)
-  double lossGrad(const float* x, const float* t, int64_t n) {
-    forward(x, n);
-    const int nb = (int)std::min<int64_t>((n * kOut + 255) / 256, 1024);
-    partial.ensure(1024);
-    hipLaunchKernelGGL(mseGrad, dim3(nb), dim3(256), 0, s, Y.p, t, n * kOut, (float)(1.0 / (double)(n * kOut)), dY.p,
-                       partial.p);
-    const int split = (int)std::max<int64_t>(1, std::min<int64_t>(n / 256, 256));
-    const unsigned nbias = (unsigned)((n + 255) / 256);
-    Gpart.ensure(std::max<int64_t>((int64_t)split * kHid * kHid, (int64_t)nbias * kHid));
-    // dW (M x N) = dZ^T A over the batch: one partial product per batch slice, folded in slice order
-    auto weightGrad = [&](int M, int N, const float* dz, const float* ain, float* dst) {
-      const int nz = gemm<EPI_PARTIAL>(M, N, (int)n, dz, 1, M, ain, N, 1, Gpart.p, N, nullptr, nullptr, split);
-      hipLaunchKernelGGL(foldSlices, dim3(g1((int64_t)M * N)), dim3(256), 0, s, Gpart.p, nz, (int64_t)M * N, dst);
-    };
-    auto biasGradient = [&](const float* dz, int cols, float* dst) {
-      hipLaunchKernelGGL(biasGrad, dim3(nbias), dim3(kHid), 0, s, dz, n, cols, Gpart.p);
-      hipLaunchKernelGGL(foldSlices, dim3(g1(cols)), dim3(256), 0, s, Gpart.p, (int)nbias, (int64_t)cols, dst);
-    };
-    // layer 4: dW4 = dY^T A3, db4, dA3 = dY W4
-    weightGrad(kOut, kHid, dY.p, Aa[2].p, G.p + oW4);
-    biasGradient(dY.p, kOut, G.p + oB4);
-    gemm<EPI_STORE>((int)n, kHid, kOut, dY.p, kOut, 1, P.p + oW4, kHid, 1, dA.p, kHid, nullptr, nullptr);
-    for (int l = 2; l >= 0; --l) {
-      hipLaunchKernelGGL(siluBackward, dim3(g1(n * kHid)), dim3(256), 0, s, dA.p, Z[l].p, dZ.p, n * kHid);
-      const float* ain = l == 0 ? x : Aa[l - 1].p;
-      const int kin    = l == 0 ? kIn : kHid;
-      const int64_t oW = l == 0 ? oW1 : (l == 1 ? oW2 : oW3), oB = l == 0 ? oB1 : (l == 1 ? oB2 : oB3);
-      weightGrad(kHid, kin, dZ.p, ain, G.p + oW);
-      biasGradient(dZ.p, kHid, G.p + oB);
-      if (l > 0) gemm<EPI_STORE>((int)n, kHid, kHid, dZ.p, kHid, 1, P.p + oW, kin, 1, dA.p, kHid, nullptr, nullptr);
+  // mean-squared-error loss and its gradient w.r.t. all parameters (into G); train: then one Adam step
+  double lossGrad(const float* x, const float* t, int64_t n, bool train = false, float lr = 0.f) {
+    const int nb = (int)std::min<int64_t>((n + 63) / 64, 256);  // one workgroup of 156 KB LDS per CU
+    partial.ensure(256);
+    hipLaunchKernelGGL((mlpRows<true>), dim3(nb), dim3(512), 0, s, P.p, x, t, n, (float)(1.0 / (double)(n * kOut)),
+                       nullptr, Aa[0].p, Aa[1].p, Aa[2].p, dZ[0].p, dZ[1].p, dZ[2].p, dY.p, partial.p);
+    // slices of 256 rows, at most 256 of them
+    const int64_t split = std::max<int64_t>(1, std::min<int64_t>(n / 256, 256));
+    const int64_t chunk = split > 1 ? ((n + split - 1) / split + 15) / 16 * 16 : n;
+    const int nz        = (int)((n + chunk - 1) / chunk);
+    Gpart.ensure((size_t)nz * kParams);
+    hipLaunchKernelGGL(mlpWeightGrad, dim3(kGradTiles, nz), dim3(256), 0, s, x, Aa[0].p, Aa[1].p, Aa[2].p, dZ[0].p,
+                       dZ[1].p, dZ[2].p, dY.p, n, chunk, Gpart.p);
+    const dim3 gf((unsigned)((kParams + 255) / 256));
+    if (train) {
+      const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
+      ++step;
+      const float c1 = 1.f / (1.f - std::pow(b1, (float)step)), c2 = 1.f / (1.f - std::pow(b2, (float)step));
+      hipLaunchKernelGGL((mlpFold<true>), gf, dim3(256), 0, s, Gpart.p, nz, G.p, P.p, Mo.p, Vo.p, lr, b1, b2, eps, c1,
+                         c2);
+    } else {
+      hipLaunchKernelGGL((mlpFold<false>), gf, dim3(256), 0, s, Gpart.p, nz, G.p, nullptr, nullptr, nullptr, 0.f, 0.f,
+                         0.f, 0.f, 0.f, 0.f);
     }
     IK_HIP(hipMemcpyAsync(hred, partial.p, nb * sizeof(double), hipMemcpyDeviceToHost, s));
     IK_HIP(hipStreamSynchronize(s));
     double sum = 0.0;
     for (int i = 0; i < nb; ++i) sum += hred[i];
     return sum / (double)(n * kOut);
-  }
-
-  void adam(float lr, float b1, float b2, float eps) {
-    ++step;
-    const float c1 = 1.f / (1.f - std::pow(b1, (float)step)), c2 = 1.f / (1.f - std::pow(b2, (float)step));
-    hipLaunchKernelGGL(adamKernel, dim3(g1(kParams)), dim3(256), 0, s, P.p, G.p, Mo.p, Vo.p, kParams, lr, b1, b2, eps,
-                       c1, c2);
   }
 };
 
@@ -448,7 +573,7 @@ Mlp* mlpCreate(hipStream_t s) {
   m->Vo.ensure(kParams);
   hipLaunchKernelGGL(fillF, dim3(g1(kParams)), dim3(256), 0, s, m->Mo.p, kParams, 0.f);
   hipLaunchKernelGGL(fillF, dim3(g1(kParams)), dim3(256), 0, s, m->Vo.p, kParams, 0.f);
-  IK_HIP(hipHostMalloc((void**)&m->hred, 1024 * sizeof(double), hipHostMallocDefault));
+  IK_HIP(hipHostMalloc((void**)&m->hred, 256 * sizeof(double), hipHostMallocDefault));
   return m;
 }
 
@@ -502,11 +627,11 @@ struct ik_mlp {
   std::string err;
 };
 
-// Scratch of the allocation-free forward (ik_mlp_forward_noalloc): two ping-pong buffers of hidden activations,
-// IK_MLP_NOALLOC_MAX_ROWS x 128 FP32 each (8 MiB), one copy per device held until the process ends. Host code
-// uses only the address hipGetSymbolAddress returns for the device (the array's name on the host is not a device
-// address), resolved once per device at ik_mlp_create with that device current.
-static __device__ __align__(256) float scratch[2 * IK_MLP_NOALLOC_MAX_ROWS * ik::kHid];
+// Scratch of the allocation-free forward (ik_mlp_forward_noalloc): the outputs of a call whose y overlaps its x (the
+// kernel's workgroups read x while others write y), IK_MLP_NOALLOC_MAX_ROWS x 3 FP32, one copy per device held until the
+// process ends. Host code uses only the address hipGetSymbolAddress returns for the device (the array's name on the
+// host is not a device address), resolved once per device at ik_mlp_create with that device current.
+static __device__ __align__(256) float scratch[IK_MLP_NOALLOC_MAX_ROWS * ik::kOut];
 
 namespace {
 constexpr int kMaxDevices = 64;
@@ -616,7 +741,7 @@ int ik_mlp_forward(ik_mlp* m, const float* x, int64_t n, float* y, int where) {
       IK_HIP(hipMemcpyAsync(m->m->Xin.p, x, n * ik::kIn * sizeof(float), hipMemcpyHostToDevice, m->s));
       xd = m->m->Xin.p;
     }
-    m->m->forward(xd, n);
+    m->m->forward(xd, n, m->m->Y.p);
     IK_HIP(hipMemcpyAsync(y, m->m->Y.p, n * ik::kOut * sizeof(float),
                           where == IK_DEVICE ? hipMemcpyDeviceToDevice : hipMemcpyDeviceToHost, m->s));
     IK_HIP(hipStreamSynchronize(m->s));
@@ -630,9 +755,11 @@ int ik_mlp_forward_noalloc(ik_mlp* m, const float* x, int64_t n, float* y) {
                 "ik_mlp_forward_noalloc: the batch must have 1 to IK_MLP_NOALLOC_MAX_ROWS (8192) rows");
     float* s0 = g_scratchPtr[m->device];  // resolved at ik_mlp_create; never the array's host-side name
     ik::require(s0 != nullptr, IK_EINVAL, "ik_mlp_forward_noalloc: scratch not resolved for this device");
-    float* s1 = s0 + (int64_t)IK_MLP_NOALLOC_MAX_ROWS * ik::kHid;
-    m->m->s = m->s;
-    m->m->forwardInto(x, n, s0, s1, y);
+    const uintptr_t x0 = (uintptr_t)x, y0 = (uintptr_t)y;
+    const bool overlap = y0 < x0 + n * ik::kIn * sizeof(float) && x0 < y0 + n * ik::kOut * sizeof(float);
+    m->m->s            = m->s;
+    m->m->forward(x, n, overlap ? s0 : y);
+    if (overlap) IK_HIP(hipMemcpyAsync(y, s0, n * ik::kOut * sizeof(float), hipMemcpyDeviceToDevice, m->s));
     IK_HIP(hipStreamSynchronize(m->s));
   });
 }
@@ -669,9 +796,7 @@ int ik_mlp_train_step(ik_mlp* m, const float* x, const float* t, int64_t n, floa
       xd = m->m->Xin.p;
       td = m->m->Tin.p;
     }
-    const double l = m->m->lossGrad(xd, td, n);
-    m->m->adam(lr, 0.9f, 0.999f, 1e-8f);
-    IK_HIP(hipStreamSynchronize(m->s));
+    const double l = m->m->lossGrad(xd, td, n, true, lr);
     if (loss) *loss = l;
   });
 }
