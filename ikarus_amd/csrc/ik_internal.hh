@@ -114,7 +114,10 @@ constexpr int kSellRows = 64;
 constexpr int kTileElems   = IK_TILE_ELEMS;
 constexpr int kTileThreads = kTileElems * 16;
 constexpr int kTileEntries = kTileElems * 36;  // upper element blocks per tile
-static_assert(kTileElems % 4 == 0 && kTileElems <= 16, "tiles hold whole wavefronts, entries fit 10 bits");
+// accumulator of a padding entry of a tile
+constexpr uint16_t kNoEntry = 0xFFFF;
+static_assert(kTileElems % 8 == 0 && kTileElems <= 24 && kTileEntries < 1024,
+              "tiles hold whole wavefronts of points, group counts fit 10 bits");
 
 }  // namespace ik
 
@@ -186,9 +189,13 @@ struct ik_handle {
   //  staging slot per group (segments ordered by tile). tileElem[t*16+s] = element (-1: padding of the
   //  last tile); tgptr[t] = first group of tile t (groups in gather order); gdst[g] = the slot of
   //  group g, or -(K slot + 1) for a direct group, whose mirror slot is gpt[g] and FULL mask gmsk[g].
-  //  epos[t*576 + j] = group | rank << 10 | transposed << 15 of the tile's entry j = 36 s + sb (rank = its
-  //  position in the group by increasing j; padding entries target spare accumulators past the groups),
-  //  tmaxr[t] = the tile's largest group size.
+  //  epos[t*576 + j] = LDS accumulator | transposed << 15 of the tile's entry j = 36 s + sb (kNoEntry: padding). A
+  //  group of one or two entries has the accumulator of its index, a larger one (these come last in the tile) an
+  //  accumulator per entry, first | count << 16 of it in gmul; tmaxr[t] = the largest count of the tile.
+  //  tmeta[4 t ..] = first group, first of gmul, staged one-accumulator groups | all of these << 10 | larger groups
+  //  << 20, accumulators | tmaxr << 16;
+  //  tileNode[(16 t + s) 8 + q] = node of corner q of the element in slot s (padding: of slot 0).
+  //  maxGroups, maxAcc = the largest numbers of groups and accumulators of a tile (they size the kernel's LDS).
   // Residual staging: node by node, each node's (element, corner) incidences ordered by element;
   // rdest[e*8+a] = slot, ncptr[n] = first slot of node n
   ik::DevBuf<int32_t> bdest, segptr, ncptr, rdest;
@@ -197,6 +204,9 @@ struct ik_handle {
   ik::DevBuf<int32_t> tileElem, tgptr, gdst, gpt;
   ik::DevBuf<uint16_t> epos, gmsk;
   ik::DevBuf<uint8_t> tmaxr;
+  ik::DevBuf<int32_t> tmeta, tileNode;
+  ik::DevBuf<uint32_t> gmul;
+  int maxGroups = 0, maxAcc = 0;
   // staging chunks (tiles when tiled, elements otherwise) and the block rows complete after each chunk
   std::vector<int64_t> chunkElem, chunkRow;
   // element-by-element staging of K_e (36 upper 3x3 blocks) and R_e (24)

@@ -628,8 +628,8 @@ struct ik_mlp {
 };
 
 // Scratch of the allocation-free forward (ik_mlp_forward_noalloc): the outputs of a call whose y overlaps its x (the
-// kernel's workgroups read x while others write y), IK_MLP_NOALLOC_MAX_ROWS x 3 FP32, one copy per device held until the
-// process ends. Host code uses only the address hipGetSymbolAddress returns for the device (the array's name on the
+// kernel's workgroups read x while others write y), IK_MLP_NOALLOC_MAX_ROWS x 3 FP32, one copy per device held until
+// the process ends. Host code uses only the address hipGetSymbolAddress returns for the device (the array's name on the
 // host is not a device address), resolved once per device at ik_mlp_create with that device current.
 static __device__ __align__(256) float scratch[IK_MLP_NOALLOC_MAX_ROWS * ik::kOut];
 

@@ -424,23 +424,30 @@ void buildPattern(ik_handle* h) {
       require(pos[q] == segBeg[q] + segCnt[q], IK_EINVAL, "internal error: staging segments do not tile the slots");
     h->bdest.upload(dest.data(), dest.size(), h->stream);
   } else {
-    // per tile: the entries j = 36 s + sb that fall on one upper block form a group; groups ordered by the gather
-    // order of their upper blocks, i.e. by staging slot and by K slot; each entry's rank = its position in its
-    // group by increasing j (the order the tile sums them).
-    // epos[t*576 + j] = group | rank << 10 | transposed << 15; padding entries target spare accumulators
-    // ng + (j - 36 nvalid), rank 0, which the tile never stores. tmaxr[t] = the largest group size.
-    // Each chunk of tiles lists its groups' upper blocks in its own buffer; tgptr places them.
+    // per tile: the entries j = 36 s + sb that fall on one upper block form a group. The tile adds its entries in LDS
+    // in one step: a group of one or two entries has one accumulator (a sum of two does not depend on the order of the
+    // adds), a larger group one accumulator per entry, summed in entry order when the group is stored. Groups come with
+    // those of one accumulator first (group g: accumulator g), those staged before those written directly, then the
+    // others, each kind in the gather order of its upper blocks, i.e. by staging slot and by K slot. epos[t*576 + j]
+    // = accumulator | transposed << 15, kNoEntry for padding; gmul = first accumulator | count << 16 of the larger
+    // groups, those of tile t at [tmptr[t], tmptr[t+1]); tmaxr[t] = the largest count. Each chunk of tiles lists its
+    // groups' upper blocks in its own buffer; tgptr places them. tmeta[4 t ..] = first group, first larger group,
+    // single-accumulator groups that are staged | single-accumulator groups << 10 | larger groups << 20, number of
+    // accumulators | largest count << 16.
     HostVec<uint16_t> epos((size_t)ntiles * kTileEntries);
     std::vector<uint8_t> tmaxr(ntiles);
-    std::vector<int32_t> tgptr(ntiles + 1, 0);
+    std::vector<int32_t> tgptr(ntiles + 1, 0), tmptr(ntiles + 1, 0);
     HostVec<int32_t> gq;
-    std::vector<int64_t> tng(ntiles);
+    HostVec<uint32_t> gmul;
+    std::vector<int64_t> tng(ntiles), tnm(ntiles);
+    int maxGroups = 0, maxAcc = 0;  // largest numbers of groups and accumulators of a tile
     // a tile's upper blocks -> group: open-addressing table of 2048 slots (a tile touches at most 576 upper blocks),
     // a slot valid when its stamp is the current tile
     constexpr int kHash = 2048;
     std::vector<std::vector<int32_t>> gpart(chunkCount(ntiles, 256));
+    std::vector<std::vector<uint32_t>> mpart(chunkCount(ntiles, 256));
     parallelChunks(ntiles, [&](int64_t t0, int64_t t1, int64_t ch) {
-      std::vector<int32_t> hkey(kHash), hval(kHash), touched, entQ(kTileEntries), fill(kTileEntries);
+      std::vector<int32_t> hkey(kHash), hval(kHash), touched, entQ(kTileEntries), cntQ(kTileEntries), accOf(kTileEntries);
       std::vector<int64_t> hstamp(kHash, -1);
       std::vector<uint16_t> entTr(kTileEntries);
       std::vector<int32_t>& out = gpart[ch];
@@ -467,8 +474,10 @@ void buildPattern(ik_handle* h) {
               if (hstamp[k] != t) {
                 hstamp[k] = t;
                 hkey[k]   = q;
+                hval[k]   = 0;
                 touched.push_back(q);
               }
+              ++hval[k];  // entries of the group
             }
         }
         // gather order: sort the ranks, then map back to upper blocks
@@ -476,22 +485,33 @@ void buildPattern(ik_handle* h) {
         std::sort(touched.begin(), touched.end());
         for (auto& q : touched) q = qord[q];
         const int ng = (int)touched.size();
-        for (int g = 0; g < ng; ++g) hval[slotOf(touched[g], t)] = g;
-        std::fill(fill.begin(), fill.begin() + ng, 0);
-        uint16_t* ep = epos.data() + t * kTileEntries;
-        int maxr     = 0;
-        for (int j = 0; j < kTileEntries; ++j) {
-          if (j < 36 * nvalid) {
-            const int g  = hval[slotOf(entQ[j], t)];
-            const int rk = fill[g]++;
-            require(rk < 16, IK_EINVAL, "more than 16 element blocks of one tile on one K block");
-            maxr  = std::max(maxr, rk + 1);
-            ep[j] = (uint16_t)(g | (rk << 10) | entTr[j]);
-          } else {
-            ep[j] = (uint16_t)(ng + (j - 36 * nvalid));
+        const int n1 = (int)(std::stable_partition(touched.begin(), touched.end(),
+                                                   [&](int32_t q) { return hval[slotOf(q, t)] <= 2; }) -
+                             touched.begin());
+        int nacc = n1, maxc = 1;
+        for (int g = 0; g < ng; ++g) {
+          int32_t& v = hval[slotOf(touched[g], t)];
+          cntQ[g]    = v;
+          v          = g;
+          accOf[g]   = g < n1 ? g : nacc;
+          if (g >= n1) {
+            mpart[ch].push_back((uint32_t)nacc | (uint32_t)cntQ[g] << 16);
+            nacc += cntQ[g];
+            maxc = std::max(maxc, (int)cntQ[g]);
           }
         }
-        tmaxr[t] = (uint8_t)maxr;
+        uint16_t* ep = epos.data() + t * kTileEntries;
+        for (int j = 0; j < kTileEntries; ++j) {
+          if (j >= 36 * nvalid) {
+            ep[j] = kNoEntry;
+            continue;
+          }
+          const int g = hval[slotOf(entQ[j], t)];
+          ep[j]       = (uint16_t)(accOf[g] | entTr[j]);
+          if (g >= n1) ++accOf[g];
+        }
+        tmaxr[t] = (uint8_t)maxc;
+        tnm[t]   = ng - n1;
         out.insert(out.end(), touched.begin(), touched.end());
         tng[t] = ng;
       }
@@ -500,12 +520,17 @@ void buildPattern(ik_handle* h) {
       int64_t tot = 0;
       for (int64_t t = 0; t < ntiles; ++t) {
         tot += tng[t];
+        maxGroups = std::max(maxGroups, (int)tng[t]);
+        tmptr[t + 1] = tmptr[t] + (int32_t)tnm[t];
         require(tot < (int64_t)INT32_MAX, IK_EINVAL, "mesh too large for int32 staging slots");
         tgptr[t + 1] = (int32_t)tot;
       }
       gq.resize(tot);
+      gmul.resize(tmptr[ntiles]);
+      for (int64_t t = 0; t < ntiles; ++t) maxAcc = std::max(maxAcc, (int)(tng[t] - tnm[t]));
       parallelChunks(ntiles, [&](int64_t t0, int64_t, int64_t ch) {  // the same chunks as the loop above
         std::copy(gpart[ch].begin(), gpart[ch].end(), gq.begin() + tgptr[t0]);
+        std::copy(mpart[ch].begin(), mpart[ch].end(), gmul.begin() + tmptr[t0]);
       }, 256);
     }
     // An upper block that only one tile touches is complete after that tile's group sum, which the tile
@@ -520,6 +545,28 @@ void buildPattern(ik_handle* h) {
       for (int64_t q = q0; q < q1; ++q) {
         gathered[q] = ntile[q] > 1;
         segCnt[q]   = gathered[q] ? ntile[q] : 0;
+      }
+    });
+    // the staged ones of a tile's single-accumulator groups move in front of the directly written ones
+    std::vector<int32_t> tns(ntiles);
+    parallelChunks(ntiles, [&](int64_t t0, int64_t t1, int64_t) {
+      std::vector<int32_t> perm(kTileEntries), old(kTileEntries);
+      for (int64_t t = t0; t < t1; ++t) {
+        int32_t* g   = gq.data() + tgptr[t];
+        const int n1 = (int)(tng[t] - tnm[t]);
+        int at       = 0;
+        std::copy(g, g + n1, old.begin());
+        for (int pass = 0; pass < 2; ++pass) {
+          for (int j = 0; j < n1; ++j)
+            if ((gathered[old[j]] != 0) == (pass == 0)) {
+              perm[j] = at;
+              g[at++] = old[j];
+            }
+          if (pass == 0) tns[t] = at;
+        }
+        uint16_t* ep = epos.data() + t * kTileEntries;
+        for (int j = 0; j < kTileEntries; ++j)
+          if (ep[j] != kNoEntry && (ep[j] & 0x7FFF) < n1) ep[j] = (uint16_t)(perm[ep[j] & 0x7FFF] | (ep[j] & 0x8000));
       }
     });
     h->nstage = layoutSegments();
@@ -554,11 +601,16 @@ void buildPattern(ik_handle* h) {
         for (int32_t k = 0; k < segCnt[q]; ++k) gdst[b[k]] = segBeg[q] + k;
       }
     });
-    // the kernel's indexing relies on these: in every tile each valid entry has a distinct (group, rank)
-    // with group < ng and rank < its group's size < tmaxr + 1, every group is non-empty, padding entries
-    // target spare accumulators in [ng, 576); the slots are a permutation of [0, nstage) with each group
-    // inside its own upper block's segment (the segments are disjoint consecutive ranges, each filled exactly
-    // by its cursor), and every upper block is either staged by two or more tiles or written by exactly one
+    // the kernel's indexing relies on these: in every tile the accumulators of the single-accumulator groups come first
+    // and get one or two entries each, those of the other groups follow without gaps and get one each, all below
+    // maxAcc; the slots are a permutation of [0, nstage) with each group inside its own upper block's segment (the
+    // segments are disjoint consecutive ranges, each filled exactly by its cursor), and every upper block is either
+    // staged by two or more tiles or written by exactly one
+    for (int64_t t = 0; t < ntiles; ++t)
+      if (tmptr[t + 1] > tmptr[t]) {
+        const uint32_t m = gmul[tmptr[t + 1] - 1];
+        maxAcc           = std::max(maxAcc, (int)((m & 0xFFFFu) + (m >> 16)));
+      }
     {
       parallelChunks(nup, [&](int64_t q0, int64_t q1, int64_t) {
         for (int64_t q = q0; q < q1; ++q)
@@ -578,31 +630,37 @@ void buildPattern(ik_handle* h) {
         }
       });
       parallelChunks(ntiles, [&](int64_t t0, int64_t t1, int64_t) {
-        std::vector<uint8_t> used(kTileEntries * 16);
-        std::vector<int32_t> fill(kTileEntries);
+        std::vector<int32_t> fill(kTileEntries);  // entries per accumulator
         for (int64_t t = t0; t < t1; ++t) {
-          const int ng = tgptr[t + 1] - tgptr[t];
-          int nvalid   = 0;
-          for (int s = 0; s < kTileElems; ++s) nvalid += tileElem[t * kTileElems + s] >= 0;
-          require(tileElem[t * kTileElems] >= 0 && ng <= 36 * nvalid && tmaxr[t] >= 1 && tmaxr[t] <= 16,
-                  IK_EINVAL, "internal error: bad tile");
-          std::fill(used.begin(), used.begin() + ng * 16, 0);
-          std::fill(fill.begin(), fill.begin() + ng, 0);
+          const int ng = tgptr[t + 1] - tgptr[t], nm = tmptr[t + 1] - tmptr[t], n1 = ng - nm;
+          int nvalid = 0;
+          while (nvalid < kTileElems && tileElem[t * kTileElems + nvalid] >= 0) ++nvalid;
+          for (int s = nvalid; s < kTileElems; ++s)
+            require(tileElem[t * kTileElems + s] < 0, IK_EINVAL, "internal error: bad tile padding");
+          require(nvalid >= 1 && ng >= 1 && n1 >= 0 && ng <= 36 * nvalid && ng <= maxGroups, IK_EINVAL,
+                  "internal error: bad tile");
+          int nacc = n1;
+          for (int m = 0; m < nm; ++m) {
+            const uint32_t v = gmul[tmptr[t] + m];
+            require((int)(v & 0xFFFFu) == nacc && (v >> 16) >= 3 && (v >> 16) <= tmaxr[t], IK_EINVAL,
+                    "internal error: bad tile accumulators");
+            nacc += (int)(v >> 16);
+          }
+          require(nacc <= maxAcc && nacc <= kTileEntries && tns[t] <= n1, IK_EINVAL,
+                  "internal error: bad tile accumulators");
+          for (int g = 0; g < n1; ++g)
+            require((gdst[tgptr[t] + g] >= 0) == (g < tns[t]), IK_EINVAL, "internal error: bad tile group order");
+          std::fill(fill.begin(), fill.begin() + nacc, 0);
           const uint16_t* ep = epos.data() + t * kTileEntries;
           for (int j = 0; j < kTileEntries; ++j) {
-            const int g = ep[j] & 0x3FF, rk = (ep[j] >> 10) & 0xF;
             if (j >= 36 * nvalid) {
-              require(g >= ng && g < kTileEntries && rk == 0 && !(ep[j] & 0x8000u), IK_EINVAL,
-                      "internal error: bad padding entry");
+              require(ep[j] == kNoEntry, IK_EINVAL, "internal error: bad padding entry");
               continue;
             }
-            require(g < ng && rk < tmaxr[t] && !used[g * 16 + rk], IK_EINVAL, "internal error: bad tile entry");
-            used[g * 16 + rk] = 1;
-            fill[g]++;
+            const int g = ep[j] & 0x7FFF;
+            require(g < nacc && ++fill[g] <= (g < n1 ? 2 : 1), IK_EINVAL, "internal error: bad tile entry");
           }
-          for (int g = 0; g < ng; ++g)
-            for (int rk = 0; rk < 16; ++rk)
-              require((rk < fill[g]) == (used[g * 16 + rk] != 0), IK_EINVAL, "internal error: gap in a tile group");
+          for (int g = 0; g < nacc; ++g) require(fill[g] >= 1, IK_EINVAL, "internal error: empty tile accumulator");
         }
       });
     }
@@ -613,7 +671,29 @@ void buildPattern(ik_handle* h) {
     h->gpt.upload(gpt.data(), gpt.size(), h->stream);
     h->gmsk.upload(gmsk.data(), gmsk.size(), h->stream);
     h->epos.upload(epos.data(), epos.size(), h->stream);
+    HostVec<int32_t> tmeta(ntiles * 4), tileNode(ntiles * kTileElems * 8);
+    parallelChunks(ntiles, [&](int64_t t0, int64_t t1, int64_t) {
+      for (int64_t t = t0; t < t1; ++t) {
+        const int32_t ng = tgptr[t + 1] - tgptr[t], nm = tmptr[t + 1] - tmptr[t];
+        const uint32_t m = nm ? gmul[tmptr[t + 1] - 1] : (uint32_t)ng;  // the last accumulators
+        tmeta[4 * t]     = tgptr[t];
+        tmeta[4 * t + 1] = tmptr[t];
+        tmeta[4 * t + 2] = tns[t] | (ng - nm) << 10 | nm << 20;
+        tmeta[4 * t + 3] = (int32_t)((m & 0xFFFFu) + (m >> 16)) | (int32_t)tmaxr[t] << 16;
+        // node of corner q of slot s (padding slots repeat slot 0): what the kernel's lanes load first
+        for (int s = 0; s < kTileElems; ++s) {
+          const int32_t e = tileElem[t * kTileElems + s];
+          std::copy_n(conn + (int64_t)(e >= 0 ? e : tileElem[t * kTileElems]) * 8, 8,
+                      &tileNode[(t * kTileElems + s) * 8]);
+        }
+      }
+    });
+    h->tmeta.upload(tmeta.data(), tmeta.size(), h->stream);
+    h->tileNode.upload(tileNode.data(), tileNode.size(), h->stream);
+    h->gmul.upload(gmul.data(), gmul.size(), h->stream);
     h->tmaxr.upload(tmaxr.data(), tmaxr.size(), h->stream);
+    h->maxGroups = maxGroups;
+    h->maxAcc    = maxAcc;
   }
   // the gather's upper blocks: the gathered ones in gather order (chunkQ[c]: first one of chunk c), placed by
   // a prefix count over qord; each one's segment must start where the previous one's ends
