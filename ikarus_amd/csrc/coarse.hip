@@ -27,6 +27,7 @@
 
 #include "host_parallel.hh"
 #include "ik_internal.hh"
+#include "wave_reduce.hh"
 
 namespace ik {
 
@@ -59,17 +60,6 @@ constexpr int kMaxAggregates    = 1024;  // the update's 2 na partials fit the f
 // threads of the per-aggregate update workgroup (64^3 learned path: 14.3 us per launch with 256, 16.4 with 512,
 // 51.9 with 1024)
 constexpr int kUpdateThreads = 256;
-
-__device__ inline double waveSumD(double v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-  return v;
-}
-__device__ inline float waveSumF(float v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-  return v;
-}
 
 // B(d)^T v for the masked modes: [v; d x v] with v's constrained components zeroed
 template <typename T>
@@ -144,7 +134,7 @@ __global__ __launch_bounds__(256) void coarseAssemble(const TV* __restrict__ K, 
     }
 #pragma unroll
     for (int m = 0; m < 36; ++m) {
-      const double v = waveSumD(acc[m]);
+      const double v = waveSum(acc[m]);
       if (lane == 0) red[wave][m] = v;
     }
     __syncthreads();
@@ -223,7 +213,7 @@ __global__ __launch_bounds__(256) void coarseRestrict(const float* __restrict__ 
   }
 #pragma unroll
   for (int m = 0; m < 6; ++m) {
-    const float v = waveSumF(acc[m]);
+    const float v = waveSum(acc[m]);
     if (lane == 0) red[wave][m] = v;
   }
   __syncthreads();
@@ -247,7 +237,7 @@ __global__ __launch_bounds__(256) void coarseGemv(const float4* __restrict__ G, 
     const float4 a = g[c], b = s[c];
     acc += a.x * b.x + a.y * b.y + a.z * b.z + a.w * b.w;
   }
-  acc = waveSumF(acc);
+  acc = waveSum(acc);
   if (lane == 0) w[row] = acc;
 }
 
@@ -279,7 +269,7 @@ __global__ __launch_bounds__(256) void coarseZ(const float* __restrict__ r, cons
       rz += (double)rl[k] * (double)zk;
     }
   }
-  rz = waveSumD(rz);
+  rz = waveSum(rz);
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = rz;
   __syncthreads();
   if (threadIdx.x == 0) partial[gridDim.x + blockIdx.x] = ((red[0] + red[1]) + red[2]) + red[3];
@@ -290,7 +280,7 @@ __global__ __launch_bounds__(256) void coarseZ(const float* __restrict__ r, cons
 template <int W, int N>
 __device__ inline void groupSums(double (&v)[N], double (&red)[W][N]) {
 #pragma unroll
-  for (int i = 0; i < N; ++i) v[i] = waveSumD(v[i]);
+  for (int i = 0; i < N; ++i) v[i] = waveSum(v[i]);
   if ((threadIdx.x & 63) == 0)
 #pragma unroll
     for (int i = 0; i < N; ++i) red[threadIdx.x >> 6][i] = v[i];
@@ -387,7 +377,7 @@ __global__ __launch_bounds__(256) void coarseGemvDot(const float4* __restrict__ 
       acc += a.x * b.x + a.y * b.y + a.z * b.z + a.w * b.w;
     }
   }
-  acc = waveSumF(acc);
+  acc = waveSum(acc);
   if (lane == 0) {
     if (row < nc) w[row] = acc;
     red[threadIdx.x >> 6] = row < nc ? (double)acc * (double)s[row] : 0.0;

@@ -245,7 +245,7 @@ struct ik_handle {
 
   // solver workspace
   ik::DevBuf<double> pr, pz, pp, pq, px, pdiag, pb, partial;
-  ik::DevBuf<float> fr, fp, fq, fx, fdiag;  // FP32 PCG vectors; fdiag holds 3x3 block inverses
+  ik::DevBuf<float> fr, fp, fp2, fz, fq, fx, fdiag;  // FP32 PCG vectors; fdiag holds 3x3 block inverses
   ik::DevBuf<ik::PcgScalars> sc;
   ik::PcgScalars* hsc = nullptr;  // pinned host mirror
   double* hred = nullptr;         // pinned host scalar for reductions
@@ -286,7 +286,6 @@ void easUpdate(ik_handle* h, const double* duDev);
 void easStage(ik_handle* h, int64_t e0, int64_t count, bool wantK, const int32_t* dest, const int32_t* rdest);
 // sparse.hip
 void spmv64(ik_handle* h, const double* x, double* y);
-void spmv32(ik_handle* h, const float* x, float* y);
 double dot(ik_handle* h, const double* a, const double* b, int64_t n);
 void axpy(ik_handle* h, double a, const double* x, double* y, int64_t n);  // y += a x
 // per-block partial sums (at most kReduceBlocks) folded in a fixed order
@@ -307,7 +306,6 @@ void coarseApply(ik_handle* h, const float* r, float* z, float* p, const float* 
 void coarseIteration(ik_handle* h, const double* pq, int npq, float* x, float* r, float* p, const float* q,
                      const float* binv, int gn, double* partial, int maxIter);
 int64_t coarseDofs(const ik_handle* h);
-void residualBlock64(ik_handle* h, const double* b, const double* x, double* r);  // r = b - K x (FP64 K)
 // mlp.hip
 Mlp* mlpCreate(hipStream_t s);
 void mlpDestroy(Mlp* m);

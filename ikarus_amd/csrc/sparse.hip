@@ -10,31 +10,32 @@
 // iterations in chunks and poll the flag asynchronously: the iterate after convergence is exactly the
 // one Eigen's loop returns.
 #include "ik_internal.hh"
+#include "wave_reduce.hh"
 
 namespace ik {
 namespace {
 
-constexpr int SPMV_BS = 256;  // threads per block
-
 // Block rows per wavefront of the SpMV lane layouts: FP64 values 3 lanes per row (21 rows, lane 63 idles),
-// FP32 values one lane per row (64 rows).
+// FP32 values one lane per row (64 rows). G wavefronts share the rows of one, taking every G-th block each, so that a
+// small matrix still puts enough loads in flight: a lane's blocks are a chain of round trips to the caches.
 template <typename TV>
 constexpr int spmvRowsPerWave() {
   return sizeof(TV) == 4 ? 64 : 21;
 }
-template <typename TV>
+constexpr int SPMV_BS = 256;
+template <typename TV, int G>
 constexpr int spmvRowsPerBlock() {
-  return (SPMV_BS / 64) * spmvRowsPerWave<TV>();
-}
-template <typename TV>
-inline unsigned spmvGrid(int64_t nrows) {
-  return (unsigned)((nrows + spmvRowsPerBlock<TV>() - 1) / spmvRowsPerBlock<TV>());
+  return SPMV_BS / 64 / G * spmvRowsPerWave<TV>();
 }
 
-__device__ inline double waveSum(double v) {
+// Waits for a loaded value here: the loads above it are in flight together, instead of each behind the branch or
+// barrier that precedes its use
+__device__ inline void arrived(double& v) { asm volatile("" : "+v"(v)); }
+__device__ inline void arrived(float& v) { asm volatile("" : "+v"(v)); }
+template <typename T, int N>
+__device__ inline void arrived(T (&v)[N]) {
 #pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-  return v;
+  for (int i = 0; i < N; ++i) arrived(v[i]);
 }
 
 // block-wide sum; result valid in thread 0
@@ -58,34 +59,32 @@ __device__ inline double blockSum(double v) {
 // block. Two lane layouts:
 //  FP64 values: lane (r, k), row r = lane / 3 (21 rows per wavefront), output component k: for a fixed j the
 //   wavefront's 21 rows read 21 adjacent 72-byte blocks (1,512 contiguous bytes), each lane its block row.
-//   Each row runs over its own blocks in column order, so the result equals a CSR SpMV's bit for bit.
 //  FP32 values: one lane per block row, the 3 outputs of the row per lane, a wavefront = one slice: for a
 //   fixed j the 64 lanes read 64 adjacent 36-byte blocks (2304 contiguous bytes). Each lane runs to the
 //   slice's longest row; padding slots hold zeros with the row's own column.
 // 64^3 pattern, alone: FP32 48.6 us against 62.3 us for 3 lanes per row over CSR (21 rows per wavefront);
 // FP64 108.4 us against 119.3 us for the former layout with one lane per block entry (7 rows per wavefront).
-// FP64 issues the loads of SPMV_UNROLL blocks (3 x 24 bytes and 3 column indices per lane) before summing their
-// products: 3 beat 2, 4, 5, 6 and 9 (111.3, 111.9, 114.8, 116.5 and 121.1 us).
+// Both issue the loads of 3 blocks before summing their products (FP64: 2, 4, 5, 6 and 9 gave 111.3, 111.9, 114.8,
+// 116.5 and 121.1 us; FP32 53.2 us against 56.3, 60.9 and 68.4 us for 2, 4 and 6).
 constexpr int SPMV_UNROLL = 3;
 static_assert(kSellRows == 64, "one slice per wavefront");
 
-// a[k] = (K x)[3 row + k], k = 0..2, for one lane per row: the slice's w slots of row `row`
-template <typename TV, typename TX, typename TA>
+// a[k] = sum of (K x)[3 row + k], k = 0..2, over the slots j = g, g + G, ... of the slice of row `row` (a lane per row)
+template <int G, typename TA, typename TV, typename TX>
 __device__ inline void rowSell3(const int32_t* __restrict__ sellStart, const int32_t* __restrict__ scol,
-                                const TV* __restrict__ val, const TX* __restrict__ x, int64_t row, TA a[3]) {
+                                const TV* __restrict__ val, const TX* __restrict__ x, int64_t row, int g, TA a[3]) {
   const int64_t s = row >> 6;
   const int r     = (int)(row & 63);
   const int32_t s0 = sellStart[s];
   const int w      = (sellStart[s + 1] - s0) >> 6;
-  const TV* V      = val + ((int64_t)s0 + r) * 9;
+  const TV* v0     = val + ((int64_t)s0 + r) * 9;
   const int32_t* C = scol + s0 + r;
   TA a0 = TA(0), a1 = TA(0), a2 = TA(0);
-  // 3 slots per unrolled step: 53.2 us at 64^3 against 56.3, 60.9 and 68.4 us for 2, 4 and 6
-#pragma unroll 3
-  for (int j = 0; j < w; ++j) {
+#pragma unroll SPMV_UNROLL
+  for (int j = g; j < w; j += G) {
     const int64_t c = (int64_t)C[j * kSellRows] * 3;
     const TA x0 = (TA)x[c], x1 = (TA)x[c + 1], x2 = (TA)x[c + 2];
-    const TV* v = V + (int64_t)j * (kSellRows * 9);
+    const TV* v = v0 + (int64_t)j * (kSellRows * 9);
     a0 += (TA)v[0] * x0 + (TA)v[1] * x1 + (TA)v[2] * x2;
     a1 += (TA)v[3] * x0 + (TA)v[4] * x1 + (TA)v[5] * x2;
     a2 += (TA)v[6] * x0 + (TA)v[7] * x1 + (TA)v[8] * x2;
@@ -95,54 +94,79 @@ __device__ inline void rowSell3(const int32_t* __restrict__ sellStart, const int
   a[2] = a2;
 }
 
-// (K x)[3 row + k] accumulated in TA with the FP64 lane layout, lane = 3 rl + k (row rl of the wavefront's 21,
-// output component k); valid on lanes with `out` set. For a fixed j the wavefront's 21 rows read 21 adjacent
-// 72-byte blocks (1,512 contiguous bytes), each lane the 24 bytes of its block row. The lane keeps one sum per
-// column l, a_l = sum_j K_j[k][l] x_j[l] in block order, and returns a_0 + (a_1 + a_2): the order of the former
-// layout with one lane per block entry (7 rows per wavefront, combined by two lane shifts), so y is bitwise the
-// same as then and as a CSR SpMV's. The loads of SPMV_UNROLL blocks are issued before their products are summed.
-template <typename TV, typename TX, typename TA>
-__device__ inline TA spmvRow3(const int32_t* __restrict__ rowptr, const int32_t* __restrict__ sellStart,
+// (K x)[3 row + k] over the blocks j = g, g + G, ... of row `row` (FP64 lane layout). The lane keeps one sum per
+// column l, a_l = sum_j K_j[k][l] x_j[l] in block order, and returns a_0 + (a_1 + a_2).
+template <int G, typename TA, typename TV, typename TX>
+__device__ inline TA rowSell1(const int32_t* __restrict__ rowptr, const int32_t* __restrict__ sellStart,
                               const int32_t* __restrict__ scol, const TV* __restrict__ val,
-                              const TX* __restrict__ x, int64_t nrows, unsigned rb, int64_t& row, int& k,
-                              bool& out) {
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int rl = lane / 3;
-  k            = lane - 3 * rl;
-  row          = ((int64_t)rb * (SPMV_BS / 64) + wave) * spmvRowsPerWave<TV>() + rl;
-  out          = rl < spmvRowsPerWave<TV>() && row < nrows;
-  if (!out) return TA(0);
+                              const TX* __restrict__ x, int64_t row, int k, int g) {
   const int64_t base = (int64_t)sellStart[row >> 6] + (row & 63);
-  const TV* V        = val + base * 9 + 3 * k;
+  const TV* v0       = val + base * 9 + 3 * k;
   const int32_t* C   = scol + base;
   const int n        = rowptr[row + 1] - rowptr[row];
   TA a0 = TA(0), a1 = TA(0), a2 = TA(0);
-  int j = 0;
-  for (; j + SPMV_UNROLL <= n; j += SPMV_UNROLL) {
+  int j = g;
+  for (; j + (SPMV_UNROLL - 1) * G < n; j += SPMV_UNROLL * G) {
     int32_t c[SPMV_UNROLL];
     TV v[SPMV_UNROLL][3];
 #pragma unroll
     for (int u = 0; u < SPMV_UNROLL; ++u) {
-      c[u] = C[(j + u) * kSellRows];
+      c[u] = C[(j + u * G) * kSellRows];
 #pragma unroll
-      for (int l = 0; l < 3; ++l) v[u][l] = V[(int64_t)(j + u) * (kSellRows * 9) + l];
+      for (int l = 0; l < 3; ++l) v[u][l] = v0[(int64_t)(j + u * G) * (kSellRows * 9) + l];
     }
 #pragma unroll
     for (int u = 0; u < SPMV_UNROLL; ++u) {
-      const TX* xc = x + (int64_t)c[u] * 3;
-      a0 += (TA)v[u][0] * (TA)xc[0];
-      a1 += (TA)v[u][1] * (TA)xc[1];
-      a2 += (TA)v[u][2] * (TA)xc[2];
+      const int64_t xc = (int64_t)c[u] * 3;
+      a0 += (TA)v[u][0] * (TA)x[xc];
+      a1 += (TA)v[u][1] * (TA)x[xc + 1];
+      a2 += (TA)v[u][2] * (TA)x[xc + 2];
     }
   }
-  for (; j < n; ++j) {
-    const TV* vj = V + (int64_t)j * (kSellRows * 9);
-    const TX* xc = x + (int64_t)C[j * kSellRows] * 3;
-    a0 += (TA)vj[0] * (TA)xc[0];
-    a1 += (TA)vj[1] * (TA)xc[1];
-    a2 += (TA)vj[2] * (TA)xc[2];
+  for (; j < n; j += G) {
+    const TV* vj     = v0 + (int64_t)j * (kSellRows * 9);
+    const int64_t xc = (int64_t)C[j * kSellRows] * 3;
+    a0 += (TA)vj[0] * (TA)x[xc];
+    a1 += (TA)vj[1] * (TA)x[xc + 1];
+    a2 += (TA)vj[2] * (TA)x[xc + 2];
   }
   return a0 + (a1 + a2);
+}
+
+// The rows of row block rb: out(i, x_i, y_i) is called once for each entry i = 3 row + k of y = K x, accumulated in TA.
+// With G > 1 the partial sums of the G wavefronts that share rows meet in LDS, summed in wavefront order.
+template <int G, typename TA, typename TV, typename TX, typename F>
+__device__ inline void spmvRows(const int32_t* __restrict__ rowptr, const int32_t* __restrict__ sellStart,
+                                const int32_t* __restrict__ scol, const TV* __restrict__ val,
+                                const TX* __restrict__ x, int64_t nrows, unsigned rb, F out) {
+  constexpr int NO = sizeof(TV) == 4 ? 3 : 1;  // outputs per lane
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, g = wave % G;
+  const int rl      = sizeof(TV) == 4 ? lane : lane / 3;
+  const int k       = sizeof(TV) == 4 ? 0 : lane - 3 * rl;
+  const int64_t row = (int64_t)rb * spmvRowsPerBlock<TV, G>() + wave / G * spmvRowsPerWave<TV>() + rl;
+  const bool in     = rl < spmvRowsPerWave<TV>() && row < nrows;
+  TA a[NO];
+  if (in) {
+    if constexpr (NO == 3)
+      rowSell3<G, TA>(sellStart, scol, val, x, row, g, a);
+    else
+      a[0] = rowSell1<G, TA>(rowptr, sellStart, scol, val, x, row, k, g);
+  }
+  if constexpr (G > 1) {
+    __shared__ TA part[SPMV_BS / 64][NO][64];
+    if (in)
+#pragma unroll
+      for (int o = 0; o < NO; ++o) part[wave][o][lane] = a[o];
+    __syncthreads();
+    if (in && g == 0)
+#pragma unroll
+      for (int w = 1; w < G; ++w)
+#pragma unroll
+        for (int o = 0; o < NO; ++o) a[o] += part[wave + w][o][lane];
+  }
+  if (in && g == 0)
+#pragma unroll
+    for (int o = 0; o < NO; ++o) out(row * 3 + k + o, a[o]);
 }
 
 // rev: workgroup i takes row block gridDim.x - 1 - i (the partial stays at the row block's index, so the fold
@@ -150,77 +174,213 @@ __device__ inline TA spmvRow3(const int32_t* __restrict__ rowptr, const int32_t*
 // the matrix (FP32 259 MB, FP64 518 MB, plus 29 MB of column indices) is larger than the 256 MB last-level
 // cache, and a pass in one direction evicts what the next pass in the same direction reads first, while a pass
 // in the other direction starts on the part just read (64^3: FP64 134.4 -> 119.0 us, FP32 57.0 -> 53.3 us).
-template <typename TV, typename TX, bool DOT>
+template <typename TV, typename TX, bool DOT, int G>
 __global__ __launch_bounds__(SPMV_BS) void spmvKernel(const int32_t* __restrict__ rowptr,
-                                                      const int32_t* __restrict__ sellStart,
-                                                      const int32_t* __restrict__ scol,
-                                                      const TV* __restrict__ val, const TX* __restrict__ x,
-                                                      TX* __restrict__ y, int64_t nrows,
-                                                      double* __restrict__ partial,
-                                                      const PcgScalars* __restrict__ sc, int rev) {
+                                                               const int32_t* __restrict__ sellStart,
+                                                               const int32_t* __restrict__ scol,
+                                                               const TV* __restrict__ val, const TX* __restrict__ x,
+                                                               TX* __restrict__ y, int64_t nrows,
+                                                               double* __restrict__ partial,
+                                                               const PcgScalars* __restrict__ sc, int rev) {
   if (sc && sc->done) return;
   const unsigned rb = rev ? gridDim.x - 1u - blockIdx.x : blockIdx.x;
   double d = 0.0;
-  if constexpr (sizeof(TV) == 4) {
-    const int64_t row = (int64_t)rb * SPMV_BS + threadIdx.x;
-    if (row < nrows) {
-      TX a[3];
-      rowSell3<TV, TX, TX>(sellStart, scol, val, x, row, a);
-#pragma unroll
-      for (int k = 0; k < 3; ++k) {
-        y[row * 3 + k] = a[k];
-        if (DOT) d += (double)x[row * 3 + k] * (double)a[k];
-      }
-    }
-  } else {
-    int64_t row;
-    int k;
-    bool out;
-    const TX yk = spmvRow3<TV, TX, TX>(rowptr, sellStart, scol, val, x, nrows, rb, row, k, out);
-    if (out) {
-      y[row * 3 + k] = yk;
-      if (DOT) d = (double)x[row * 3 + k] * (double)yk;
-    }
-  }
+  spmvRows<G, TX>(rowptr, sellStart, scol, val, x, nrows, rb, [&](int64_t i, TX yi) {
+    y[i] = yi;
+    if (DOT) d += (double)x[i] * (double)yi;
+  });
   if (DOT) {
     const double s = blockSum<SPMV_BS>(d);
     if (threadIdx.x == 0) partial[rb] = s;
   }
 }
 
-// r = b - K x with FP64 accumulation (K may be FP32); used by iterative refinement. Same lane layouts.
-template <typename TV>
-__global__ __launch_bounds__(SPMV_BS) void residualKernel(const int32_t* __restrict__ rowptr,
-                                                          const int32_t* __restrict__ sellStart,
-                                                          const int32_t* __restrict__ scol,
-                                                          const TV* __restrict__ val,
-                                                          const double* __restrict__ x,
-                                                          const double* __restrict__ b, double* __restrict__ r,
-                                                          int64_t nrows, double* __restrict__ partial) {
-  double d = 0.0;
-  if constexpr (sizeof(TV) == 4) {
-    const int64_t row = (int64_t)blockIdx.x * SPMV_BS + threadIdx.x;
-    if (row < nrows) {
-      double a[3];
-      rowSell3<TV, double, double>(sellStart, scol, val, x, row, a);
-#pragma unroll
-      for (int k = 0; k < 3; ++k) {
-        const double rk = b[row * 3 + k] - a[k];
-        r[row * 3 + k]  = rk;
-        d += rk * rk;
+// Convergence test and beta of a PCG iteration from the update kernel's partials (r.r, r.z). Every calling block folds
+// them in the same fixed order, so all blocks agree bitwise; the one with `record` writes the scalars. test() returns
+// false when the iteration has converged. beta = r.z / (r.z of the previous iterate), which only the update kernel
+// writes. fetch() issues the loads, so that they are in flight with the caller's.
+template <int BS>
+struct PcgTest {
+  const double* __restrict__ partial;
+  int nb;
+  PcgScalars* __restrict__ sc;
+  double rr, rz, threshold, rzPrev;
+  __device__ void fetch(const double* __restrict__ part, int n, PcgScalars* __restrict__ scalars) {
+    partial   = part;
+    nb        = n;
+    sc        = scalars;
+    const bool in = (int)threadIdx.x < nb;
+    rr        = in ? partial[threadIdx.x] : 0.0;
+    rz        = in ? partial[nb + threadIdx.x] : 0.0;
+    threshold = sc->threshold;
+    rzPrev    = sc->rz;
+  }
+  __device__ void wait() {
+    arrived(rr);
+    arrived(rz);
+  }
+  __device__ bool test(int maxIter, bool record, double& beta) {
+    __shared__ double bc[2];
+    for (int i = threadIdx.x + BS; i < nb; i += BS) {
+      rr += partial[i];
+      rz += partial[nb + i];
+    }
+    rr = blockSum<BS>(rr);
+    rz = blockSum<BS>(rz);
+    if (threadIdx.x == 0) {
+      bc[0] = rr;
+      bc[1] = rz;
+    }
+    __syncthreads();
+    rr              = bc[0];
+    rz              = bc[1];
+    const bool conv = rr < threshold;
+    beta            = rz / rzPrev;
+    if (record && threadIdx.x == 0) {
+      sc->rr = rr;
+      if (conv) {
+        sc->done = 1;
+      } else {
+        sc->beta   = beta;
+        sc->rz_new = rz;
+        sc->iters += 1;
+        if (sc->iters >= maxIter) sc->done = 2;
       }
     }
-  } else {
-    int64_t row;
-    int k;
-    bool out;
-    const double kx = spmvRow3<TV, double, double>(rowptr, sellStart, scol, val, x, nrows, blockIdx.x, row, k, out);
-    if (out) {
-      const double rk = b[row * 3 + k] - kx;
-      r[row * 3 + k]  = rk;
-      d               = rk * rk;
-    }
+    return !conv;
   }
+};
+
+// The first half of a PCG iteration in one launch, for small systems whose kernels are bound by launch and latency:
+// with `test` the convergence test and beta of the previous iteration (else beta as recorded), then q = K p with
+// p = z + beta p_old formed at every read (the neighbours' too: twice the gathered bytes, which stay in the caches
+// at these sizes), p stored beside p_old's buffer, and p.q partials. Lanes as spmvRows (G wavefronts share the rows);
+// the loads of a lane's first DEPTH blocks, of z and p_old included, are in flight while the block folds the partials.
+template <typename TV, int G>
+__global__ __launch_bounds__(SPMV_BS) void pcgDirectionSpmv(
+    const int32_t* __restrict__ rowptr, const int32_t* __restrict__ sellStart, const int32_t* __restrict__ scol,
+    const TV* __restrict__ val, const TV* __restrict__ z, const TV* __restrict__ pOld, TV* __restrict__ p,
+    TV* __restrict__ q, int64_t nrows, const double* __restrict__ partial, int nb, double* __restrict__ pq,
+    PcgScalars* __restrict__ sc, int maxIter, int test) {
+  int done = sc->done;
+  PcgTest<SPMV_BS> t;
+  if (test) t.fetch(partial, nb, sc);
+  double bt        = sc->beta;
+  constexpr int NO = sizeof(TV) == 4 ? 3 : 1;  // outputs per lane
+  constexpr int DEPTH = 27 / G + 1 < 4 ? 27 / G + 1 : 4;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, g = wave % G;
+  const int rl      = sizeof(TV) == 4 ? lane : lane / 3;
+  const int k       = sizeof(TV) == 4 ? 0 : lane - 3 * rl;
+  const int64_t row = (int64_t)blockIdx.x * spmvRowsPerBlock<TV, G>() + wave / G * spmvRowsPerWave<TV>() + rl;
+  const bool in     = rl < spmvRowsPerWave<TV>() && row < nrows;
+  const int64_t base = in ? (int64_t)sellStart[row >> 6] + (row & 63) : 0;
+  const int w        = in ? rowptr[row + 1] - rowptr[row] : 0;
+  const int32_t* C   = scol + base;
+  const TV* v0       = val + base * 9 + 3 * k;
+  TV v[DEPTH][3 * NO], zc[DEPTH][3], pc[DEPTH][3], zr[NO], pr[NO];
+  auto load = [&](int j, TV (&vj)[3 * NO], TV (&zj)[3], TV (&pj)[3]) {
+    const int64_t c = (int64_t)C[j * kSellRows] * 3;
+#pragma unroll
+    for (int l = 0; l < 3 * NO; ++l) vj[l] = v0[(int64_t)j * (kSellRows * 9) + l];
+#pragma unroll
+    for (int l = 0; l < 3; ++l) {
+      zj[l] = z[c + l];
+      pj[l] = pOld[c + l];
+    }
+  };
+#pragma unroll
+  for (int u = 0; u < DEPTH; ++u)
+    if (g + u * G < w) load(g + u * G, v[u], zc[u], pc[u]);
+  if (in)
+#pragma unroll
+    for (int o = 0; o < NO; ++o) {
+      zr[o] = z[row * 3 + k + o];
+      pr[o] = pOld[row * 3 + k + o];
+    }
+#pragma unroll
+  for (int u = 0; u < DEPTH; ++u) {
+    arrived(v[u]);
+    arrived(zc[u]);
+    arrived(pc[u]);
+  }
+  arrived(zr);
+  arrived(pr);
+  if (test) t.wait();
+  if (done) return;
+  if (test && !t.test(maxIter, blockIdx.x == 0, bt)) return;
+  const TV beta = (TV)bt;
+  TV a[NO][3];  // one sum per output and column
+#pragma unroll
+  for (int o = 0; o < NO; ++o) a[o][0] = a[o][1] = a[o][2] = TV(0);
+  auto add = [&](const TV (&vj)[3 * NO], const TV (&zj)[3], const TV (&pj)[3]) {
+#pragma unroll
+    for (int l = 0; l < 3; ++l) {
+      const TV x = zj[l] + beta * pj[l];
+#pragma unroll
+      for (int o = 0; o < NO; ++o) a[o][l] += vj[3 * o + l] * x;
+    }
+  };
+#pragma unroll
+  for (int u = 0; u < DEPTH; ++u)
+    if (g + u * G < w) add(v[u], zc[u], pc[u]);
+  for (int j = g + DEPTH * G; j < w; j += G) {
+    load(j, v[0], zc[0], pc[0]);
+    add(v[0], zc[0], pc[0]);
+  }
+  TV y[NO];
+#pragma unroll
+  for (int o = 0; o < NO; ++o) y[o] = a[o][0] + (a[o][1] + a[o][2]);
+  if constexpr (G > 1) {
+    __shared__ TV part[SPMV_BS / 64][NO][64];
+#pragma unroll
+    for (int o = 0; o < NO; ++o) part[wave][o][lane] = y[o];
+    __syncthreads();
+    if (g == 0)
+#pragma unroll
+      for (int wv = 1; wv < G; ++wv)
+#pragma unroll
+        for (int o = 0; o < NO; ++o) y[o] += part[wave + wv][o][lane];
+  }
+  double d = 0.0;
+  if (in && g == 0)
+#pragma unroll
+    for (int o = 0; o < NO; ++o) {
+      const int64_t i = row * 3 + k + o;
+      const TV pi     = zr[o] + beta * pr[o];
+      p[i]            = pi;
+      q[i]            = y[o];
+      d += (double)pi * (double)y[o];
+    }
+  const double s = blockSum<SPMV_BS>(d);
+  if (threadIdx.x == 0) pq[blockIdx.x] = s;
+}
+
+// the convergence test of the last iteration of a chunk of them, before the host looks at the flag
+__global__ __launch_bounds__(256) void pcgTestKernel(const double* __restrict__ partial, int nb,
+                                                     PcgScalars* __restrict__ sc, int maxIter) {
+  if (sc->done) return;
+  PcgTest<256> t;
+  t.fetch(partial, nb, sc);
+  double beta;
+  (void)t.test(maxIter, true, beta);
+}
+
+// r = b - K x with FP64 accumulation (K may be FP32); used by iterative refinement. Same lane layouts.
+template <typename TV, int G>
+__global__ __launch_bounds__(SPMV_BS) void residualKernel(const int32_t* __restrict__ rowptr,
+                                                                   const int32_t* __restrict__ sellStart,
+                                                                   const int32_t* __restrict__ scol,
+                                                                   const TV* __restrict__ val,
+                                                                   const double* __restrict__ x,
+                                                                   const double* __restrict__ b,
+                                                                   double* __restrict__ r, int64_t nrows,
+                                                                   double* __restrict__ partial) {
+  double d = 0.0;
+  spmvRows<G, double>(rowptr, sellStart, scol, val, x, nrows, blockIdx.x, [&](int64_t i, double kx) {
+    const double ri = b[i] - kx;
+    r[i]            = ri;
+    d += ri * ri;
+  });
   const double s = blockSum<SPMV_BS>(d);
   if (threadIdx.x == 0) partial[blockIdx.x] = s;
 }
@@ -234,7 +394,8 @@ __global__ __launch_bounds__(256) void dotKernel(const double* __restrict__ a, c
   if (threadIdx.x == 0) partial[blockIdx.x] = s;
 }
 
-__global__ __launch_bounds__(1024) void foldKernel(const double* __restrict__ partial, int n, double* __restrict__ out) {
+__global__ __launch_bounds__(1024) void foldKernel(const double* __restrict__ partial, int n,
+                                                   double* __restrict__ out) {
   double s = 0.0;
   for (int i = threadIdx.x; i < n; i += 1024) s += partial[i];
   s = blockSum<1024>(s);
@@ -256,10 +417,10 @@ __global__ void jacobiDiagKernel(const int32_t* __restrict__ diag, const double*
   dinv[i]            = d != 0.0 ? 1.0 / d : 1.0;
 }
 
-// r = b, x = 0, p = Dinv r; partials of rr and rz
+// r = b, x = 0, p = Dinv r (with z: z = Dinv r and p = 0); partials of rr and rz
 __global__ __launch_bounds__(256) void pcgInitKernel(const double* __restrict__ b, const double* __restrict__ dinv,
                                                      double* __restrict__ x, double* __restrict__ r,
-                                                     double* __restrict__ p, int64_t n,
+                                                     double* __restrict__ p, double* __restrict__ zOut, int64_t n,
                                                      double* __restrict__ partial /* 2*grid */) {
   double rr = 0.0, rz = 0.0;
   for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) {
@@ -267,7 +428,8 @@ __global__ __launch_bounds__(256) void pcgInitKernel(const double* __restrict__ 
     x[i]            = 0.0;
     r[i]            = bi;
     const double z  = dinv[i] * bi;
-    p[i]            = z;
+    p[i]            = zOut ? 0.0 : z;
+    if (zOut) zOut[i] = z;
     rr += bi * bi;
     rz += bi * z;
   }
@@ -320,25 +482,53 @@ __global__ __launch_bounds__(256) void pcgPqFold(const double* __restrict__ part
 
 // alpha = r.z / p.q (every block folds the npq values pq[] -- pcgPqFold's kPqBlocks sums or the SpMV's
 // partials -- in the same order, so all blocks agree bitwise; block 0 records the scalars), then
-// x += alpha p, r -= alpha q with partials of r.r and r.z (z = M^-1 r)
-template <typename T>
+// x += alpha p, r -= alpha q with partials of r.r and r.z (z = M^-1 r, stored when zOut is given)
+template <typename T, bool BLOCK>
 __global__ __launch_bounds__(256) void pcgUpdateKernel(T* __restrict__ x, T* __restrict__ r,
                                                        const T* __restrict__ p, const T* __restrict__ q,
-                                                       const T* __restrict__ pre, int blockPre, int64_t n,
-                                                       PcgScalars* __restrict__ sc, const double* __restrict__ pq,
-                                                       int npq, double* __restrict__ partial /* 2*grid */) {
-  if (sc->done) return;
+                                                       const T* __restrict__ pre, T* __restrict__ zOut,
+                                                       int64_t n, PcgScalars* __restrict__ sc,
+                                                       const double* __restrict__ pq, int npq,
+                                                       double* __restrict__ partial /* 2*grid */) {
+  const int done = sc->done;
+  // N entries per unit: one, or a node's three with the 3x3 block of the preconditioner
+  constexpr int N = BLOCK ? 3 : 1;
+  struct Unit {
+    T x[N], r[N], p[N], q[N], m[N * N];
+  };
+  auto load = [&](int64_t u, Unit& v) {
+#pragma unroll
+    for (int k = 0; k < N; ++k) {
+      v.x[k] = x[u * N + k];
+      v.r[k] = r[u * N + k];
+      v.p[k] = p[u * N + k];
+      v.q[k] = q[u * N + k];
+    }
+#pragma unroll
+    for (int k = 0; k < N * N; ++k) v.m[k] = pre[u * N * N + k];
+  };
+  const int64_t nu = n / N;
+  int64_t u        = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  Unit v;
+  if (u < nu) load(u, v);
+  const double rzNew = sc->rz_new;  // r.z of the current iterate (set by the previous p update)
+  double pqSum       = (int)threadIdx.x < npq ? pq[threadIdx.x] : 0.0;
+  arrived(v.x);
+  arrived(v.r);
+  arrived(v.p);
+  arrived(v.q);
+  arrived(v.m);
+  arrived(pqSum);
+  if (done) return;
   __shared__ double alphaS;
   {
-    double v = 0.0;
-    for (int i = threadIdx.x; i < npq; i += 256) v += pq[i];
-    v = blockSum<256>(v);
+    for (int i = threadIdx.x + 256; i < npq; i += 256) pqSum += pq[i];
+    pqSum = blockSum<256>(pqSum);
     if (threadIdx.x == 0) {
-      const double rz = sc->rz_new;  // r.z of the current iterate (set by the previous p update)
-      alphaS          = rz / v;
+      alphaS = rzNew / pqSum;
       if (blockIdx.x == 0) {
-        sc->rz    = rz;
-        sc->pq    = v;
+        sc->rz    = rzNew;
+        sc->pq    = pqSum;
         sc->alpha = alphaS;
       }
     }
@@ -346,30 +536,26 @@ __global__ __launch_bounds__(256) void pcgUpdateKernel(T* __restrict__ x, T* __r
   }
   const T alpha = (T)alphaS;
   double rr = 0.0, rz = 0.0;
-  if (!blockPre) {
-    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) {
-      x[i] += alpha * p[i];
-      const T ri = r[i] - alpha * q[i];
-      r[i]       = ri;
-      rr += (double)ri * (double)ri;
-      rz += (double)ri * (double)(pre[i] * ri);
-    }
-  } else {
-    const int64_t nn = n / 3;
-    for (int64_t nd = (int64_t)blockIdx.x * 256 + threadIdx.x; nd < nn; nd += (int64_t)gridDim.x * 256) {
-      T rl[3];
+  while (u < nu) {
+    T z[N];
 #pragma unroll
-      for (int k = 0; k < 3; ++k) {
-        const int64_t i = nd * 3 + k;
-        x[i] += alpha * p[i];
-        rl[k] = r[i] - alpha * q[i];
-        r[i]  = rl[k];
-        rr += (double)rl[k] * (double)rl[k];
-      }
-      const T* B = pre + nd * 9;
-#pragma unroll
-      for (int k = 0; k < 3; ++k) rz += (double)rl[k] * (double)(B[k * 3] * rl[0] + B[k * 3 + 1] * rl[1] + B[k * 3 + 2] * rl[2]);
+    for (int k = 0; k < N; ++k) {
+      x[u * N + k] = v.x[k] + alpha * v.p[k];
+      v.r[k] -= alpha * v.q[k];
+      r[u * N + k] = v.r[k];
+      rr += (double)v.r[k] * (double)v.r[k];
     }
+#pragma unroll
+    for (int k = 0; k < N; ++k) {
+      if constexpr (BLOCK)
+        z[k] = v.m[3 * k] * v.r[0] + v.m[3 * k + 1] * v.r[1] + v.m[3 * k + 2] * v.r[2];
+      else
+        z[k] = v.m[0] * v.r[0];
+      if (zOut) zOut[u * N + k] = z[k];
+      rz += (double)v.r[k] * (double)z[k];
+    }
+    u += (int64_t)gridDim.x * 256;
+    if (u < nu) load(u, v);
   }
   rr = blockSum<256>(rr);
   rz = blockSum<256>(rz);
@@ -379,56 +565,50 @@ __global__ __launch_bounds__(256) void pcgUpdateKernel(T* __restrict__ x, T* __r
   }
 }
 
-// Convergence test, beta and p = M^-1 r + beta p in one launch. Every block folds the update kernel's
-// partials (rr, rz) itself in the same fixed order, so all blocks agree bitwise; block 0 records the
-// scalars. beta = rz_new / rz uses the r.z of the previous iterate, which only pcgAlphaFold writes.
-template <typename T>
+// Convergence test, beta and p = M^-1 r + beta p in one launch
+template <typename T, bool BLOCK>
 __global__ __launch_bounds__(256) void pcgBetaPKernel(T* __restrict__ p, const T* __restrict__ r,
-                                                      const T* __restrict__ pre, int blockPre, int64_t n,
+                                                      const T* __restrict__ pre, int64_t n,
                                                       const double* __restrict__ partial, int nb,
                                                       PcgScalars* __restrict__ sc, int maxIter) {
-  if (sc->done) return;
-  __shared__ double bc[2];
-  double rr = 0.0, rz = 0.0;
-  for (int i = threadIdx.x; i < nb; i += 256) {
-    rr += partial[i];
-    rz += partial[nb + i];
-  }
-  rr = blockSum<256>(rr);
-  rz = blockSum<256>(rz);
-  if (threadIdx.x == 0) {
-    bc[0] = rr;
-    bc[1] = rz;
-  }
-  __syncthreads();
-  rr              = bc[0];
-  rz              = bc[1];
-  const bool conv = rr < sc->threshold;
-  const double bt = rz / sc->rz;
-  if (blockIdx.x == 0 && threadIdx.x == 0) {
-    sc->rr = rr;
-    if (conv) {
-      sc->done = 1;
-    } else {
-      sc->beta   = bt;
-      sc->rz_new = rz;
-      sc->iters += 1;
-      if (sc->iters >= maxIter) sc->done = 2;
-    }
-  }
-  if (conv) return;
-  const T beta = (T)bt;
-  if (!blockPre) {
-    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256)
-      p[i] = pre[i] * r[i] + beta * p[i];
-  } else {
-    const int64_t nn = n / 3;
-    for (int64_t nd = (int64_t)blockIdx.x * 256 + threadIdx.x; nd < nn; nd += (int64_t)gridDim.x * 256) {
-      const T r0 = r[nd * 3], r1 = r[nd * 3 + 1], r2 = r[nd * 3 + 2];
-      const T* B = pre + nd * 9;
+  const int done = sc->done;
+  PcgTest<256> t;
+  t.fetch(partial, nb, sc);
+  constexpr int N = BLOCK ? 3 : 1;
+  struct Unit {
+    T r[N], p[N], m[N * N];
+  };
+  auto load = [&](int64_t u, Unit& v) {
 #pragma unroll
-      for (int k = 0; k < 3; ++k) p[nd * 3 + k] = B[k * 3] * r0 + B[k * 3 + 1] * r1 + B[k * 3 + 2] * r2 + beta * p[nd * 3 + k];
+    for (int k = 0; k < N; ++k) {
+      v.r[k] = r[u * N + k];
+      v.p[k] = p[u * N + k];
     }
+#pragma unroll
+    for (int k = 0; k < N * N; ++k) v.m[k] = pre[u * N * N + k];
+  };
+  const int64_t nu = n / N;
+  int64_t u        = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  Unit v;
+  if (u < nu) load(u, v);
+  arrived(v.r);
+  arrived(v.p);
+  arrived(v.m);
+  t.wait();
+  if (done) return;
+  double bt;
+  if (!t.test(maxIter, blockIdx.x == 0, bt)) return;
+  const T beta = (T)bt;
+  while (u < nu) {
+#pragma unroll
+    for (int k = 0; k < N; ++k) {
+      if constexpr (BLOCK)
+        p[u * N + k] = v.m[3 * k] * v.r[0] + v.m[3 * k + 1] * v.r[1] + v.m[3 * k + 2] * v.r[2] + beta * v.p[k];
+      else
+        p[u * N + k] = v.m[0] * v.r[0] + beta * v.p[0];
+    }
+    u += (int64_t)gridDim.x * 256;
+    if (u < nu) load(u, v);
   }
 }
 
@@ -462,7 +642,8 @@ __global__ void blockInvKernel(const int32_t* __restrict__ diag, const float* __
 // FP32 PCG init from an FP64 right-hand side scaled by 1/s (s = ||r||, keeps FP32 in range)
 __global__ __launch_bounds__(256) void pcgInitF32(const double* __restrict__ b, double invScale,
                                                   const float* __restrict__ binv, float* __restrict__ x,
-                                                  float* __restrict__ r, float* __restrict__ p, int64_t nn,
+                                                  float* __restrict__ r, float* __restrict__ p,
+                                                  float* __restrict__ zOut, int64_t nn,
                                                   double* __restrict__ partial) {
   double rr = 0.0, rz = 0.0;
   for (int64_t nd = (int64_t)blockIdx.x * 256 + threadIdx.x; nd < nn; nd += (int64_t)gridDim.x * 256) {
@@ -478,7 +659,8 @@ __global__ __launch_bounds__(256) void pcgInitF32(const double* __restrict__ b, 
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
       const float z = B[k * 3] * rl[0] + B[k * 3 + 1] * rl[1] + B[k * 3 + 2] * rl[2];
-      p[nd * 3 + k] = z;
+      p[nd * 3 + k] = zOut ? 0.0f : z;
+      if (zOut) zOut[nd * 3 + k] = z;
       rz += (double)rl[k] * (double)z;
     }
   }
@@ -526,46 +708,80 @@ static double* pq2(ik_handle* h) { return h->partial.p + h->partial.n - 8 - kPqB
 // kernel reads the former while its blocks write the latter)
 static double* pqPartials(ik_handle* h) { return h->partial.p + 2 * kReduceBlocks; }
 
+// Wavefronts that share a row group of the SpMV (G), and whether the PCG forms its direction inside the SpMV. us per
+// PCG iteration, hex8 grids of 20^3 / 27^3 / 34^3 / 42^3 / 52^3 elements (9,261 to 148,877 nodes):
+//  FP64 Jacobi        G = 1: 16.5 / 18.6 / 24.5 / 37.6 / 65.0   G = 4: 12.8 / 18.3 / 27.8 / 40.2 / 69.0
+//                     G = 4, direction in the SpMV: 12.8 / 19.4 / 28.9 / 47.8 / 94.2 (8^3: 10.6 against 13.0 for G = 1)
+//  FP32 block Jacobi  G = 1: 17.9 / 19.3 / 19.7 / 23.9 / 37.4   G = 4: 15.8 / 17.1 / 19.1 / 24.3 / 37.5
+//                     G = 4, direction in the SpMV: 10.9 / 13.5 / 16.6 / 23.5 / 38.7
+// Shuffled element order at 42^3: FP64 43.0 (G = 1) and 49.1; FP32 34.8 (G = 1), 29.2 and 36.5 with the direction.
+// Small systems lack wavefronts and are bound by the chain of loads of one row and by launches (a host that launches
+// slowly: 198 ms against 154 for ten plane load steps at 2,210 nodes with the same split), so the split and the launch
+// saved count; large ones are bound by bytes and prefer long runs of one wavefront.
+constexpr int64_t kSplitRows64 = 15000, kSplitRows32 = 120000;
+constexpr int64_t kDirectionRows64 = kSplitRows64, kDirectionRows32 = 50000;
+constexpr int kSplit = 4;
+template <typename TV>
+static bool directionInSpmv(int64_t nn) {
+  return nn <= (sizeof(TV) == 4 ? kDirectionRows32 : kDirectionRows64);
+}
+// calls f(std::integral_constant<int, G>) for the split of TV's layout on nn rows
+template <typename TV, typename F>
+static void withSplit(int64_t nn, F f) {
+  if (nn <= (sizeof(TV) == 4 ? kSplitRows32 : kSplitRows64))
+    f(std::integral_constant<int, kSplit>{});
+  else
+    f(std::integral_constant<int, 1>{});
+}
+template <typename TV>
+static unsigned spmvGrid(int64_t nn) {
+  unsigned g = 0;
+  withSplit<TV>(nn, [&](auto G) {
+    constexpr int R = spmvRowsPerBlock<TV, decltype(G)::value>();
+    g               = (unsigned)((nn + R - 1) / R);
+  });
+  return g;
+}
+
 // partial[] holds one launch's per-block partials at its start, the PCG SpMV's partials from 2 kReduceBlocks
 // on, the p.q first-stage sums (kPqBlocks) in a region of their own before the last 8 entries, and fold
 // results in its last entry
 static void ensureWork(ik_handle* h) {
-  const int64_t n = h->ndof;
-  const int64_t spmvBlocks = spmvGrid<double>(h->nn);  // the FP64 layout launches the most blocks
+  const int64_t spmvBlocks = std::max(spmvGrid<double>(h->nn), spmvGrid<float>(h->nn));
   h->partial.ensure((size_t)(2 * kReduceBlocks + spmvBlocks) + kPqBlocks + 8);
   if (!h->sc.p) {
     h->sc.ensure(1);
     IK_HIP(hipHostMalloc((void**)&h->hsc, sizeof(PcgScalars), hipHostMallocDefault));
     IK_HIP(hipHostMalloc((void**)&h->hred, sizeof(double) * 4, hipHostMallocDefault));
   }
-  (void)n;
+}
+
+// y = K x (partial: with x.y partials per block, and skipped once sc->done)
+template <typename TV, typename TX>
+static void launchSpmv(ik_handle* h, const TV* K, const TX* x, TX* y, double* partial, const PcgScalars* sc, int rev) {
+  ScopedKernelTimer t(h, KSPMV);
+  const unsigned grid = spmvGrid<TV>(h->nn);
+  withSplit<TV>(h->nn, [&](auto G) {
+    constexpr int g = decltype(G)::value;
+    if (partial)
+      hipLaunchKernelGGL((spmvKernel<TV, TX, true, g>), dim3(grid), dim3(SPMV_BS), 0, h->stream, h->rowptr.p,
+                         h->sellStart.p, h->scol.p, K, x, y, h->nn, partial, sc, rev);
+    else
+      hipLaunchKernelGGL((spmvKernel<TV, TX, false, g>), dim3(grid), dim3(SPMV_BS), 0, h->stream, h->rowptr.p,
+                         h->sellStart.p, h->scol.p, K, x, y, h->nn, nullptr, nullptr, 0);
+  });
 }
 
 void spmv64(ik_handle* h, const double* x, double* y) {
   ensureWork(h);
-  const unsigned grid = spmvGrid<double>(h->nn);
-  ScopedKernelTimer t(h, KSPMV);
-  hipLaunchKernelGGL((spmvKernel<double, double, false>), dim3(grid), dim3(SPMV_BS), 0, h->stream, h->rowptr.p,
-                     h->sellStart.p, h->scol.p, h->K64.p, x, y, h->nn, nullptr, nullptr, 0);
-}
-
-void spmv32(ik_handle* h, const float* x, float* y) {
-  ensureWork(h);
-  const unsigned grid = spmvGrid<float>(h->nn);
-  ScopedKernelTimer t(h, KSPMV);
-  hipLaunchKernelGGL((spmvKernel<float, float, false>), dim3(grid), dim3(SPMV_BS), 0, h->stream, h->rowptr.p,
-                     h->sellStart.p, h->scol.p, h->K32.p, x, y, h->nn, nullptr, nullptr, 0);
+  launchSpmv<double, double>(h, h->K64.p, x, y, nullptr, nullptr, 0);
 }
 
 double dot(ik_handle* h, const double* a, const double* b, int64_t n) {
   ensureWork(h);
   const int g = vecGrid(n);
   hipLaunchKernelGGL(dotKernel, dim3(g), dim3(256), 0, h->stream, a, b, n, h->partial.p);
-  hipLaunchKernelGGL(foldKernel, dim3(1), dim3(1024), 0, h->stream, h->partial.p, g, h->partial.p + h->partial.n - 1);
-  IK_HIP(hipMemcpyAsync(h->hred, h->partial.p + h->partial.n - 1, sizeof(double), hipMemcpyDeviceToHost, h->stream));
-  IK_HIP(hipStreamSynchronize(h->stream));
-  finishErrCheck(h);
-  return h->hred[0];
+  return foldPartials(h, g);
 }
 
 double* partialsFor(ik_handle* h, int nb) {
@@ -586,42 +802,30 @@ void axpy(ik_handle* h, double a, const double* x, double* y, int64_t n) {
   hipLaunchKernelGGL(axpyKernel, dim3(vecGrid(n)), dim3(256), 0, h->stream, a, x, y, n);
 }
 
-void residualBlock64(ik_handle* h, const double* b, const double* x, double* r) {
-  ensureWork(h);
-  const unsigned grid = spmvGrid<double>(h->nn);
-  hipLaunchKernelGGL((residualKernel<double>), dim3(grid), dim3(SPMV_BS), 0, h->stream, h->rowptr.p, h->sellStart.p,
-                     h->scol.p, h->K64.p, x, b, r, h->nn, h->partial.p);
-}
-
 // Poll interval: iterations enqueued before the first host check of the done flag (32: a two-level inner solve
 // takes 24-32 at 64^3, so most need no second check) and between later checks (64). Iterations enqueued after
 // convergence return at once (a few us of launches each); a check leaves the device idle for a host round trip
 // (20-45 us) while the next iterations are enqueued.
 static int pollChunk(int enq) { return enq == 0 ? 32 : 64; }
 
-void pcgJacobi64(ik_handle* h, const double* b, double* x, double rtol, int maxIter, int* iters, double* relres) {
-  ensureWork(h);
-  const int64_t n = h->ndof;
-  h->pr.ensure(n);
-  h->pp.ensure(n);
-  h->pq.ensure(n);
-  h->pdiag.ensure(n);
-  const int g = vecGrid(n);
-  const unsigned sgrid = spmvGrid<double>(h->nn);
-  hipLaunchKernelGGL(jacobiDiagKernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, h->stream, h->diagBlk.p,
-                     h->K64.p, h->nn, h->pdiag.p);
-  hipLaunchKernelGGL(pcgInitKernel, dim3(g), dim3(256), 0, h->stream, b, h->pdiag.p, x, h->pr.p, h->pp.p, n,
-                     h->partial.p);
-  hipLaunchKernelGGL(pcgInitFold, dim3(1), dim3(1024), 0, h->stream, h->partial.p, g, rtol * rtol, h->sc.p);
-  if (maxIter <= 0) maxIter = (int)(2 * n);
-  int enq = 0;
+// The iterations of one PCG solve, after its init kernels: enqueued in chunks until the done flag or maxIter. p holds
+// the first direction, or zero with z = M^-1 r when z is given (the direction is then formed inside the SpMV,
+// alternating between p and p2). coarse: the two-level form's vector kernels instead of update and direction.
+template <typename T>
+static void pcgLoop(ik_handle* h, const T* K, T* x, T* r, T* p, T* p2, T* z, T* q, const T* pre, int64_t n,
+                    int grid, int maxIter, bool coarse) {
+  const unsigned sgrid = spmvGrid<T>(h->nn);
+  int enq              = 0;
   for (;;) {
     for (int c = 0, cn = pollChunk(enq); c < cn && enq < maxIter; ++c, ++enq) {
-      {
+      if (z) {
+        if (enq > 0) std::swap(p, p2);
         ScopedKernelTimer t(h, KSPMV);
-        hipLaunchKernelGGL((spmvKernel<double, double, true>), dim3(sgrid), dim3(SPMV_BS), 0, h->stream, h->rowptr.p,
-                           h->sellStart.p, h->scol.p, h->K64.p, h->pp.p, h->pq.p, h->nn, pqPartials(h), h->sc.p,
-                           enq & 1);
+        hipLaunchKernelGGL((pcgDirectionSpmv<T, kSplit>), dim3(sgrid), dim3(SPMV_BS), 0, h->stream, h->rowptr.p,
+                           h->sellStart.p, h->scol.p, K, z, p, p2, q, h->nn, h->partial.p, grid, pqPartials(h),
+                           h->sc.p, maxIter, c > 0 ? 1 : 0);
+      } else {
+        launchSpmv<T, T>(h, K, p, q, pqPartials(h), h->sc.p, enq & 1);
       }
       const double* pqSrc = pqPartials(h);
       int npq             = (int)sgrid;
@@ -631,16 +835,48 @@ void pcgJacobi64(ik_handle* h, const double* b, double* x, double rtol, int maxI
         pqSrc = pq2(h);
         npq   = kPqBlocks;
       }
-      hipLaunchKernelGGL((pcgUpdateKernel<double>), dim3(g), dim3(256), 0, h->stream, x, h->pr.p, h->pp.p, h->pq.p,
-                         h->pdiag.p, 0, n, h->sc.p, pqSrc, npq, h->partial.p);
-      hipLaunchKernelGGL((pcgBetaPKernel<double>), dim3(g), dim3(256), 0, h->stream, h->pp.p, h->pr.p, h->pdiag.p, 0,
-                         n, h->partial.p, g, h->sc.p, maxIter);
+      if constexpr (std::is_same<T, float>::value)
+        if (coarse) {
+          coarseIteration(h, pqSrc, npq, x, r, p, q, pre, grid, h->partial.p, maxIter);
+          continue;
+        }
+      constexpr bool B = std::is_same<T, float>::value;  // FP64: diagonal preconditioner, FP32: 3x3 blocks
+      hipLaunchKernelGGL((pcgUpdateKernel<T, B>), dim3(grid), dim3(256), 0, h->stream, x, r, z ? p2 : p, q, pre, z, n,
+                         h->sc.p, pqSrc, npq, h->partial.p);
+      if (!z)
+        hipLaunchKernelGGL((pcgBetaPKernel<T, B>), dim3(grid), dim3(256), 0, h->stream, p, r, pre, n, h->partial.p,
+                           grid, h->sc.p, maxIter);
     }
+    if (z)
+      hipLaunchKernelGGL(pcgTestKernel, dim3(1), dim3(256), 0, h->stream, h->partial.p, grid, h->sc.p, maxIter);
     IK_HIP(hipMemcpyAsync(h->hsc, h->sc.p, sizeof(PcgScalars), hipMemcpyDeviceToHost, h->stream));
     IK_HIP(hipStreamSynchronize(h->stream));
     finishErrCheck(h);
     if (h->hsc->done || enq >= maxIter) break;
   }
+}
+
+void pcgJacobi64(ik_handle* h, const double* b, double* x, double rtol, int maxIter, int* iters, double* relres) {
+  ensureWork(h);
+  const int64_t n  = h->ndof;
+  const bool fused = directionInSpmv<double>(h->nn);
+  h->pr.ensure(n);
+  h->pp.ensure(n);
+  h->pq.ensure(n);
+  h->pdiag.ensure(n);
+  if (fused) {
+    h->pz.ensure(n);
+    h->pb.ensure(n);
+  }
+  double* z   = fused ? h->pz.p : nullptr;
+  const int g = vecGrid(n);
+  hipLaunchKernelGGL(jacobiDiagKernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, h->stream, h->diagBlk.p,
+                     h->K64.p, h->nn, h->pdiag.p);
+  hipLaunchKernelGGL(pcgInitKernel, dim3(g), dim3(256), 0, h->stream, b, h->pdiag.p, x, h->pr.p, h->pp.p, z, n,
+                     h->partial.p);
+  hipLaunchKernelGGL(pcgInitFold, dim3(1), dim3(1024), 0, h->stream, h->partial.p, g, rtol * rtol, h->sc.p);
+  if (maxIter <= 0) maxIter = (int)(2 * n);
+  pcgLoop<double>(h, h->K64.p, x, h->pr.p, h->pp.p, h->pb.p, z, h->pq.p, h->pdiag.p, n, g, maxIter, false);
   *iters  = h->hsc->iters;
   *relres = h->hsc->bb > 0 ? std::sqrt(h->hsc->rr / h->hsc->bb) : 0.0;
 }
@@ -649,6 +885,7 @@ void pcgMixed(ik_handle* h, const double* b, double* x, const ik_solver_opts* o,
               double bnormKnown) {
   ensureWork(h);
   const bool twoLevel = o->kind == IK_PCG_TWOLEVEL_FP32_IR;
+  const bool fused    = !twoLevel && directionInSpmv<float>(h->nn);
   const int64_t n = h->ndof;
   h->fr.ensure(n);
   h->fp.ensure(n);
@@ -656,6 +893,11 @@ void pcgMixed(ik_handle* h, const double* b, double* x, const ik_solver_opts* o,
   h->fx.ensure(n);
   h->fdiag.ensure((size_t)h->nn * 9);
   h->pr.ensure(n);
+  if (fused) {
+    h->fz.ensure(n);
+    h->fp2.ensure(n);
+  }
+  float* z    = fused ? h->fz.p : nullptr;
   const int g = vecGrid(n);
   // vector kernels over nodes: 512 blocks (the p update folds 2 partials per block in every block; 512 vs
   // 1024 blocks measured 2.28 vs 2.31 s on the 64^3 mixed Newton path)
@@ -689,54 +931,21 @@ void pcgMixed(ik_handle* h, const double* b, double* x, const ik_solver_opts* o,
       coarseApply(h, h->fr.p, h->fp.p, nullptr, h->fdiag.p, gn, h->partial.p);  // p = z
     } else {
       hipLaunchKernelGGL(pcgInitF32, dim3(gn), dim3(256), 0, h->stream, h->pr.p, 1.0 / rnorm, h->fdiag.p, h->fx.p,
-                         h->fr.p, h->fp.p, h->nn, h->partial.p);
+                         h->fr.p, h->fp.p, z, h->nn, h->partial.p);
     }
     hipLaunchKernelGGL(pcgInitFold, dim3(1), dim3(1024), 0, h->stream, h->partial.p, gn, innerTol * innerTol,
                        h->sc.p);
-    int enq = 0;
-    for (;;) {
-      for (int c = 0, cn = pollChunk(enq); c < cn && enq < maxIter; ++c, ++enq) {
-        {
-          ScopedKernelTimer t(h, KSPMV);
-          hipLaunchKernelGGL((spmvKernel<float, float, true>), dim3(sgrid), dim3(SPMV_BS), 0, h->stream,
-                             h->rowptr.p, h->sellStart.p, h->scol.p, h->K32.p, h->fp.p, h->fq.p, h->nn,
-                             pqPartials(h), h->sc.p, enq & 1);
-        }
-        const double* pqSrc = pqPartials(h);
-        int npq             = (int)sgrid;
-        if (sgrid > (unsigned)kPqDirect) {
-          hipLaunchKernelGGL(pcgPqFold, dim3(kPqBlocks), dim3(256), 0, h->stream, pqPartials(h), (int)sgrid,
-                             pq2(h), h->sc.p);
-          pqSrc = pq2(h);
-          npq   = kPqBlocks;
-        }
-        if (twoLevel) {
-          coarseIteration(h, pqSrc, npq, h->fx.p, h->fr.p, h->fp.p, h->fq.p, h->fdiag.p, gn, h->partial.p, maxIter);
-          continue;
-        }
-        hipLaunchKernelGGL((pcgUpdateKernel<float>), dim3(gn), dim3(256), 0, h->stream, h->fx.p, h->fr.p, h->fp.p,
-                           h->fq.p, h->fdiag.p, 1, n, h->sc.p, pqSrc, npq, h->partial.p);
-        hipLaunchKernelGGL((pcgBetaPKernel<float>), dim3(gn), dim3(256), 0, h->stream, h->fp.p, h->fr.p, h->fdiag.p,
-                           1, n, h->partial.p, gn, h->sc.p, maxIter);
-      }
-      IK_HIP(hipMemcpyAsync(h->hsc, h->sc.p, sizeof(PcgScalars), hipMemcpyDeviceToHost, h->stream));
-      IK_HIP(hipStreamSynchronize(h->stream));
-      finishErrCheck(h);
-      if (h->hsc->done || enq >= maxIter) break;
-    }
+    pcgLoop<float>(h, h->K32.p, h->fx.p, h->fr.p, h->fp.p, h->fp2.p, z, h->fq.p, h->fdiag.p, n, gn, maxIter, twoLevel);
     info->iterations += h->hsc->iters + 1;
     info->refinements += 1;
     // x += ||r|| d ; r = b - K x in FP64
     hipLaunchKernelGGL(accumulateF32, dim3(g), dim3(256), 0, h->stream, x, h->fx.p, rnorm, n);
-    hipLaunchKernelGGL((residualKernel<float>), dim3(sgrid), dim3(SPMV_BS), 0, h->stream, h->rowptr.p, h->sellStart.p,
-                       h->scol.p, h->K32.p, x, b, h->pr.p, h->nn, h->partial.p);
-    hipLaunchKernelGGL(foldKernel, dim3(1), dim3(1024), 0, h->stream, h->partial.p, (int)sgrid,
-                       h->partial.p + h->partial.n - 1);
-    IK_HIP(hipMemcpyAsync(h->hred, h->partial.p + h->partial.n - 1, sizeof(double), hipMemcpyDeviceToHost,
-                          h->stream));
-    IK_HIP(hipStreamSynchronize(h->stream));
-    finishErrCheck(h);
-    rnorm              = std::sqrt(h->hred[0]);
+    withSplit<float>(h->nn, [&](auto G) {
+      constexpr int gs = decltype(G)::value;
+      hipLaunchKernelGGL((residualKernel<float, gs>), dim3(sgrid), dim3(SPMV_BS), 0, h->stream, h->rowptr.p,
+                         h->sellStart.p, h->scol.p, h->K32.p, x, b, h->pr.p, h->nn, h->partial.p);
+    });
+    rnorm              = std::sqrt(foldPartials(h, (int)sgrid));
     info->rel_residual = rnorm / bnorm;
     if (info->rel_residual <= o->rtol) {
       info->converged = 1;
