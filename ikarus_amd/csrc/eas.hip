@@ -11,20 +11,28 @@
 //   alpha <- alpha - D^{-1}(Rt + L du_e) on CORRECTION_UPDATED, with D, L, Rt of the state the tangent
 //   was assembled at (the reference recomputes them at that same state).
 //
-// One 64-lane workgroup (one wave) per element, all lanes busy in every phase: Gauss-point kinematics and
-// material per (point, node) lane pair, K_uu in the Ci form per (node, node) lane pair, D / L / Rt / R_u by
-// owned entries, forward elimination of [D | L | Rt] one column per lane (D = L_D diag(d) L_D^T), and the
-// rank-21 update of K and R. Outputs go to the same element-by-element staging as the plain element (36 upper
-// blocks + 24 residual entries), plus the cache of the alpha update: diag(d)^{-1} L_D^{-1} L (21x24),
-// diag(d)^{-1} L_D^{-1} Rt (21) and L_D (210), so that D^{-1} v = L_D^{-T} diag(d)^{-1} L_D^{-1} v.
+// One contraction gives everything but the geometric stiffness: with the 6 x 48 matrix N = [M | B | 0] per Gauss point
+// (21 mode columns, 24 displacement columns) and CN = [C dV M | C dV B | S dV | 0], sum over the points of N^T CN holds
+// D, L, Rt, the material part of K_uu and R_u as one symmetric 48 x 48 array of 16 x 16 matrix-core tiles; block
+// elimination of the 21 mode rows in those tiles leaves K and R. Outputs go to the same element-by-element staging as
+// the plain element (36 upper blocks + 24 residual entries), plus the cache of the alpha update.
 #include "ik_internal.hh"
+#include "wave_reduce.hh"
 
 namespace ik {
 namespace {
 
 constexpr int NE = 21;  // enhanced modes
-// doubles per element of the alpha-update cache: What (24 columns of 21), what (21), the strictly lower L_D (210)
-constexpr int kEasCache = NE * 24 + NE + NE * (NE - 1) / 2;
+typedef double v2d __attribute__((ext_vector_type(2)));
+typedef double v4d __attribute__((ext_vector_type(4)));
+
+// The alpha-update cache of an element: the rows What = Db^-1 Lb^-1 [.| L | Rt] of the block elimination
+// D = Lb Db Lb^T (panels p of mode rows 4 p .. 4 p + 3, the last of row 20 alone), as the chunks in which the
+// element kernel holds them (row k of a panel, column c of [D | L | Rt]): columns 16..31 of panel p at
+// 64 p + 16 k + (c - 16), columns 32..45 at 320 + 56 p + 14 k + (c - 32), columns 4 (p + 1)..15 of panels 0-2 behind
+// 600, columns 21..45 of row 20 at 696. The stride is a multiple of 64 bytes.
+constexpr int kEasCache = 728;
+__host__ __device__ constexpr int cacheLow(int p) { return p == 0 ? 600 : (p == 1 ? 648 : 680); }
 
 __host__ __device__ constexpr int vI(int v) { return v < 3 ? v : (v == 3 ? 1 : 0); }
 __host__ __device__ constexpr int vJ(int v) { return v < 3 ? v : (v == 5 ? 1 : 2); }
@@ -33,78 +41,26 @@ __host__ __device__ constexpr int sym6(int p, int q) {
 }
 __host__ __device__ constexpr int upperBlock(int a, int b) { return 8 * a - (a * (a - 1)) / 2 + (b - a); }
 
-// Row-major upper triangle of an n x n matrix: entry idx in [0, n(n+1)/2) -> (row i, column c >= i). Rows
-// before i hold S(i) = i n - i(i-1)/2 entries, so i is the root of that quadratic, rounded down (the float
-// root is off by at most one, which the integer checks correct).
-__device__ inline void triDecode(int idx, int n, int& i, int& c) {
-  const float b = 2.0f * n + 1.0f;
-  int r         = (int)((b - sqrtf(fmaxf(b * b - 8.0f * idx, 0.0f))) * 0.5f);
-  r             = r < 0 ? 0 : (r > n - 1 ? n - 1 : r);
-  auto S        = [n](int k) { return k * n - (k * (k - 1)) / 2; };
-  if (r < n - 1 && S(r + 1) <= idx) ++r;
-  if (r > 0 && S(r) > idx) --r;
-  i = r;
-  c = r + (idx - S(r));
-}
-
-// E21 ansatz in reference coordinates: column c has one nonzero, in Voigt row kRow[c], of value
-// f_c(x, y, z) with x = 2 xi - 1 etc. (linearandglstrains.hh:300-322)
-__constant__ int kRow[NE] = {0, 1, 2, 3, 3, 4, 4, 5, 5, 3, 3, 4, 4, 5, 5, 0, 0, 1, 1, 2, 2};
+// E21 ansatz in reference coordinates (linearandglstrains.hh:300-322): column c has one nonzero, in Voigt row
+// kRowOf(c), of value f_c(x, y, z) with x = 2 xi - 1 etc., a product of the coordinates in the mask (bit 0: x, 1: y,
+// 2: z).
 __host__ __device__ constexpr int kRowOf(int c) {
   return c < 3 ? c : (c < 9 ? 3 + (c - 3) / 2 : (c < 15 ? 3 + (c - 9) / 2 : (c - 15) / 2));
 }
-__device__ inline double ansatz(int c, double x, double y, double z) {
-  switch (c) {
-    case 0: return x;
-    case 1: return y;
-    case 2: return z;
-    case 3: return y;
-    case 4: return z;
-    case 5: return x;
-    case 6: return z;
-    case 7: return x;
-    case 8: return y;
-    case 9: return x * y;
-    case 10: return x * z;
-    case 11: return x * y;
-    case 12: return y * z;
-    case 13: return x * z;
-    case 14: return y * z;
-    case 15: return x * y;
-    case 16: return x * z;
-    case 17: return x * y;
-    case 18: return y * z;
-    case 19: return x * z;
-    default: return y * z;
-  }
+__host__ __device__ constexpr int monomialOf(int c) {
+  constexpr int m[NE] = {1, 2, 4, 2, 4, 1, 4, 1, 2, 3, 5, 3, 6, 5, 6, 3, 5, 3, 6, 5, 6};
+  return m[c];
 }
-
-__device__ inline void dShape(int a, const double xi[3], double dN[3]) {
-  double f[3], s[3];
-  for (int k = 0; k < 3; ++k) {
-    const bool hi = (a >> k) & 1;
-    f[k]          = hi ? xi[k] : 1.0 - xi[k];
-    s[k]          = hi ? 1.0 : -1.0;
-  }
-  dN[0] = s[0] * f[1] * f[2];
-  dN[1] = f[0] * s[1] * f[2];
-  dN[2] = f[0] * f[1] * s[2];
+// both as 3-bit fields, for a lane's own column
+constexpr unsigned long long packModes(bool rows) {
+  unsigned long long v = 0;
+  for (int c = 0; c < NE; ++c) v |= (unsigned long long)(rows ? kRowOf(c) : monomialOf(c)) << (3 * c);
+  return v;
 }
 
 __device__ inline double det3(const double A[3][3]) {
   return A[0][0] * (A[1][1] * A[2][2] - A[1][2] * A[2][1]) - A[0][1] * (A[1][0] * A[2][2] - A[1][2] * A[2][0]) +
          A[0][2] * (A[1][0] * A[2][1] - A[1][1] * A[2][0]);
-}
-
-__device__ inline void jacobianAt(const double (*X)[3], const double xi[3], double J[3][3]) {
-  for (int i = 0; i < 3; ++i)
-    for (int j = 0; j < 3; ++j) J[i][j] = 0.0;
-  for (int a = 0; a < 8; ++a) {
-    double dN[3];
-    dShape(a, xi, dN);
-    for (int i = 0; i < 3; ++i)
-      for (int j = 0; j < 3; ++j) J[i][j] += X[a][i] * dN[j];
-  }
 }
 
 // value of lane `lane` (uniform) of a 64-bit register, as two 32-bit lane reads into scalar registers
@@ -115,67 +71,118 @@ __device__ inline double readLane(double x, int lane) {
   return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
 }
 
-// maximum over the 64 lanes of the wavefront (every lane active), as a uniform value
-__device__ inline double waveMax(double x) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) x = fmax(x, __shfl_xor(x, o, 64));
-  return readLane(x, 0);
+// 1/d by the hardware estimate and two Newton steps: within an ulp of the division, at a third of its instructions
+__device__ inline double reciprocal(double d) {
+  double r = __builtin_amdgcn_rcp(d);
+  r        = fma(fma(-d, r, 1.0), r, r);
+  return fma(fma(-d, r, 1.0), r, r);
 }
 
-// Voigt index of the symmetric pair (i, j): 00 11 22 12 02 01
-__host__ __device__ constexpr int v6(int i, int j) {
-  return i == j ? i : (i + j == 3 ? 3 : (i + j == 2 ? 4 : 5));
+// min(a, |b|); the compiler's fmin first quiets both operands, an instruction each
+__device__ inline double minAbs(double a, double b) {
+  double m;
+  asm("v_min_f64 %0, %1, |%2|" : "=v"(m) : "v"(a), "v"(b));
+  return m;
+}
+__device__ inline double minOf(double a, double b) {
+  double m;
+  asm("v_min_f64 %0, %1, %2" : "=v"(m) : "v"(a), "v"(b));
+  return m;
+}
+__device__ inline double maxAbs(double a, double b) {
+  double m;
+  asm("v_max_f64 %0, %1, |%2|" : "=v"(m) : "v"(a), "v"(b));
+  return m;
 }
 
-// One 64-lane workgroup (one wave) per element. The LDS (13.6 KB; 11.2 KB for the residual alone) holds two
-// unions: the K_uu inputs (later the parked K_uu blocks) and the point data of
-// the D / L / Rt loop (later the condensation operands).
-template <bool WANT_K>
+// orders the LDS accesses of one wavefront's lanes
+__device__ inline void waveSync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+}
+
+// One wavefront per workgroup takes E elements: it evaluates their 8 E Gauss points together, then condenses one element
+// after the other. The points' data stay in LDS (4 KB per element); an element's K and R replace them on their way out.
+// 96 x 96 x 48 elements, Neo-Hooke: 2.84 ms against 5.4 ms for the former kernel (one element per wavefront, sums by
+// owned entries), whose 1,300 LDS accesses per element alone need 3.7 ms. With E = 4; 2: 3.1 ms; 8 elements in 2 or 4
+// wavefronts: 2.9 and 3.1 ms; three wavefronts per SIMD at 168 registers: 3.3 ms with C in LDS, 4.3 ms with spills.
+// What bounds it now: the matrix and vector pipes one after the other (per element 99 MFMAs of 64 cycles and 1,350
+// vector instructions of 4: 2.3 ms); 3.8 GB are written (0.6 ms).
+// Meshes that leave SIMDs idle take fewer elements per wavefront; assembly and update with E = 1 / 2 / 4, us:
+//   512 elements 105 / 111 / 124, 2,048: 116 / 117 / 130, 9,216: 190 / 187 / 194, 18,432: 287 / 264 / 266,
+//   98,304: 1,146 / 1,035 / 988.
+constexpr int64_t kEasOne = 2048, kEasTwo = 16384;  // largest counts for E = 1 and 2
+constexpr double kGaussX  = 2.0 * 0.28867513459481288225;  // |x| of a Gauss point
+
+struct EasPoint {
+  double C[22];     // C dV (packed upper; one entry of padding)
+  double G[8][3];   // shape-function gradients g_a
+  double F[9];
+  double w;         // 1 / (detJ detJ0)
+  double S[6];      // S dV
+};
+static_assert(sizeof(EasPoint) == 62 * 8, "62 doubles: the four points of a step lie in different LDS banks");
+template <int E>
 struct EasLds {
-  static constexpr int NK = WANT_K ? 8 : 1;  // the residual-only kernel keeps no K_uu inputs
-  double X[8][3], U[8][3];
-  double alpha[NE];
-  double T0[6][6];  // (T(xi0) detJ0)^-1
   union {
     struct {
-      double G[8][8][3];  // [gp][node][dir] shape-function gradients g_a
-      double S[8][6];     // S dV
-      double P[NK][8][3]; // F Ci g_a
-      double Ci[NK][6];   // Ci (Voigt order), the identity for SVK
-      double Phi[NK][6];  // F Ci F^T (Voigt order)
-      double w[NK][2];    // lambda dV, c2 dV: material tangent weights of the Ci form
-    } k;
-    struct {
-      double Kuu[WANT_K ? 36 : 1][9];  // K_uu upper blocks while the elimination runs
-    } q;
-  } uk;
-  union {
-    struct {
-      double F[8][9];
-      double C[8][21];    // C dV (packed)
-      double f[8][NE];    // E21 mode scalings f_c(xi_gp) / detJ_gp: column c of M = T0^-1[:, kRow[c]] f_c
-      double CT[6][6];    // current point: C dV T0^-1
-      double Ch[6][6];    // T0^-T C dV T0^-1
-      double TS[6];       // T0^-T S dV
-      double Z[6][24];    // (C dV T0^-1)^T B
-      double ru[8][8][3]; // R_u contribution F S dV g_a of point gp, node a
-    } g;
-    struct {
-      double A[NE][24];   // D (columns 0-20), then What = diag(d)^-1 L_D^-1 L
-      double Lm[NE][24];  // L, then W = L_D^-1 L (row j written at elimination step j)
-      double rt[NE];      // Rt, then what = diag(d)^-1 L_D^-1 Rt
-      double Ru[24];
-    } c;
-  } u;
-  int bad;
+      double X[24], U[24], alpha[NE + 1];
+    } in;
+    EasPoint pt[8];
+    double out[36 * 9 + 24 + 4 + 64];  // K blocks, R, one slot per lane for entries that are not stored
+  } u[E];
+  double Ji0[E][10];  // inverse Jacobian at the centre
+  int bad[E];
 };
 
-// S and C (Voigt) at the enhanced strain, plus the factors of the tangent's Ci form
-// C = lambda Ci(x)Ci + c2 (Ci box Ci + transposed): Ci (Voigt) and c2 (Neo-Hooke: mu - lambda ln J; SVK: Ci = I,
-// c2 = mu)
+// Where the lanes of an element's wavefront put K and R into its output area, and find the blocks' entries there
+struct EasTables {
+  uint32_t put[6][64];  // positions of registers 2 m and 2 m + 1 of the tiles (1,1), (1,2), (2,2)
+  uint32_t get[6][64];  // entry n = 64 m + lane of the 36 blocks: n % 9, block << 4, position << 10, transposed << 20
+};
+constexpr EasTables easTables() {
+  EasTables t{};
+  for (int lane = 0; lane < 64; ++lane)
+    for (int m = 0; m < 6; ++m) {
+      uint32_t w = 0;
+      for (int h = 0; h < 2; ++h) {
+        const int v = 2 * m + h, I = v < 8 ? 1 : 2, J = v < 4 ? 1 : 2;
+        const int i = 16 * I + 4 * (v & 3) + lane / 16 - NE, j = 16 * J + lane % 16 - NE;
+        uint32_t o = 352 + lane;  // not stored from there
+        if (i >= 0 && i < 24 && j == 24) o = 324 + i;
+        if (i >= 0 && i <= j && j < 24) o = 9 * upperBlock(i / 3, j / 3) + 3 * (i % 3) + j % 3;
+        w |= o << (16 * h);
+      }
+      t.put[m][lane] = w;
+      const int n = 64 * m + lane;
+      if (n >= 324) continue;
+      const int blk = n / 9, r = n % 9, rt = 3 * (r % 3) + r / 3;
+      int src = r, srcT = rt;  // diagonal blocks: the lower triangle from the upper one
+      for (int a = 0; a < 8; ++a)
+        if (blk == upperBlock(a, a)) src = srcT = r < rt ? r : rt;
+      t.get[m][lane] = r | blk << 4 | (9 * blk + src) << 10 | (9 * blk + srcT) << 20;
+    }
+  return t;
+}
+__constant__ const EasTables kEasTables = easTables();
+
+// inverse of a 3x3 matrix of determinant 1 / id
+__device__ inline void inv3(const double J[3][3], double id, double Ji[3][3]) {
+  Ji[0][0] = (J[1][1] * J[2][2] - J[1][2] * J[2][1]) * id;
+  Ji[0][1] = (J[0][2] * J[2][1] - J[0][1] * J[2][2]) * id;
+  Ji[0][2] = (J[0][1] * J[1][2] - J[0][2] * J[1][1]) * id;
+  Ji[1][0] = (J[1][2] * J[2][0] - J[1][0] * J[2][2]) * id;
+  Ji[1][1] = (J[0][0] * J[2][2] - J[0][2] * J[2][0]) * id;
+  Ji[1][2] = (J[0][2] * J[1][0] - J[0][0] * J[1][2]) * id;
+  Ji[2][0] = (J[1][0] * J[2][1] - J[1][1] * J[2][0]) * id;
+  Ji[2][1] = (J[0][1] * J[2][0] - J[0][0] * J[2][1]) * id;
+  Ji[2][2] = (J[0][0] * J[1][1] - J[0][1] * J[1][0]) * id;
+}
+
+// S and C (Voigt) at the enhanced strain
 template <int KIND>
-__device__ inline bool material(double lam, double mu, const double Ev[6], double S[6], double Cp[21], double Ci6[6],
-                                double& c2) {
+__device__ inline bool material(double lam, double mu, const double Ev[6], double S[6], double Cp[21]) {
   if constexpr (KIND == IK_SVK) {
     const double tr = Ev[0] + Ev[1] + Ev[2];
     for (int i = 0; i < 3; ++i) S[i] = lam * tr + 2.0 * mu * Ev[i];
@@ -184,8 +191,6 @@ __device__ inline bool material(double lam, double mu, const double Ev[6], doubl
     for (int p = 0; p < 3; ++p)
       for (int q = p; q < 3; ++q) Cp[sym6(p, q)] = lam + (p == q ? 2.0 * mu : 0.0);
     for (int p = 3; p < 6; ++p) Cp[sym6(p, p)] = mu;
-    for (int v = 0; v < 6; ++v) Ci6[v] = v < 3 ? 1.0 : 0.0;
-    c2 = mu;
     return true;
   } else {
     double C[3][3];
@@ -198,20 +203,11 @@ __device__ inline bool material(double lam, double mu, const double Ev[6], doubl
     if (!(detC > 0.0)) return false;
     const double id = 1.0 / detC;
     double Ci[3][3];
-    Ci[0][0] = (C[1][1] * C[2][2] - C[1][2] * C[2][1]) * id;
-    Ci[0][1] = (C[0][2] * C[2][1] - C[0][1] * C[2][2]) * id;
-    Ci[0][2] = (C[0][1] * C[1][2] - C[0][2] * C[1][1]) * id;
-    Ci[1][0] = (C[1][2] * C[2][0] - C[1][0] * C[2][2]) * id;
-    Ci[1][1] = (C[0][0] * C[2][2] - C[0][2] * C[2][0]) * id;
-    Ci[1][2] = (C[0][2] * C[1][0] - C[0][0] * C[1][2]) * id;
-    Ci[2][0] = (C[1][0] * C[2][1] - C[1][1] * C[2][0]) * id;
-    Ci[2][1] = (C[0][1] * C[2][0] - C[0][0] * C[2][1]) * id;
-    Ci[2][2] = (C[0][0] * C[1][1] - C[0][1] * C[1][0]) * id;
+    inv3(C, id, Ci);
     const double lnJ = log(sqrt(detC));
-    c2               = mu - lam * lnJ;
+    const double c2  = mu - lam * lnJ;
     for (int v = 0; v < 6; ++v) {
       const double ci = Ci[vI(v)][vJ(v)];
-      Ci6[v]          = ci;
       S[v]            = mu * ((v < 3 ? 1.0 : 0.0) - ci) + lam * lnJ * ci;
     }
     for (int p = 0; p < 6; ++p)
@@ -223,449 +219,448 @@ __device__ inline bool material(double lam, double mu, const double Ev[6], doubl
   }
 }
 
-// y = A x for a symmetric 3x3 A in Voigt order
-__device__ inline void symMul(const double* A6, const double x[3], double y[3]) {
+// Phase 1 (lane (element, Gauss point)): kinematics, enhanced strain E + M alpha, material.
+// Phase 2 (element by element): lane (c, q) = (lane % 16, lane / 16) forms columns c, 16 + c and 32 + c of N and CN at
+// the points 2 q and 2 q + 1, whose 6 rows are the contraction steps: the values are the operands of
+// v_mfma_f64_16x16x4 (A[i][k] and B[k][j] at lane 16 k + i or j) as they stand. Tile (I, J) of the sum holds entry
+// (16 I + 4 v + q, 16 J + c) in its register v; columns 0-20 are the modes, 21-44 the displacements, 45 the residual.
+// Phase 3: elimination of the mode rows, four at a time: register v of a tile row is the panel P (rows 4 v + q), again
+// in operand layout; with the inverse of its 4 x 4 diagonal block (by 2 x 2 blocks; the reference inverts D by LU,
+// enhancedassumedstrains.hh:243,294,344) What = P_pp^-1 P, and tiles -= P^T What. What remains at the displacement
+// columns is K_uu - L^T D^-1 L and R_u - L^T D^-1 Rt. D is SPD while the material tangent is positive definite; a pivot
+// that is not finite or vanishes against the largest entry of D makes the element singular (error flag word 1).
+// Phase 4: the geometric part sum_g g_a . S dV g_b, diagonal blocks mirrored from their upper triangle, faces' loads.
+template <int KIND, bool WANT_K, int E>
+__global__ __launch_bounds__(64, 2) void easElement(const double* __restrict__ X, const double* __restrict__ U,
+                                                          const int32_t* __restrict__ conn,
+                                                          const double* __restrict__ alpha, int64_t e0, int64_t count,
+                                                          double lam, double mu, const int32_t* __restrict__ dest,
+                                                          const int32_t* __restrict__ rdest,
+                                                          double* __restrict__ Kebe, double* __restrict__ Rebe,
+                                                          const uint8_t* __restrict__ fbits, double3 trac,
+                                                          double* __restrict__ cache,
+                                                          unsigned long long* __restrict__ err) {
+  __shared__ __attribute__((aligned(16))) EasLds<E> s;
+  const int lane   = threadIdx.x;
+  const int64_t i0 = (int64_t)blockIdx.x * E;  // first element of the workgroup, of `count` from e0
+  const int nel    = count - i0 < E ? (int)(count - i0) : E;
+  const int el0 = lane >> 3, gp = lane & 7;  // phase 1: the lane's element (el0 < nel) and Gauss point
+  if (el0 < nel) {
+    const int64_t nd = conn[(e0 + i0 + el0) * 8 + gp];
 #pragma unroll
-  for (int i = 0; i < 3; ++i) y[i] = A6[v6(i, 0)] * x[0] + A6[v6(i, 1)] * x[1] + A6[v6(i, 2)] * x[2];
-}
-
-// Phases (all 64 lanes): (1) Gauss-point kinematics, enhanced strain and material, lane (gp, node): each lane
-// keeps its node's g_a and F Ci g_a, node 0 the point's data; (2) the point loop: K_uu in the Ci form,
-//   K_ab[k][l] += lambda dV p_ak p_bl + c2 dV (p_al p_bk + (g_a.Ci g_b) Phi_kl) + (g_a.S dV g_b) delta_kl,
-//   p_a = F Ci g_a, Phi = F Ci F^T (the material part of B^T C B written with C = lambda Ci(x)Ci + 2 c2 sym(Ci box
-//   Ci); SVK: Ci = I, c2 = mu), lane (a, b) per 3x3 block; then D, L = sum f_i Z[kRow_i], Rt and R_u
-//   = sum (F S dV g_b)_l with Z[w][3b+l] = (F Q^w g_b)_l, Q^w the symmetric tensor of column w of C dV T0^-1;
-// (3) W = L_D^-1 [L | Rt] and What = diag(d)^-1 W by forward elimination, one column per lane; (4) K = K_uu -
-// W^T What, lane (a, b) per block (the diagonal blocks mirrored from their upper triangle), R = R_u - W^T what.
-template <int KIND, bool WANT_K>
-__global__ __launch_bounds__(64) void easElement(const double* __restrict__ X, const double* __restrict__ U,
-                                                 const int32_t* __restrict__ conn,
-                                                 const double* __restrict__ alpha, int64_t e0, double lam,
-                                                 double mu, const int32_t* __restrict__ dest,
-                                                 const int32_t* __restrict__ rdest, double* __restrict__ Kebe,
-                                                 double* __restrict__ Rebe, const uint8_t* __restrict__ fbits,
-                                                 double3 trac, double* __restrict__ cache,
-                                                 unsigned long long* __restrict__ err) {
-  __shared__ EasLds<WANT_K> s;
-  auto& sk        = s.uk.k;
-  auto& sq        = s.uk.q;
-  auto& sg        = s.u.g;
-  auto& sc        = s.u.c;
-  const int t     = threadIdx.x;
-  const int64_t e = e0 + blockIdx.x;
-  if (t < 24) {
-    const int64_t nd = conn[e * 8 + t / 3];
-    s.X[t / 3][t % 3] = X[nd * 3 + t % 3];
-    s.U[t / 3][t % 3] = U[nd * 3 + t % 3];
-  } else if (t >= 32 && t < 32 + NE) {
-    s.alpha[t - 32] = alpha[e * NE + (t - 32)];
-  } else if (t == 63) {
-    s.bad = 0;
+    for (int k = 0; k < 3; ++k) {
+      s.u[el0].in.X[3 * gp + k] = X[nd * 3 + k];
+      s.u[el0].in.U[3 * gp + k] = U[nd * 3 + k];
+    }
   }
-  __syncthreads();
-  // (T(xi0) detJ0)^-1 (tensorutils.hh:440-465; helperfunctions.hh:19-25). The Voigt strain transformation is
-  // a representation of the Jacobian, T(J)^-1 = T(J^-1), so each of 36 lanes writes one entry directly.
-  if (t < 36) {
-    const double xc[3] = {0.5, 0.5, 0.5};
-    double J[3][3];
-    jacobianAt(s.X, xc, J);
-    const double dJ = det3(J);
-    const double id = 1.0 / dJ;
-    double Ji[3][3];
-    Ji[0][0]       = (J[1][1] * J[2][2] - J[1][2] * J[2][1]) * id;
-    Ji[0][1]       = (J[0][2] * J[2][1] - J[0][1] * J[2][2]) * id;
-    Ji[0][2]       = (J[0][1] * J[1][2] - J[0][2] * J[1][1]) * id;
-    Ji[1][0]       = (J[1][2] * J[2][0] - J[1][0] * J[2][2]) * id;
-    Ji[1][1]       = (J[0][0] * J[2][2] - J[0][2] * J[2][0]) * id;
-    Ji[1][2]       = (J[0][2] * J[1][0] - J[0][0] * J[1][2]) * id;
-    Ji[2][0]       = (J[1][0] * J[2][1] - J[1][1] * J[2][0]) * id;
-    Ji[2][1]       = (J[0][1] * J[2][0] - J[0][0] * J[2][1]) * id;
-    Ji[2][2]       = (J[0][0] * J[1][1] - J[0][1] * J[1][0]) * id;
-    const int r = t / 6, c = t % 6;
-    const int a = vI(r), b = vJ(r), k = vI(c), l = vJ(c);
-    const double v = Ji[k][a] * Ji[l][b] + Ji[l][a] * Ji[k][b];
-    s.T0[r][c]     = (a == b ? 0.5 * v : v) / fabs(dJ);
-  }
-  __syncthreads();
-  // (1) Gauss point gp = t / 8 (kinematics repeated by its 8 lanes), node na = t % 8
-  {
-    const int gp = t >> 3, na = t & 7;
+  for (int i = lane; i < nel * NE; i += 64) s.u[i / NE].in.alpha[i % NE] = alpha[(e0 + i0) * NE + i];
+  if (lane < E) s.bad[lane] = 0;
+  waveSync();
+  if (el0 < nel) {
     const double d = 0.28867513459481288225;
-    double xi[3];
-    for (int k = 0; k < 3; ++k) xi[k] = ((gp >> k) & 1) ? 0.5 + d : 0.5 - d;
-    double J[3][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}};
+    double xi[3], xm[3];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      xi[k] = ((gp >> k) & 1) ? 0.5 + d : 0.5 - d;
+      xm[k] = 1.0 - xi[k];
+    }
+    // dN_a/dxi_k = +- f[k][m], m the corner's position in the other two directions
+    double f[3][4];
+#pragma unroll
+    for (int m = 0; m < 4; ++m) {
+      f[0][m] = ((m & 1) ? xi[1] : xm[1]) * ((m & 2) ? xi[2] : xm[2]);
+      f[1][m] = ((m & 1) ? xi[0] : xm[0]) * ((m & 2) ? xi[2] : xm[2]);
+      f[2][m] = ((m & 1) ? xi[0] : xm[0]) * ((m & 2) ? xi[1] : xm[1]);
+    }
+    // A[i][k] = sum_a Y_ai dN_a/dxi_k, and at the centre
+    auto gradient = [&](const double* Y, double A[3][3], double (*A0)[3]) {
+#pragma unroll
+      for (int i = 0; i < 3; ++i)
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+          double a = 0.0, a0 = 0.0;
+#pragma unroll
+          for (int m = 0; m < 4; ++m) {
+            const int lo = k == 0 ? 2 * m : (k == 1 ? (m & 1) + 4 * (m >> 1) : m);
+            const double y = Y[3 * (lo + (1 << k)) + i] - Y[3 * lo + i];
+            a += y * f[k][m];
+            a0 += y;
+          }
+          A[i][k] = a;
+          if (A0) A0[i][k] = 0.25 * a0;
+        }
+    };
+    double J[3][3], J0[3][3], Ji[3][3], Ji0[3][3], H[3][3], F[3][3];
+    gradient(s.u[el0].in.X, J, J0);
+    const double detJ = det3(J), dJ0 = det3(J0);
+    inv3(J, 1.0 / detJ, Ji);
+    inv3(J0, 1.0 / dJ0, Ji0);
+    gradient(s.u[el0].in.U, H, nullptr);
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+#pragma unroll
+      for (int j = 0; j < 3; ++j)
+        F[i][j] = (i == j ? 1.0 : 0.0) + H[i][0] * Ji[0][j] + H[i][1] * Ji[1][j] + H[i][2] * Ji[2][j];
+    // Mtilde alpha: one term per mode, in its row
+    double wv[6] = {0, 0, 0, 0, 0, 0};
+    const double sx[3] = {2.0 * xi[0] - 1.0, 2.0 * xi[1] - 1.0, 2.0 * xi[2] - 1.0};
+#pragma unroll
+    for (int c = 0; c < NE; ++c) {
+      double fc = s.u[el0].in.alpha[c];
+#pragma unroll
+      for (int k = 0; k < 3; ++k)
+        if ((monomialOf(c) >> k) & 1) fc *= sx[k];
+      wv[kRowOf(c)] += fc;
+    }
+    waveSync();  // the points' data take the place of the element's inputs
+    EasPoint& P = s.u[el0].pt[gp];
 #pragma unroll
     for (int a = 0; a < 8; ++a) {
-      double dN[3];
-      dShape(a, xi, dN);
-      for (int i = 0; i < 3; ++i)
-        for (int j = 0; j < 3; ++j) J[i][j] += s.X[a][i] * dN[j];
-    }
-    const double detJ = det3(J);
-    const double id   = 1.0 / detJ;
-    double Ji[3][3];
-    Ji[0][0] = (J[1][1] * J[2][2] - J[1][2] * J[2][1]) * id;
-    Ji[0][1] = (J[0][2] * J[2][1] - J[0][1] * J[2][2]) * id;
-    Ji[0][2] = (J[0][1] * J[1][2] - J[0][2] * J[1][1]) * id;
-    Ji[1][0] = (J[1][2] * J[2][0] - J[1][0] * J[2][2]) * id;
-    Ji[1][1] = (J[0][0] * J[2][2] - J[0][2] * J[2][0]) * id;
-    Ji[1][2] = (J[0][2] * J[1][0] - J[0][0] * J[1][2]) * id;
-    Ji[2][0] = (J[1][0] * J[2][1] - J[1][1] * J[2][0]) * id;
-    Ji[2][1] = (J[0][1] * J[2][0] - J[0][0] * J[2][1]) * id;
-    Ji[2][2] = (J[0][0] * J[1][1] - J[0][1] * J[1][0]) * id;
-    double F[3][3] = {{1, 0, 0}, {0, 1, 0}, {0, 0, 1}};
+      const double d0 = (a & 1) ? f[0][a >> 1] : -f[0][a >> 1];
+      const double d1 = (a & 2) ? f[1][(a & 1) + 2 * (a >> 2)] : -f[1][(a & 1) + 2 * (a >> 2)];
+      const double d2 = (a & 4) ? f[2][a & 3] : -f[2][a & 3];
 #pragma unroll
-    for (int a = 0; a < 8; ++a) {
-      double dN[3], g[3];
-      dShape(a, xi, dN);
-      for (int i = 0; i < 3; ++i) g[i] = Ji[0][i] * dN[0] + Ji[1][i] * dN[1] + Ji[2][i] * dN[2];
-      for (int i = 0; i < 3; ++i)
-        for (int j = 0; j < 3; ++j) F[i][j] += s.U[a][i] * g[j];
-    }
-    double go[3];
-    {
-      double dN[3];
-      dShape(na, xi, dN);
-      for (int i = 0; i < 3; ++i) go[i] = Ji[0][i] * dN[0] + Ji[1][i] * dN[1] + Ji[2][i] * dN[2];
+      for (int i = 0; i < 3; ++i) P.G[a][i] = Ji[0][i] * d0 + Ji[1][i] * d1 + Ji[2][i] * d2;
     }
     double Ev[6];
+#pragma unroll
     for (int v = 0; v < 6; ++v) {
       const int I = vI(v), Jj = vJ(v);
       const double c = F[0][I] * F[0][Jj] + F[1][I] * F[1][Jj] + F[2][I] * F[2][Jj];
       Ev[v]          = v < 3 ? 0.5 * (c - 1.0) : c;  // engineering shear 2E_IJ = C_IJ
     }
-    // E_enh = E + M alpha, M = T0^{-1} Mtilde / detJ: Mtilde alpha has one term per mode in row kRow[c]
-    const double x = 2 * xi[0] - 1.0, y = 2 * xi[1] - 1.0, z = 2 * xi[2] - 1.0;
-    const double sc1 = 1.0 / fabs(detJ);
-    double wv[6] = {0, 0, 0, 0, 0, 0};
+    // E += M alpha = T0^-1 (Mtilde alpha) / detJ, T0^-1 w = Ji0^T w Ji0 / detJ0 on the strain tensor w (T(J)^-1 =
+    // T(J^-1): the Voigt strain transformation represents the Jacobian, tensorutils.hh:440-465)
+    const double w = 1.0 / (fabs(detJ) * fabs(dJ0));
+    double T[3][3];
 #pragma unroll
-    for (int c = 0; c < NE; ++c) wv[kRowOf(c)] += ansatz(c, x, y, z) * s.alpha[c];
+    for (int k = 0; k < 3; ++k)
 #pragma unroll
-    for (int r = 0; r < 6; ++r) {
-      double acc = 0.0;
-#pragma unroll
-      for (int q = 0; q < 6; ++q) acc += s.T0[r][q] * wv[q];
-      Ev[r] += acc * sc1;
-    }
-    double Sv[6], Cp[21], Ci6[6], c2;
-    if (!material<KIND>(lam, mu, Ev, Sv, Cp, Ci6, c2)) {
-      atomicMin(err, (unsigned long long)e);
-      s.bad = 1;
-    }
-    const double dV = fabs(detJ) * 0.125;
-    double sgo[3];
-    symMul(Sv, go, sgo);
-    for (int i = 0; i < 3; ++i) {
-      sk.G[gp][na][i]  = go[i];
-      sg.ru[gp][na][i] = (F[i][0] * sgo[0] + F[i][1] * sgo[1] + F[i][2] * sgo[2]) * dV;
-    }
-    if constexpr (WANT_K) {
-      double q[3];
-      symMul(Ci6, go, q);
-      for (int i = 0; i < 3; ++i) sk.P[gp][na][i] = F[i][0] * q[0] + F[i][1] * q[1] + F[i][2] * q[2];
-    }
-    if (na == 0) {
-      for (int i = 0; i < 9; ++i) sg.F[gp][i] = F[i / 3][i % 3];
-      for (int v = 0; v < 6; ++v) sk.S[gp][v] = Sv[v] * dV;
-      for (int i = 0; i < 21; ++i) sg.C[gp][i] = Cp[i] * dV;
-      if constexpr (WANT_K) {
-        for (int v = 0; v < 6; ++v) sk.Ci[gp][v] = Ci6[v];
-        // Phi = F Ci F^T
-        double FC[3][3];
-        for (int i = 0; i < 3; ++i) symMul(Ci6, F[i], FC[i]);  // row i of F Ci (Ci symmetric)
-        for (int v = 0; v < 6; ++v) {
-          const int k = vI(v), l = vJ(v);
-          sk.Phi[gp][v] = FC[k][0] * F[l][0] + FC[k][1] * F[l][1] + FC[k][2] * F[l][2];
-        }
-        sk.w[gp][0] = lam * dV;
-        sk.w[gp][1] = c2 * dV;
-      }
-#pragma unroll
-      for (int c = 0; c < NE; ++c) sg.f[gp][c] = ansatz(c, x, y, z) * sc1;
-    }
-  }
-  __syncthreads();
-  if (s.bad) return;  // uniform: the error flag is already set
-
-  // (2a) point loop for D, L and Rt: D upper entries t + 64 j (< 231), L columns and Rt (lanes 0-20) are owned by
-  // fixed lanes; R_u (lanes 40-63) is summed from the per-point contributions afterwards
-  const int ka = t >> 3, kbn = t & 7;
-  double dacc[4] = {0, 0, 0, 0};
-  double racc    = 0.0;
-  int dI[4], dC[4], dKi[4], dKc[4];
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    triDecode(t + 64 * j < 231 ? t + 64 * j : 230, NE, dI[j], dC[j]);
-    dKi[j] = kRow[dI[j]];
-    dKc[j] = kRow[dC[j]];
-  }
-  // L: lane t < 48 owns column lc = t % 24 of rows lh + 2m (lh = t / 24)
-  const int lc = t % 24, lh = t / 24;
-  double lacc[11] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-  const int rK = kRow[t < NE ? t : 0];
-  // the one column of T0 each lane's role reads at every point: w (C T0^-1), p (T0^-T C T0^-1), w (T0^-T S)
-  int chP = 0, chQ = 0;
-  if (t >= 43) triDecode(t >= 48 ? t - 48 : t - 27, 6, chP, chQ);
-  double t0c[6];
-  {
-    const int tc = t < 36 ? t % 6 : (t >= 43 ? chP : (t >= 37 ? t - 37 : 0));
-#pragma unroll
-    for (int u = 0; u < 6; ++u) t0c[u] = s.T0[u][tc];
-  }
-  for (int g = 0; g < 8; ++g) {
-    if (t < 36) {
-      const int v = t / 6, w = t % 6;
-      double acc = 0.0;
-#pragma unroll
-      for (int u = 0; u < 6; ++u) acc += sg.C[g][sym6(v, u)] * t0c[u];
-      sg.CT[v][w] = acc;
-    }
-    __syncthreads();
-    // Z[w][3b+l] = (F Q^w g_b)_l (lane (w, b) < 48), Ch = T0^-T CT (lanes 48-63, then 43-47), TS (lanes 37-42)
-    if (t < 48) {
-      const int w = t >> 3, b = t & 7;
-      double Q[6], gbv[3], h[3];
-      for (int v = 0; v < 6; ++v) Q[v] = sg.CT[v][w];
-      for (int i = 0; i < 3; ++i) gbv[i] = sk.G[g][b][i];
-      symMul(Q, gbv, h);
-#pragma unroll
-      for (int l = 0; l < 3; ++l)
-        sg.Z[w][3 * b + l] = sg.F[g][3 * l] * h[0] + sg.F[g][3 * l + 1] * h[1] + sg.F[g][3 * l + 2] * h[2];
-    }
-    if (t >= 43) {
-      double acc = 0.0;
-#pragma unroll
-      for (int v = 0; v < 6; ++v) acc += t0c[v] * sg.CT[v][chQ];
-      sg.Ch[chP][chQ] = acc;
-      sg.Ch[chQ][chP] = acc;
-    }
-    if (t >= 37 && t < 43) {
-      const int w = t - 37;
-      double acc = 0.0;
-#pragma unroll
-      for (int v = 0; v < 6; ++v) acc += t0c[v] * sk.S[g][v];
-      sg.TS[w] = acc;
-    }
-    __syncthreads();
-    // D[i][c] += f_i f_c Ch[kRow_i][kRow_c]; L[i][col] += f_i Z[kRow_i][col]; Rt[i] += f_i TS[kRow_i];
-    // R_u[3b+l] += (F S dV g_b)_l
-    const double* fg = sg.f[g];
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-      if (t + 64 * j < 231) dacc[j] += fg[dI[j]] * fg[dC[j]] * sg.Ch[dKi[j]][dKc[j]];
-    if (t < 48) {
-#pragma unroll
-      for (int m = 0; m < 11; ++m) {
-        if (m < 10 || lh == 0) {
-          const int kr = lh ? kRowOf(2 * m + 1) : kRowOf(2 * m);
-          lacc[m] += fg[lh + 2 * m] * sg.Z[kr][lc];
-        }
-      }
-    }
-    if (t < NE) racc += fg[t] * sg.TS[rK];
-  }
-  if (t >= 40) {
-    const int col = t - 40;
-#pragma unroll
-    for (int g = 0; g < 8; ++g) racc += sg.ru[g][col / 3][col % 3];
-  }
-  __syncthreads();  // the point data is dead from here: the condensation operands take its place
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    if (t + 64 * j < 231) {
-      sc.A[dI[j]][dC[j]] = dacc[j];
-      sc.A[dC[j]][dI[j]] = dacc[j];
-    }
-  }
-  if (t < 48) {
-#pragma unroll
-    for (int m = 0; m < 11; ++m)
-      if (m < 10 || lh == 0) sc.Lm[lh + 2 * m][lc] = lacc[m];
-  }
-  if (t < NE) sc.rt[t] = racc;
-  if (t >= 40) sc.Ru[t - 40] = racc;
-  // (2b) K_uu, lane (ka, kb) per 3x3 block (the K_uu inputs are untouched by the spill above)
-  if constexpr (WANT_K) {
-    double kb[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
-#pragma unroll 1  // unrolled, the hoisted loads take registers (2 or 4: 166 / 154 VGPRs, no faster)
-    for (int g = 0; g < 8; ++g) {
-      double pa[3], pb[3], ga[3], gb[3], Ci6[6], S6[6], Ph[6];
-      for (int i = 0; i < 3; ++i) {
-        pa[i] = sk.P[g][ka][i];
-        pb[i] = sk.P[g][kbn][i];
-        ga[i] = sk.G[g][ka][i];
-        gb[i] = sk.G[g][kbn][i];
-      }
-      for (int v = 0; v < 6; ++v) {
-        Ci6[v] = sk.Ci[g][v];
-        S6[v]  = sk.S[g][v];
-        Ph[v]  = sk.Phi[g][v];
-      }
-      const double wl = sk.w[g][0], wc = sk.w[g][1];
-      double qb[3], sb[3];
-      symMul(Ci6, gb, qb);
-      symMul(S6, gb, sb);
-      const double gCg = ga[0] * qb[0] + ga[1] * qb[1] + ga[2] * qb[2];
-      const double gSg = ga[0] * sb[0] + ga[1] * sb[1] + ga[2] * sb[2];
-#pragma unroll
-      for (int k = 0; k < 3; ++k)
+      for (int b = 0; b < 3; ++b) {
+        T[k][b] = 0.0;
 #pragma unroll
         for (int l = 0; l < 3; ++l)
-          kb[3 * k + l] += wl * pa[k] * pb[l] + wc * (pa[l] * pb[k] + gCg * Ph[v6(k, l)]) + (k == l ? gSg : 0.0);
-    }
-    __syncthreads();  // the K_uu inputs are dead: park the blocks in their place
-    if (ka <= kbn)
+          T[k][b] += (k == l ? wv[k] : 0.5 * wv[k + l == 3 ? 3 : (k + l == 2 ? 4 : 5)]) * Ji0[l][b];
+      }
 #pragma unroll
-      for (int i = 0; i < 9; ++i) sq.Kuu[upperBlock(ka, kbn)][i] = kb[i];
+    for (int v = 0; v < 6; ++v) {
+      const int a = vI(v), b = vJ(v);
+      const double m = Ji0[0][a] * T[0][b] + Ji0[1][a] * T[1][b] + Ji0[2][a] * T[2][b];
+      Ev[v] += (v < 3 ? m : 2.0 * m) * w;
+    }
+    double Sv[6], Cp[21];
+    if (!material<KIND>(lam, mu, Ev, Sv, Cp)) {
+      atomicMin(err, (unsigned long long)(e0 + i0 + el0));
+      s.bad[el0] = 1;
+    }
+    const double dV = fabs(detJ) * 0.125;
+#pragma unroll
+    for (int i = 0; i < 21; ++i) P.C[i] = Cp[i] * dV;
+#pragma unroll
+    for (int i = 0; i < 9; ++i) P.F[i] = F[i / 3][i % 3];
+#pragma unroll
+    for (int v = 0; v < 6; ++v) P.S[v] = Sv[v] * dV;
+    P.w = w;
+    if (gp == 0)
+#pragma unroll
+      for (int i = 0; i < 9; ++i) s.Ji0[el0][i] = Ji0[i / 3][i % 3];
   }
   __syncthreads();
 
-  // (3) The condensation L^T D^-1 [L | Rt] (enhancedassumedstrains.hh inverts D by LU, :243,294,344) through
-  // D = L_D diag(d) L_D^T without pivoting (D is SPD while the material tangent is positive definite):
-  // L^T D^-1 L = W^T diag(d)^-1 W with W = L_D^-1 L, so forward elimination of the augmented 21 x 46 matrix
-  // [D | L | Rt] suffices. Lane c < 46 keeps column c in registers; step j reads rows j..20 of the pivot
-  // column from lane j's registers (readlane), and every lane divides its row j, final from then on, by d_j and
-  // subtracts the multiples from its rows below j. The L lanes first save their row j of W over the same row
-  // of L in LDS. Afterwards the L lanes hold What = diag(d)^-1 W, the Rt lane what = diag(d)^-1 L_D^-1 Rt, and
-  // lane c < 21 holds the multipliers (L_D)_cj = U_jc / d_j in rows j < c (U = diag(d) L_D^T, the eliminated
-  // D). Half the lane reads and updates of a Gauss-Jordan elimination; the back substitution D^-1 needs for
-  // the alpha update runs there, on 21 values per element.
-  double col[NE];
+  // the lane's columns: modes c and, for c < 5, 16 + c; displacements c - 5 (c >= 5, tile 1), 11 + c (c < 13, tile 2)
+  const int c = lane & 15, q = lane >> 4;
+  const bool mode1 = c < 5, rhs2 = c == 13;
+  const int col1 = mode1 ? 0 : c - 5, col2 = c < 13 ? c + 11 : 23;
+  const int b1 = col1 / 3, l1 = col1 - 3 * b1, b2 = col2 / 3, l2 = col2 - 3 * b2;
+  // Voigt row and monomial of the lane's modes
+  const int md1 = mode1 ? 16 + c : 16;
+  const int row0 = (int)((packModes(true) >> (3 * c)) & 7), row1 = (int)((packModes(true) >> (3 * md1)) & 7);
+  const int mono0 = (int)((packModes(false) >> (3 * c)) & 7), mono1 = (int)((packModes(false) >> (3 * md1)) & 7);
+  // rows k, l of the centre's inverse Jacobian for them
+  const int k0 = 3 * (row0 < 3 ? row0 : (row0 == 3 ? 1 : 0)), n0 = 3 * (row0 < 3 ? row0 : (row0 == 5 ? 1 : 2));
+  const int k1 = 3 * (row1 < 3 ? row1 : (row1 == 3 ? 1 : 0)), n1 = 3 * (row1 < 3 ? row1 : (row1 == 5 ? 1 : 2));
+  auto modeAt = [](int mono, int gp) {  // f_c at a Gauss point
+    const double f = __popc(mono) == 1 ? kGaussX : kGaussX * kGaussX;
+    return (__popc(mono & ~gp) & 1) ? -f : f;
+  };
+  const int ga = 4 * ((lane >> 3) & 1) + (lane & 3), gb = 4 * ((lane >> 2) & 1) + (lane & 3);  // geometric part: nodes
+  const double unit[4] = {q == 0 ? 1.0 : 0.0, q == 1 ? 1.0 : 0.0, q == 2 ? 1.0 : 0.0, q == 3 ? 1.0 : 0.0};
+
+  for (int el = 0; el < nel; ++el) {
+    if (s.bad[el]) continue;  // uniform: the error flag is already set
+    const int64_t e   = e0 + i0 + el;
+    const EasPoint* points = s.u[el].pt;
+    v4d t00 = {0, 0, 0, 0}, t01 = t00, t02 = t00, t11 = t00, t12 = t00, t22 = t00;
+    double kg = 0.0;
+    // columns of T0^-1 detJ0: the strain of directions (Jk, Jl), as a displacement column is that of (F_l, g_b)
+    const double* Ji = s.Ji0[el];
+#pragma unroll 1  // both points at once take more registers than two wavefronts per SIMD leave
+    for (int p = 0; p < 2; ++p) {
+      const EasPoint& P = points[2 * q + p];
+      double C[21], S[6], N0[6], N1[6], N2[6], cn[6];
 #pragma unroll
-  for (int i = 0; i < NE; ++i)
-    col[i] = t < NE ? sc.A[i][t] : (t < NE + 24 ? sc.Lm[i][t - NE] : (t == NE + 24 ? sc.rt[i] : 0.0));
-  // pivot guard: the reference inverts D with partial pivoting; without pivoting a pivot that is not finite or
-  // vanishes against the largest entry of D makes the element singular here (error flag word 1, lowest element)
-  double dmax = 0.0;
-  if (t < NE)
+      for (int i = 0; i < 21; ++i) C[i] = P.C[i];
 #pragma unroll
-    for (int i = 0; i < NE; ++i) dmax = fmax(dmax, fabs(col[i]));
-  dmax = waveMax(dmax);
-  bool singular = !(dmax < INFINITY);
+      for (int v = 0; v < 6; ++v) S[v] = P.S[v];
+      auto strainColumn = [&](const double* A, const double* G, double f, double N[6]) {
+        const double A0 = f * A[0], A1 = f * A[1], A2 = f * A[2], g0 = G[0], g1 = G[1], g2 = G[2];
+        N[0] = A0 * g0;
+        N[1] = A1 * g1;
+        N[2] = A2 * g2;
+        N[3] = A1 * g2 + A2 * g1;
+        N[4] = A0 * g2 + A2 * g0;
+        N[5] = A0 * g1 + A1 * g0;
+      };
+      auto times = [&](const double N[6], double y[6]) {
 #pragma unroll
-  for (int j = 0; j < NE; ++j) {
-    double piv[NE];  // rows j.. of lane j's column, read into scalar registers (no LDS round trip, no barrier)
+        for (int v = 0; v < 6; ++v) {
+          double a = C[sym6(v, 0)] * N[0];
 #pragma unroll
-    for (int i = j; i < NE; ++i) piv[i] = readLane(col[i], j);
-    singular |= !(fabs(piv[j]) > 1e-13 * dmax && fabs(piv[j]) < INFINITY);
-    if (t >= NE && t < NE + 24) sc.Lm[j][t - NE] = col[j];  // W_jc; lane c alone reads and writes column c
-    const double f = col[j] / piv[j];
+          for (int u = 1; u < 6; ++u) a += C[sym6(v, u)] * N[u];
+          y[v] = a;
+        }
+      };
+      const double w = P.w;
+      // column by column of tiles, and no reordering across them: the registers of one column at a time
+      strainColumn(Ji + k0, Ji + n0, modeAt(mono0, 2 * q + p) * w, N0);
+      times(N0, cn);
 #pragma unroll
-    for (int i = j + 1; i < NE; ++i) col[i] -= piv[i] * f;
-    col[j] = f;
-  }
-  if (singular && t == 0) atomicMin(err + 1, (unsigned long long)e);
-  // cache for the alpha update, per element: What column by column (entry (i, c) at 21 c + i, so that the
-  // update's lane per mode reads 21 adjacent values at a time), what, then (L_D)_ij for i > j row by row
-  // (offset 525 + i (i - 1) / 2 + j)
-  double* cy = cache + e * kEasCache;
-  if (t >= NE && t < NE + 24) {
+      for (int v = 0; v < 6; ++v) t00 = __builtin_amdgcn_mfma_f64_16x16x4f64(N0[v], cn[v], t00, 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+      strainColumn(mode1 ? Ji + k1 : P.F + 3 * l1, mode1 ? Ji + n1 : P.G[b1],
+                   mode1 ? modeAt(mono1, 2 * q + p) * w : 1.0, N1);
+      times(N1, cn);
 #pragma unroll
-    for (int i = 0; i < NE; ++i) {
-      cy[(t - NE) * NE + i] = col[i];
-      sc.A[i][t - NE]       = col[i];
-    }
-  } else if (t == NE + 24) {
-#pragma unroll
-    for (int i = 0; i < NE; ++i) {
-      cy[NE * 24 + i] = col[i];
-      sc.rt[i]        = col[i];
-    }
-  } else if (t > 0 && t < NE) {
-    double* lrow = cy + NE * 25 + t * (t - 1) / 2;
-#pragma unroll
-    for (int j = 0; j < NE - 1; ++j)
-      if (j < t) lrow[j] = col[j];
-  }
-  __syncthreads();
-  // (4) K = K_uu - W^T What = K_uu - L^T D^-1 L, block (ka, kb) per lane; upper blocks stored, the diagonal
-  // ones mirrored from their upper triangle (enhancedassumedstrains.hh:291-296)
-  if constexpr (WANT_K) {
-    const int blk = upperBlock(ka <= kbn ? ka : kbn, ka <= kbn ? kbn : ka);
-    double kb[9];
-#pragma unroll
-    for (int i = 0; i < 9; ++i) kb[i] = sq.Kuu[blk][i];
-#pragma unroll
-    for (int i = 0; i < NE; ++i) {
-      double la[3], yb[3];
-      for (int k = 0; k < 3; ++k) {
-        la[k] = sc.Lm[i][3 * ka + k];
-        yb[k] = sc.A[i][3 * kbn + k];
+      for (int v = 0; v < 6; ++v) {
+        t01 = __builtin_amdgcn_mfma_f64_16x16x4f64(N0[v], cn[v], t01, 0, 0, 0);
+        t11 = __builtin_amdgcn_mfma_f64_16x16x4f64(N1[v], cn[v], t11, 0, 0, 0);
       }
+      __builtin_amdgcn_sched_barrier(0);
+      strainColumn(P.F + 3 * l2, P.G[b2], 1.0, N2);  // lanes 13-15: rows and columns that nothing reads
+      times(N2, cn);
 #pragma unroll
-      for (int k = 0; k < 3; ++k)
+      for (int v = 0; v < 6; ++v) cn[v] = rhs2 ? S[v] : cn[v];
 #pragma unroll
-        for (int l = 0; l < 3; ++l) kb[3 * k + l] -= la[k] * yb[l];
-    }
-    if (ka == kbn) {
-      kb[3] = kb[1];
-      kb[6] = kb[2];
-      kb[7] = kb[5];
-    }
-    if (ka <= kbn) {
-      if (dest) {
-        const int32_t code = dest[e * 36 + blk];
-        double* dst        = Kebe + (int64_t)(code >> 1) * 9;
-        for (int k = 0; k < 3; ++k)
-          for (int l = 0; l < 3; ++l) dst[3 * k + l] = (code & 1) ? kb[3 * l + k] : kb[3 * k + l];
-      } else {
-        double* dst = Kebe + (e * 36 + blk) * 9;
-        for (int i = 0; i < 9; ++i) dst[i] = kb[i];
+      for (int v = 0; v < 6; ++v) {
+        t02 = __builtin_amdgcn_mfma_f64_16x16x4f64(N0[v], cn[v], t02, 0, 0, 0);
+        t12 = __builtin_amdgcn_mfma_f64_16x16x4f64(N1[v], cn[v], t12, 0, 0, 0);
+        t22 = __builtin_amdgcn_mfma_f64_16x16x4f64(N2[v], cn[v], t22, 0, 0, 0);
+      }
+      if constexpr (WANT_K) {
+        double g[3], h[3];
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+          g[i] = P.G[ga][i];
+          h[i] = P.G[gb][i];
+        }
+        kg = __builtin_amdgcn_mfma_f64_4x4x4f64(g[0], S[0] * h[0] + S[5] * h[1] + S[4] * h[2], kg, 0, 0, 0);
+        kg = __builtin_amdgcn_mfma_f64_4x4x4f64(g[1], S[5] * h[0] + S[1] * h[1] + S[3] * h[2], kg, 0, 0, 0);
+        kg = __builtin_amdgcn_mfma_f64_4x4x4f64(g[2], S[4] * h[0] + S[3] * h[1] + S[2] * h[2], kg, 0, 0, 0);
       }
     }
-  }
-  if (t >= 40) {
-    const int r = t - 40;
-    double acc  = sc.Ru[r];
+
+    // the lane's table entries and destinations, in flight during the elimination: ahead of the stores, whose
+    // completion a load behind them waits for. (Loaded for each element, from a stand-in where there are none: held
+    // over the loop above they would take its registers, and a branch would wait for them.)
+    uint32_t put[6], get[6];
+    int32_t code[6];
+    int ln = lane;
+    asm volatile("" : "+v"(ln));
+    const int nd = ln < 24 ? ln / 3 : 7, kd = ln % 3;
+    const int32_t* dfrom = dest ? dest + e * 36 : (const int32_t*)kEasTables.get;
+    const int32_t* rfrom = (rdest ? rdest : conn) + e * 8;
+    const uint8_t* ffrom = fbits ? fbits + e : (const uint8_t*)kEasTables.get;
 #pragma unroll
-    for (int i = 0; i < NE; ++i) acc -= sc.Lm[i][r] * sc.rt[i];
-    const unsigned bits = fbits ? fbits[e] : 0u;
-    if (bits) {  // Traction skill, after the EAS element's condensed internal forces
-      const int k = r % 3;
-      acc += faceLoad(X, conn, e, bits, r / 3, k == 0 ? trac.x : (k == 1 ? trac.y : trac.z));
+    for (int m = 0; m < 6; ++m) {
+      put[m]  = kEasTables.put[m][ln];
+      get[m]  = kEasTables.get[m][ln];
+      code[m] = dfrom[m < 5 || ln < 4 ? (ln + 64 * m) / 9 : 35];
     }
-    Rebe[rdest ? (int64_t)rdest[e * 8 + r / 3] * 3 + r % 3 : e * 24 + r] = acc;
+    const int32_t rcode = rfrom[nd];
+    unsigned bits       = *ffrom;
+
+    // the largest entry of D: all of tile (0, 0), columns 16-20 of (0, 1) and (1, 1) (rows 16-19 and 20)
+    double dmax = 0.0;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) dmax = maxAbs(maxAbs(dmax, t00[v]), mode1 ? t01[v] : 0.0);
+    dmax = maxAbs(maxAbs(dmax, mode1 ? t11[0] : 0.0), mode1 && q == 0 ? t11[1] : 0.0);
+    dmax = maxAbs(dmax, dppMove<0x111, 0xF>(dmax));  // over the wavefront, as waveSum
+    dmax = maxAbs(dmax, dppMove<0x112, 0xF>(dmax));
+    dmax = maxAbs(dmax, dppMove<0x114, 0xF>(dmax));
+    dmax = maxAbs(dmax, dppMove<0x118, 0xF>(dmax));
+    dmax = maxAbs(dmax, dppMove<0x142, 0xA>(dmax));
+    dmax = maxAbs(dmax, dppMove<0x143, 0xC>(dmax));
+    dmax = lane63(dmax);
+    // Pivots against the threshold, per 2 x 2 block its first entry and its determinant over that. One that is not
+    // finite makes all later ones NaN (its reciprocal is), so the last one shows it.
+    const double limit = 1e-13 * dmax;
+    double least = INFINITY, gap = INFINITY;
+    auto block2 = [&](double a, double b, double c) {  // 1 / determinant
+      const double det = a * c - b * b;
+      least            = minAbs(least, a);
+      gap              = minOf(gap, fma(-limit, fabs(a), fabs(det)));
+      return reciprocal(det);
+    };
+    double* cy = cache + e * kEasCache;
+#pragma unroll
+    for (int p = 0; p < 5; ++p) {
+      const double P0 = p < 4 ? t00[p & 3] : 0.0, P1 = p < 4 ? t01[p & 3] : t11[0], P2 = p < 4 ? t02[p & 3] : t12[0];
+      const double Pd = p < 4 ? P0 : P1;
+      const int lc    = p < 4 ? 4 * p : 0;
+      auto a = [&](int k, int l) { return readLane(Pd, 16 * k + lc + l); };
+      // D_pp = [A B; B^T C] by 2 x 2 blocks; x = column q of its inverse
+      const double a00 = a(0, 0), a01 = a(0, 1), a11 = a(1, 1);
+      const double b00 = a(0, 2), b01 = a(0, 3), b10 = a(1, 2), b11 = a(1, 3);
+      const double ra = block2(a00, a01, a11);
+      const double i00 = a11 * ra, i01 = -a01 * ra, i11 = a00 * ra;
+      const double m00 = i00 * b00 + i01 * b10, m01 = i00 * b01 + i01 * b11;
+      const double m10 = i01 * b00 + i11 * b10, m11 = i01 * b01 + i11 * b11;
+      const double s00 = a(2, 2) - (b00 * m00 + b10 * m10), s01 = a(2, 3) - (b00 * m01 + b10 * m11);
+      const double s11 = a(3, 3) - (b01 * m01 + b11 * m11);
+      const double rs  = block2(s00, s01, s11);
+      const double v0 = unit[2] - (m00 * unit[0] + m10 * unit[1]), v1 = unit[3] - (m01 * unit[0] + m11 * unit[1]);
+      const double x2 = (s11 * v0 - s01 * v1) * rs, x3 = (s00 * v1 - s01 * v0) * rs;
+      const double x0 = i00 * unit[0] + i01 * unit[1] - (m00 * x2 + m01 * x3);
+      const double x1 = i01 * unit[0] + i11 * unit[1] - (m10 * x2 + m11 * x3);
+      asm("" : : "v"(x0), "v"(x1), "v"(x2), "v"(x3));  // all four before the selection: no branches around them
+      const double xr = (lane & 2) ? ((lane & 1) ? x3 : x2) : ((lane & 1) ? x1 : x0);
+      const double W1 = __builtin_amdgcn_mfma_f64_4x4x4f64(xr, P1, 0.0, 0, 0, 0);
+      const double W2 = __builtin_amdgcn_mfma_f64_4x4x4f64(xr, P2, 0.0, 0, 0, 0);
+      if (p < 3) {
+        const double W0 = __builtin_amdgcn_mfma_f64_4x4x4f64(xr, P0, 0.0, 0, 0, 0);
+        t00             = __builtin_amdgcn_mfma_f64_16x16x4f64(-P0, W0, t00, 0, 0, 0);
+        t01             = __builtin_amdgcn_mfma_f64_16x16x4f64(-P0, W1, t01, 0, 0, 0);
+        t02             = __builtin_amdgcn_mfma_f64_16x16x4f64(-P0, W2, t02, 0, 0, 0);
+        const int w = 12 - 4 * p;
+        if (c >= 4 * (p + 1)) cy[cacheLow(p) + w * q + c - 4 * (p + 1)] = W0;
+      }
+      t11 = __builtin_amdgcn_mfma_f64_16x16x4f64(-P1, W1, t11, 0, 0, 0);
+      t12 = __builtin_amdgcn_mfma_f64_16x16x4f64(-P1, W2, t12, 0, 0, 0);
+      t22 = __builtin_amdgcn_mfma_f64_16x16x4f64(-P2, W2, t22, 0, 0, 0);
+      cy[64 * p + lane] = W1;
+      if (c < 14) cy[320 + 56 * p + 14 * q + c] = W2;
+    }
+    {  // row 20: register 1 of the tiles (1, J), lanes q = 0
+      const double d20 = readLane(t11[1], 4), r20 = reciprocal(d20);
+      if (!(least > limit && gap > 0.0 && fabs(d20) > limit && fabs(d20) < INFINITY && dmax < INFINITY) && lane == 0)
+        atomicMin(err + 1, (unsigned long long)e);
+      const double P1 = q == 0 ? t11[1] : 0.0, P2 = q == 0 ? t12[1] : 0.0;
+      const double W1 = P1 * r20, W2 = P2 * r20;
+      t11 = __builtin_amdgcn_mfma_f64_16x16x4f64(-P1, W1, t11, 0, 0, 0);
+      t12 = __builtin_amdgcn_mfma_f64_16x16x4f64(-P1, W2, t12, 0, 0, 0);
+      t22 = __builtin_amdgcn_mfma_f64_16x16x4f64(-P2, W2, t22, 0, 0, 0);
+      if (q == 0) {
+        if (c >= 5) cy[696 + c - 5] = W1;
+        if (c < 14) cy[696 + 11 + c] = W2;
+      }
+    }
+
+    // K and R to LDS, over the element's points
+    double* out = s.u[el].out;
+    waveSync();
+#pragma unroll
+    for (int v = 0; v < 12; ++v) {
+      const uint32_t o = (put[v / 2] >> (16 * (v & 1))) & 0xFFFF;
+      out[o]           = v < 4 ? t11[v & 3] : (v < 8 ? t12[v & 3] : t22[v & 3]);
+    }
+    waveSync();
+    if constexpr (WANT_K) {
+      const int a = 4 * ((lane >> 3) & 1) + q;  // geometric entry (a, gb) of the lane
+      if (a <= gb) {
+        const int o = upperBlock(a, gb) * 9;
+        const double d0 = out[o], d1 = out[o + 4], d2 = out[o + 8];
+        out[o]     = d0 + kg;
+        out[o + 4] = d1 + kg;
+        out[o + 8] = d2 + kg;
+      }
+      waveSync();
+#pragma unroll
+      for (int m = 0; m < 6; ++m)
+        if (lane + 64 * m < 324) {
+          const int64_t pos = dest ? (int64_t)(code[m] >> 1) : e * 36 + ((get[m] >> 4) & 63);
+          const bool turned = dest && (code[m] & 1);
+          Kebe[pos * 9 + (get[m] & 15)] = out[turned ? get[m] >> 20 : (get[m] >> 10) & 1023];
+        }
+    }
+    if (lane < 24) {
+      double acc = out[324 + lane];
+      if (fbits && bits)  // Traction skill, after the EAS element's condensed internal forces
+        acc += faceLoad(X, conn, e, bits, nd, kd == 0 ? trac.x : (kd == 1 ? trac.y : trac.z));
+      Rebe[rdest ? (int64_t)rcode * 3 + kd : e * 24 + lane] = acc;
+    }
   }
 }
 
-// alpha_e -= D_e^-1 (Rt_e + L_e du_e) = L_D^-T (what_e + What_e du_e): 21 lanes per element, 3 elements per
-// wavefront (lane 63 idle). Lane i forms z_i = what_i + (What du)_i; the back substitution with the unit upper
-// triangle L_D^T then runs from the last mode up, x_k = z_k reaching lanes i < k of its element by a shuffle.
-constexpr int kUpdElemsPerWave = 64 / NE;
-__global__ __launch_bounds__(256) void easUpdateKernel(const double* __restrict__ cache,
-                                                       const int32_t* __restrict__ conn,
-                                                       const double* __restrict__ du, int64_t ne,
-                                                       double* __restrict__ alpha) {
-  const int lane = threadIdx.x & 63, sub = lane / NE, i = lane - NE * sub;
-  const int64_t e   = ((int64_t)blockIdx.x * 4 + (threadIdx.x >> 6)) * kUpdElemsPerWave + sub;
+// alpha_e -= D_e^-1 (Rt_e + L_e du_e) = Lb^-T (what_e + What_e du_e): 21 lanes per element, 3 elements per wavefront
+// (lane 63 idle). The cache is read in one run per wavefront, into LDS. Lane i forms z_i = what_i + (What du)_i; the
+// back substitution with Lb^T then runs from the last mode up, x_m = z_m reaching the lanes of earlier panels by a
+// shuffle.
+constexpr int kUpdElemsPerWave = 64 / NE, kUpdWaves = 4;
+__global__ __launch_bounds__(64 * kUpdWaves) void easUpdateKernel(const double* __restrict__ cache,
+                                                                  const int32_t* __restrict__ conn,
+                                                                  const double* __restrict__ du, int64_t ne,
+                                                                  double* __restrict__ alpha) {
+  __shared__ v2d sw[kUpdWaves][kUpdElemsPerWave * kEasCache / 2];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, sub = lane / NE, i = lane - NE * sub;
+  const int64_t ew  = ((int64_t)blockIdx.x * kUpdWaves + wave) * kUpdElemsPerWave, e = ew + sub;
   const bool active = sub < kUpdElemsPerWave && e < ne;
-  const double* cy  = cache + (active ? e : 0) * kEasCache;
-  double z          = 0.0;
-  if (active) {
-    z = cy[NE * 24 + i];
+  const int64_t nw  = ne - ew < kUpdElemsPerWave ? (ne - ew > 0 ? ne - ew : 0) : kUpdElemsPerWave;
+  constexpr int RUN = (kUpdElemsPerWave * kEasCache / 2 + 63) / 64;
+  const int run     = (int)nw * (kEasCache / 2);
+  const v2d* src = (const v2d*)(cache + ew * kEasCache);
+  v2d v[RUN];
+#pragma unroll
+  for (int m = 0; m < RUN; ++m)
+    if (lane + 64 * m < run) v[m] = src[lane + 64 * m];
+  double d[24];
+  if (active)
+#pragma unroll
     for (int a = 0; a < 8; ++a) {
       const int64_t nd = conn[e * 8 + a];
-      for (int k = 0; k < 3; ++k) z += cy[(a * 3 + k) * NE + i] * du[nd * 3 + k];
+#pragma unroll
+      for (int k = 0; k < 3; ++k) d[3 * a + k] = du[nd * 3 + k];
     }
+#pragma unroll
+  for (int m = 0; m < RUN; ++m)
+    if (lane + 64 * m < run) sw[wave][lane + 64 * m] = v[m];
+  waveSync();
+  const double* cy = (const double*)sw[wave] + (active ? sub : 0) * kEasCache;
+  const int p = i >> 2, k = i & 3;
+  const double* c1 = i < 20 ? cy + 64 * p + 16 * k - 16 : cy + 696 - NE;        // columns 16-31
+  const double* c2 = i < 20 ? cy + 320 + 56 * p + 14 * k - 32 : cy + 696 - NE;  // columns 32-45
+  double z         = 0.0;
+  if (active) {
+    z = c2[45];
+#pragma unroll
+    for (int j = 0; j < 24; ++j) z += (j < 11 ? c1 : c2)[NE + j] * d[j];
   }
   // every lane takes part in the shuffles; lanes of other elements and idle lanes read values they drop
-  for (int k = NE - 1; k > 0; --k) {
-    const double xk = __shfl(z, NE * sub + k, 64);
-    if (active && i < k) z -= cy[NE * 25 + k * (k - 1) / 2 + i] * xk;
+  const double* c0 = cy + cacheLow(p) + (12 - 4 * p) * k - 4 * (p + 1);  // columns below 16 (panels 0-2)
+#pragma unroll
+  for (int m = NE - 1; m >= 4; --m) {
+    const double xm = __shfl(z, NE * sub + m, 64);
+    if (active && p < (m >> 2)) z -= (m < 16 ? c0 : c1)[m] * xm;
   }
   if (active) alpha[e * NE + i] -= z;
 }
 
+template <bool WK, int E>
+void launchEasElems(ik_handle* h, int64_t e0, int64_t count, const int32_t* dest, const int32_t* rdest, double* Kebe) {
+  auto launch = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3((unsigned)((count + E - 1) / E)), dim3(64), 0, h->stream, h->X.p, h->u.p,
+                       h->conn.p, h->alpha.p, e0, count, h->lam, h->mu, dest, rdest, Kebe, h->ebeR.p, h->faceBits.p,
+                       loadedTraction(h), h->easCache.p, h->errFlag.p);
+  };
+  if (h->material == IK_SVK)
+    launch(easElement<IK_SVK, WK, E>);
+  else
+    launch(easElement<IK_NEOHOOKE, WK, E>);
+}
 template <bool WK>
 void launchEas(ik_handle* h, int64_t e0, int64_t count, const int32_t* dest, const int32_t* rdest, double* Kebe) {
-  if (h->material == IK_SVK)
-    hipLaunchKernelGGL((easElement<IK_SVK, WK>), dim3((unsigned)count), dim3(64), 0, h->stream, h->X.p, h->u.p,
-                       h->conn.p, h->alpha.p, e0, h->lam, h->mu, dest, rdest, Kebe, h->ebeR.p, h->faceBits.p, loadedTraction(h), h->easCache.p,
-                       h->errFlag.p);
-  else
-    hipLaunchKernelGGL((easElement<IK_NEOHOOKE, WK>), dim3((unsigned)count), dim3(64), 0, h->stream, h->X.p,
-                       h->u.p, h->conn.p, h->alpha.p, e0, h->lam, h->mu, dest, rdest, Kebe, h->ebeR.p, h->faceBits.p, loadedTraction(h), h->easCache.p,
-                       h->errFlag.p);
+  (count <= kEasOne   ? launchEasElems<WK, 1>
+   : count <= kEasTwo ? launchEasElems<WK, 2>
+                      : launchEasElems<WK, 4>)(h, e0, count, dest, rdest, Kebe);
 }
 
 }  // namespace
@@ -680,9 +675,9 @@ void easStage(ik_handle* h, int64_t e0, int64_t count, bool wantK, const int32_t
 
 void easUpdate(ik_handle* h, const double* duDev) {
   require(h->easCacheValid, IK_EINVAL, "EAS update needs D, L, Rt of the current state (assemble first)");
-  const int64_t perBlock = 4 * kUpdElemsPerWave;
-  hipLaunchKernelGGL(easUpdateKernel, dim3((unsigned)((h->ne + perBlock - 1) / perBlock)), dim3(256), 0, h->stream, h->easCache.p,
-                     h->conn.p, duDev, h->ne, h->alpha.p);
+  const int64_t perBlock = kUpdWaves * kUpdElemsPerWave;
+  hipLaunchKernelGGL(easUpdateKernel, dim3((unsigned)((h->ne + perBlock - 1) / perBlock)), dim3(64 * kUpdWaves), 0,
+                     h->stream, h->easCache.p, h->conn.p, duDev, h->ne, h->alpha.p);
   h->easCacheValid = false;
 }
 
