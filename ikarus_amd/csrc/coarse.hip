@@ -296,26 +296,66 @@ __device__ inline void groupSums(double (&v)[N], double (&red)[W][N]) {
 }
 
 // PCG iteration of the two-level form, part 1 (one workgroup per aggregate, over its nodes): alpha = r.z / p.q
-// (every workgroup folds the npq p.q partials in the same order; workgroup 0 records the scalars),
-// x += alpha p, r -= alpha q, and for the new r: the r.r and r.D^-1 r partials (partial[a], partial[na + a]) and
-// the restriction s_a = sum B(d_i)^T r_i (constrained components zeroed). With w = G s, r.z = r.D^-1 r + w.s,
-// since r . B(d_i) w_a summed over the nodes is w_a . s_a.
+// (every workgroup folds the npq p.q partials in the same order; workgroup 0 records the scalars), r -= alpha q, and
+// for the new r: the r.r and r.D^-1 r partials (partial[a], partial[na + a]) and the restriction s_a = sum B(d_i)^T r_i
+// (constrained components zeroed). With w = G s, r.z = r.D^-1 r + w.s, since r . B(d_i) w_a summed over the nodes is
+// w_a . s_a. Bound by the nodes' scattered lines (an aggregate's nodes are runs of about 9), so it reads only what it
+// must: x += alpha p waits for part 3, which reads p in node order anyway (64^3: 15.8 -> 12.8 us here, 6.6 -> 8.1
+// there; with the loads behind the folds instead of ahead of them both kernels take 2 us more).
 template <int BS>
-__global__ __launch_bounds__(BS) void coarseUpdate(float* __restrict__ x, float* __restrict__ r,
-                                                    const float* __restrict__ p, const float* __restrict__ q,
+__global__ __launch_bounds__(BS) void coarseUpdate(float* __restrict__ r, const float* __restrict__ q,
                                                     const float* __restrict__ binv, const uint8_t* __restrict__ fixed,
                                                     const float* __restrict__ dd, const int32_t* __restrict__ aggPtr,
                                                     const int32_t* __restrict__ aggNodes, int na, float* __restrict__ s,
                                                     const double* __restrict__ pq, int npq,
                                                     double* __restrict__ partial, PcgScalars* __restrict__ sc) {
-  if (sc->done) return;
   __shared__ double red1[BS / 64][1];
   __shared__ double red8[BS / 64][8];
-  const int a = blockIdx.x;
-  double pqv[1] = {0.0};
-  for (int i = threadIdx.x; i < npq; i += BS) pqv[0] += pq[i];
-  groupSums<BS / 64, 1>(pqv, red1);
+  const int a = blockIdx.x, end = aggPtr[a + 1];
+  if (sc->done) {
+    if (a == 0 && threadIdx.x == 0) sc->halt = 1;  // part 3 sets `done` itself, while its other workgroups start
+    return;
+  }
+  struct Node {
+    float r[3], q[3], B[9], d[3];
+    int f[3];
+    int i;
+  };
+  auto load = [&](int i, Node& n) {
+    n.i = i;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      const int64_t j = 3 * (int64_t)i + k;
+      n.r[k] = r[j];
+      n.q[k] = q[j];
+      n.d[k] = dd[j];
+      n.f[k] = fixed[j];
+    }
+#pragma unroll
+    for (int k = 0; k < 9; ++k) n.B[k] = binv[9 * (int64_t)i + k];
+  };
+  // the loads of the thread's first two nodes are in flight while the block folds p.q
+  int t          = aggPtr[a] + threadIdx.x;
+  const int i0 = t < end ? aggNodes[t] : 0, i1 = t + BS < end ? aggNodes[t + BS] : 0;
   const double rz = sc->rz_new;  // r.z of the current iterate (set by the previous p update or the init fold)
+  double pv[4];
+#pragma unroll
+  for (int u = 0; u < 4; ++u) pv[u] = (int)threadIdx.x + u * BS < npq ? pq[threadIdx.x + u * BS] : 0.0;
+  Node n0, n1;
+  load(i0, n0);
+  load(i1, n1);
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    Node& n = h ? n1 : n0;
+    arrived(n.r);
+    arrived(n.q);
+    arrived(n.B);
+    arrived(n.d);
+    arrived(n.f);
+  }
+  double pqv[1] = {(pv[0] + pv[1]) + (pv[2] + pv[3])};
+  for (int i = threadIdx.x + 4 * BS; i < npq; i += BS) pqv[0] += pq[i];
+  groupSums<BS / 64, 1>(pqv, red1);
   const double alpha = rz / pqv[0];
   if (a == 0 && threadIdx.x == 0) {
     sc->rz    = rz;
@@ -325,26 +365,28 @@ __global__ __launch_bounds__(BS) void coarseUpdate(float* __restrict__ x, float*
   const float al = (float)alpha;
   double rr = 0.0, rzb = 0.0;
   float sa[6] = {0, 0, 0, 0, 0, 0};
-  for (int t = aggPtr[a] + threadIdx.x; t < aggPtr[a + 1]; t += BS) {
-    const int64_t i = aggNodes[t];
+  auto add = [&](const Node& n) {
     float rl[3], v[3], o[6];
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
-      const int64_t j = 3 * i + k;
-      x[j] += al * p[j];
-      rl[k] = r[j] - al * q[j];
+      const int64_t j = 3 * (int64_t)n.i + k;
+      rl[k] = n.r[k] - al * n.q[k];
       r[j]  = rl[k];
       rr += (double)rl[k] * (double)rl[k];
-      v[k] = fixed[j] ? 0.0f : rl[k];
+      v[k] = n.f[k] ? 0.0f : rl[k];
     }
-    const float* B = binv + i * 9;
 #pragma unroll
     for (int k = 0; k < 3; ++k)
-      rzb += (double)rl[k] * (double)(B[3 * k] * rl[0] + B[3 * k + 1] * rl[1] + B[3 * k + 2] * rl[2]);
-    const float di[3] = {dd[3 * i], dd[3 * i + 1], dd[3 * i + 2]};
-    modesT<float>(v, di, o);
+      rzb += (double)rl[k] * (double)(n.B[3 * k] * rl[0] + n.B[3 * k + 1] * rl[1] + n.B[3 * k + 2] * rl[2]);
+    modesT<float>(v, n.d, o);
 #pragma unroll
     for (int m = 0; m < 6; ++m) sa[m] += o[m];
+  };
+  if (t < end) add(n0);
+  if (t + BS < end) add(n1);
+  for (t += 2 * BS; t < end; t += BS) {
+    load(aggNodes[t], n0);
+    add(n0);
   }
   double v[8] = {rr, rzb, sa[0], sa[1], sa[2], sa[3], sa[4], sa[5]};
   groupSums<BS / 64, 8>(v, red8);
@@ -387,27 +429,72 @@ __global__ __launch_bounds__(256) void coarseGemvDot(const float4* __restrict__ 
 }
 
 // part 3: every workgroup folds r.r, r.D^-1 r (2 na partials) and w.s (nws partials) in the same order; the
-// convergence test and beta = r.z / r.z_prev, then p = z + beta p with z_i = D_i^-1 r_i + B(d_i) w_a
-// (constrained components of the coarse part zeroed) formed on the fly
-__global__ __launch_bounds__(256) void coarseBetaP(float* __restrict__ p, const float* __restrict__ r,
+// convergence test and beta = r.z / r.z_prev, then x += alpha p and, unless converged, p = z + beta p with
+// z_i = D_i^-1 r_i + B(d_i) w_a (constrained components of the coarse part zeroed) formed on the fly
+__global__ __launch_bounds__(256) void coarseBetaP(float* __restrict__ x, float* __restrict__ p,
+                                                   const float* __restrict__ r,
                                                    const float* __restrict__ binv, const uint8_t* __restrict__ fixed,
                                                    const float* __restrict__ dd, const int32_t* __restrict__ agg,
                                                    const float* __restrict__ w, int64_t nn,
                                                    const double* __restrict__ partial, int na,
                                                    const double* __restrict__ ws, int nws,
                                                    PcgScalars* __restrict__ sc, int maxIter) {
-  if (sc->done) return;
+  if (sc->halt) return;
   __shared__ double red3[4][3];
-  double f[3] = {0.0, 0.0, 0.0};  // r.r, r.D^-1 r, w.s
-  for (int i = threadIdx.x; i < na; i += 256) {
-    f[0] += partial[i];
-    f[1] += partial[na + i];
+  struct Node {
+    float x[3], r[3], p[3], d[3], B[9], w[6];
+    int f[3];
+  };
+  auto load = [&](int64_t i, int32_t a, Node& n) {
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      n.r[k] = r[3 * i + k];
+      n.p[k] = p[3 * i + k];
+      n.x[k] = x[3 * i + k];
+      n.d[k] = dd[3 * i + k];
+      n.f[k] = fixed[3 * i + k];
+    }
+#pragma unroll
+    for (int k = 0; k < 9; ++k) n.B[k] = binv[9 * i + k];
+#pragma unroll
+    for (int m = 0; m < 6; ++m) n.w[m] = w[6 * a + m];
+  };
+  // the loads of the thread's first two nodes are in flight while the block folds the partials
+  const int64_t stride = (int64_t)gridDim.x * 256;
+  int64_t i            = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  const int64_t i0 = i < nn ? i : 0, i1 = i + stride < nn ? i + stride : 0;
+  const int32_t a0 = agg[i0], a1 = agg[i1];
+  const double threshold = sc->threshold, rzPrev = sc->rz, alpha = sc->alpha;
+  double v[4][3];
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    const int j = threadIdx.x + 256 * u;
+    v[u][0] = j < na ? partial[j] : 0.0;
+    v[u][1] = j < na ? partial[na + j] : 0.0;
+    v[u][2] = j < nws ? ws[j] : 0.0;
   }
-  for (int i = threadIdx.x; i < nws; i += 256) f[2] += ws[i];
+  Node n0, n1;
+  load(i0, a0, n0);
+  load(i1, a1, n1);
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    Node& n = h ? n1 : n0;
+    arrived(n.r);
+    arrived(n.p);
+    arrived(n.x);
+    arrived(n.d);
+    arrived(n.f);
+    arrived(n.B);
+    arrived(n.w);
+  }
+  double f[3];  // r.r, r.D^-1 r, w.s
+#pragma unroll
+  for (int k = 0; k < 3; ++k) f[k] = (v[0][k] + v[1][k]) + (v[2][k] + v[3][k]);
+  for (int j = threadIdx.x + 1024; j < nws; j += 256) f[2] += ws[j];  // na <= kMaxAggregates = 1024
   groupSums<4, 3>(f, red3);
   const double rr = f[0], rz = f[1] + f[2];
-  const bool conv = rr < sc->threshold;
-  const double bt = rz / sc->rz;
+  const bool conv = rr < threshold;
+  const double bt = rz / rzPrev;
   if (blockIdx.x == 0 && threadIdx.x == 0) {
     sc->rr = rr;
     if (conv) {
@@ -419,23 +506,25 @@ __global__ __launch_bounds__(256) void coarseBetaP(float* __restrict__ p, const 
       if (sc->iters >= maxIter) sc->done = 2;
     }
   }
-  if (conv) return;
-  const float beta = (float)bt;
-  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < nn; i += (int64_t)gridDim.x * 256) {
-    const float rl[3] = {r[3 * i], r[3 * i + 1], r[3 * i + 2]};
-    const float di[3] = {dd[3 * i], dd[3 * i + 1], dd[3 * i + 2]};
-    const int32_t a   = agg[i];
-    float wa[6], cz[3];
+  const float beta = (float)bt, al = (float)alpha;
+  auto store = [&](int64_t i, const Node& n) {
 #pragma unroll
-    for (int m = 0; m < 6; ++m) wa[m] = w[6 * a + m];
-    modes<float>(wa, di, cz);
-    const float* B = binv + i * 9;
+    for (int k = 0; k < 3; ++k) x[3 * i + k] = n.x[k] + al * n.p[k];
+    if (conv) return;
+    float cz[3];
+    modes<float>(n.w, n.d, cz);
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
-      float zk = B[3 * k] * rl[0] + B[3 * k + 1] * rl[1] + B[3 * k + 2] * rl[2];
-      if (!fixed[3 * i + k]) zk += cz[k];
-      p[3 * i + k] = zk + beta * p[3 * i + k];
+      float zk = n.B[3 * k] * n.r[0] + n.B[3 * k + 1] * n.r[1] + n.B[3 * k + 2] * n.r[2];
+      if (!n.f[k]) zk += cz[k];
+      p[3 * i + k] = zk + beta * n.p[k];
     }
+  };
+  if (i < nn) store(i, n0);
+  if (i + stride < nn) store(i + stride, n1);
+  for (i += 2 * stride; i < nn; i += stride) {
+    load(i, agg[i], n0);
+    store(i, n0);
   }
 }
 
@@ -702,14 +791,14 @@ void coarseApply(ik_handle* h, const float* r, float* z, float* p, const float* 
 void coarseIteration(ik_handle* h, const double* pq, int npq, float* x, float* r, float* p, const float* q,
                      const float* binv, int gn, double* partial, int maxIter) {
   Coarse& cs = *h->coarse;
-  hipLaunchKernelGGL(coarseUpdate<kUpdateThreads>, dim3((unsigned)cs.na), dim3(kUpdateThreads), 0, h->stream, x, r,
-                     p, q, binv, h->fixed.p,
-                     cs.d.p, cs.aggPtr.p, cs.aggNodes.p, (int)cs.na, cs.s.p, pq, npq, partial, h->sc.p);
+  hipLaunchKernelGGL(coarseUpdate<kUpdateThreads>, dim3((unsigned)cs.na), dim3(kUpdateThreads), 0, h->stream, r, q,
+                     binv, h->fixed.p, cs.d.p, cs.aggPtr.p, cs.aggNodes.p, (int)cs.na, cs.s.p, pq, npq, partial,
+                     h->sc.p);
   const unsigned gg = (unsigned)((cs.nc + 3) / 4);
   hipLaunchKernelGGL(coarseGemvDot, dim3(gg), dim3(256), 0, h->stream, (const float4*)cs.G.p, (const float4*)cs.s.p,
                      cs.s.p, cs.w.p, cs.nc, cs.ld / 4, cs.ws.p, h->sc.p);
-  hipLaunchKernelGGL(coarseBetaP, dim3(gn), dim3(256), 0, h->stream, p, r, binv, h->fixed.p, cs.d.p, cs.agg.p, cs.w.p,
-                     h->nn, partial, (int)cs.na, cs.ws.p, (int)gg, h->sc.p, maxIter);
+  hipLaunchKernelGGL(coarseBetaP, dim3(gn), dim3(256), 0, h->stream, x, p, r, binv, h->fixed.p, cs.d.p, cs.agg.p,
+                     cs.w.p, h->nn, partial, (int)cs.na, cs.ws.p, (int)gg, h->sc.p, maxIter);
 }
 
 }  // namespace ik

@@ -96,6 +96,7 @@ struct PcgScalars {
   double threshold; // tol^2 ||b||^2
   int32_t done;
   int32_t iters;
+  int32_t halt;     // two-level form: `done` was set before the current iteration
   double bb;        // ||b||^2
 };
 

@@ -28,16 +28,6 @@ constexpr int spmvRowsPerBlock() {
   return SPMV_BS / 64 / G * spmvRowsPerWave<TV>();
 }
 
-// Waits for a loaded value here: the loads above it are in flight together, instead of each behind the branch or
-// barrier that precedes its use
-__device__ inline void arrived(double& v) { asm volatile("" : "+v"(v)); }
-__device__ inline void arrived(float& v) { asm volatile("" : "+v"(v)); }
-template <typename T, int N>
-__device__ inline void arrived(T (&v)[N]) {
-#pragma unroll
-  for (int i = 0; i < N; ++i) arrived(v[i]);
-}
-
 // block-wide sum; result valid in thread 0
 template <int BS>
 __device__ inline double blockSum(double v) {
@@ -458,6 +448,7 @@ __global__ __launch_bounds__(1024) void pcgInitFold(const double* __restrict__ p
     const double thr = tol2 * rr;
     sc->threshold = thr > 2.2250738585072014e-308 ? thr : 2.2250738585072014e-308;
     sc->iters     = 0;
+    sc->halt      = 0;
     sc->done      = (rr == 0.0 || rr < sc->threshold) ? 1 : 0;
     sc->alpha = sc->beta = 0.0;
   }

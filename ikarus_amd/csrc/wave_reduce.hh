@@ -1,4 +1,4 @@
-// wave_reduce.hh — sums over the 64 lanes of a wavefront by DPP moves.
+// wave_reduce.hh — sums over the 64 lanes of a wavefront by DPP moves, and a wait for loads.
 //
 // Shifts within rows of 16 lanes, then the row totals broadcast across rows; lane 63 ends with the total, read into a
 // scalar register. A shuffle-based tree goes through the LDS crossbar at every step: a double's six steps take about
@@ -40,6 +40,17 @@ __device__ inline T waveSum(T v) {
   v += dppMove<0x142, 0xA>(v);  // row_bcast:15 into rows 1 and 3
   v += dppMove<0x143, 0xC>(v);  // row_bcast:31 into rows 2 and 3
   return lane63(v);
+}
+
+// Waits for a loaded value here: the loads above it are in flight together, instead of each behind the branch or
+// barrier that precedes its use
+__device__ inline void arrived(double& v) { asm volatile("" : "+v"(v)); }
+__device__ inline void arrived(int& v) { asm volatile("" : "+v"(v)); }
+__device__ inline void arrived(float& v) { asm volatile("" : "+v"(v)); }
+template <typename T, int N>
+__device__ inline void arrived(T (&v)[N]) {
+#pragma unroll
+  for (int i = 0; i < N; ++i) arrived(v[i]);
 }
 
 }  // namespace ik

@@ -78,3 +78,21 @@ def test_residual_at_the_splits(kind, n, shuffle):
     again, _ = dev.solve(b, ia.solver_opts(kind=kind, rtol=1e-9, inner_rtol=1e-3))
     assert np.array_equal(x, again)  # fixed summation order
     dev.close()
+
+
+@pytest.mark.parametrize("kind", [capi.PCG_BJACOBI_FP32_IR, capi.PCG_TWOLEVEL_FP32_IR])
+@pytest.mark.parametrize("max_iter", [1, 2, 16, 17])
+def test_mixed_iterate_at_the_limit(kind, max_iter):
+    """After any number of inner iterations of one sweep the iterate is orthogonal to its residual (conjugate gradients
+    minimise over the directions, which span it): to 1e-4 in FP32, with 13^3 nodes in several workgroups."""
+    print(f"case: mixed limit kind={kind} max_iter={max_iter}", flush=True)
+    p, u, b = _setup((12, 12, 12))
+    dev = ia.Device(p)
+    dev.set_requirement(u, 0.5)
+    dev.matrix(capi.DBC_FULL, capi.FP32)
+    x, info = dev.solve(b, ia.solver_opts(kind=kind, rtol=1e-12, inner_rtol=1e-9, max_iter=max_iter, max_refine=1))
+    outer, inner, vals = dev.csc(capi.DBC_FULL)
+    r = b - sp.csc_matrix((vals, inner, outer), shape=(p.ndof, p.ndof)) @ x
+    assert np.linalg.norm(r) / np.linalg.norm(b) == pytest.approx(info.rel_residual, rel=1e-9)
+    assert abs(x @ r) < 1e-4 * np.linalg.norm(x) * np.linalg.norm(r)
+    dev.close()
