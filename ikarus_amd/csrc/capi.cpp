@@ -578,7 +578,7 @@ int ik_create(ik_handle** out, const ik_problem_desc* d0) {
 void ik_destroy(ik_handle* h) {
   if (!h) return;
   if (h->stream) (void)hipStreamSynchronize(h->stream);
-  if (h->hsc) (void)hipHostFree(h->hsc);
+  if (h->pcg) (void)hipHostFree(h->pcg);
   if (h->hred) (void)hipHostFree(h->hred);
   if (h->herr) (void)hipHostFree(h->herr);
   if (h->ev0) (void)hipEventDestroy(h->ev0);

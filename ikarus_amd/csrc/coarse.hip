@@ -27,6 +27,7 @@
 
 #include "host_parallel.hh"
 #include "ik_internal.hh"
+#include "pcg_record.hh"
 #include "wave_reduce.hh"
 
 namespace ik {
@@ -495,17 +496,7 @@ __global__ __launch_bounds__(256) void coarseBetaP(float* __restrict__ x, float*
   const double rr = f[0], rz = f[1] + f[2];
   const bool conv = rr < threshold;
   const double bt = rz / rzPrev;
-  if (blockIdx.x == 0 && threadIdx.x == 0) {
-    sc->rr = rr;
-    if (conv) {
-      sc->done = 1;
-    } else {
-      sc->beta   = bt;
-      sc->rz_new = rz;
-      sc->iters += 1;
-      if (sc->iters >= maxIter) sc->done = 2;
-    }
-  }
+  if (blockIdx.x == 0 && threadIdx.x == 0) pcgRecord(sc, rr, rz, bt, conv, maxIter);
   const float beta = (float)bt, al = (float)alpha;
   auto store = [&](int64_t i, const Node& n) {
 #pragma unroll

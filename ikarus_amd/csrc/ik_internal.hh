@@ -86,6 +86,13 @@ struct DevBuf {
   }
 };
 
+// Progress of a PCG run in pinned host memory, written by the device at its end and every kPcgPublish iterations
+constexpr int kPcgPublish = 8;
+struct PcgMirror {
+  double rr, bb;             // valid once done
+  unsigned long long state;  // run << 32 | iterations << 2 | done
+};
+
 // Device scalars of one PCG run (Eigen ConjugateGradient state, linearsolver.cpp:23-24)
 struct PcgScalars {
   double rz;        // r . z of the current iterate
@@ -98,6 +105,8 @@ struct PcgScalars {
   int32_t iters;
   int32_t halt;     // two-level form: `done` was set before the current iteration
   double bb;        // ||b||^2
+  PcgMirror* mirror;
+  uint32_t run;     // number of the run, in the mirror's state
 };
 
 enum KernelId { KASM_KR = 0, KASM_R = 1, KSPMV = 2, KMLP = 3, KGATHER = 4, KCOUNT = 5 };
@@ -248,7 +257,8 @@ struct ik_handle {
   ik::DevBuf<double> pr, pz, pp, pq, px, pdiag, pb, partial;
   ik::DevBuf<float> fr, fp, fp2, fz, fq, fx, fdiag;  // FP32 PCG vectors; fdiag holds 3x3 block inverses
   ik::DevBuf<ik::PcgScalars> sc;
-  ik::PcgScalars* hsc = nullptr;  // pinned host mirror
+  ik::PcgMirror* pcg = nullptr;  // pinned
+  uint32_t pcgRun = 0;           // number of the last PCG run
   double* hred = nullptr;         // pinned host scalar for reductions
   unsigned long long* herr = nullptr;  // pinned host copy of the determinant-failure flag
 

@@ -7,9 +7,9 @@
 // preconditioner, wrapped in FP64 iterative refinement (r = b - K x accumulated in FP64).
 //
 // All PCG scalars live on the device; each kernel reads a `done` flag so the host can enqueue
-// iterations in chunks and poll the flag asynchronously: the iterate after convergence is exactly the
-// one Eigen's loop returns.
+// iterations ahead of the test: the iterate after convergence is exactly the one Eigen's loop returns.
 #include "ik_internal.hh"
+#include "pcg_record.hh"
 #include "wave_reduce.hh"
 
 namespace ik {
@@ -226,17 +226,7 @@ struct PcgTest {
     rz              = bc[1];
     const bool conv = rr < threshold;
     beta            = rz / rzPrev;
-    if (record && threadIdx.x == 0) {
-      sc->rr = rr;
-      if (conv) {
-        sc->done = 1;
-      } else {
-        sc->beta   = beta;
-        sc->rz_new = rz;
-        sc->iters += 1;
-        if (sc->iters >= maxIter) sc->done = 2;
-      }
-    }
+    if (record && threadIdx.x == 0) pcgRecord(sc, rr, rz, beta, conv, maxIter);
     return !conv;
   }
 };
@@ -432,7 +422,7 @@ __global__ __launch_bounds__(256) void pcgInitKernel(const double* __restrict__ 
 }
 
 __global__ __launch_bounds__(1024) void pcgInitFold(const double* __restrict__ partial, int nb, double tol2,
-                                                    PcgScalars* __restrict__ sc) {
+                                                    PcgScalars* __restrict__ sc, PcgMirror* mirror, uint32_t run) {
   double rr = 0.0, rz = 0.0;
   for (int i = threadIdx.x; i < nb; i += 1024) {
     rr += partial[i];
@@ -451,6 +441,9 @@ __global__ __launch_bounds__(1024) void pcgInitFold(const double* __restrict__ p
     sc->halt      = 0;
     sc->done      = (rr == 0.0 || rr < sc->threshold) ? 1 : 0;
     sc->alpha = sc->beta = 0.0;
+    sc->mirror           = mirror;
+    sc->run              = run;
+    pcgPublish(sc, rr, 0, sc->done);
   }
 }
 
@@ -742,7 +735,8 @@ static void ensureWork(ik_handle* h) {
   h->partial.ensure((size_t)(2 * kReduceBlocks + spmvBlocks) + kPqBlocks + 8);
   if (!h->sc.p) {
     h->sc.ensure(1);
-    IK_HIP(hipHostMalloc((void**)&h->hsc, sizeof(PcgScalars), hipHostMallocDefault));
+    IK_HIP(hipHostMalloc((void**)&h->pcg, sizeof(PcgMirror), hipHostMallocCoherent));
+    h->pcg->state = 0;
     IK_HIP(hipHostMalloc((void**)&h->hred, sizeof(double) * 4, hipHostMallocDefault));
   }
 }
@@ -793,57 +787,85 @@ void axpy(ik_handle* h, double a, const double* x, double* y, int64_t n) {
   hipLaunchKernelGGL(axpyKernel, dim3(vecGrid(n)), dim3(256), 0, h->stream, a, x, y, n);
 }
 
-// Poll interval: iterations enqueued before the first host check of the done flag (32: a two-level inner solve
-// takes 24-32 at 64^3, so most need no second check) and between later checks (64). Iterations enqueued after
-// convergence return at once (a few us of launches each); a check leaves the device idle for a host round trip
-// (20-45 us) while the next iterations are enqueued.
-static int pollChunk(int enq) { return enq == 0 ? 32 : 64; }
+// Iterations are enqueued at most kPcgAhead beyond the count that the device last wrote into the handle's pinned
+// mirror: enough that it never waits for the host (the four left when a count arrives take it 40 us or more), and few
+// launches after convergence (they return at once, one and a half to two us each). Against 32, then 64 iterations
+// between reads of the flag with the stream drained: two-level solve at 64^3 13.45 -> 12.44 ms, FP32 block Jacobi at
+// 20^3 8.4 -> 7.2 ms, ten load steps of the 64 x 16 plane 147-154 -> 132-138 ms. 4 / 8 / 12 / 16 / 24 iterations
+// between the counts, four more ahead: the two-level solve 12.6 / 12.44 / 12.41 / 12.44 / 12.67 ms, the others within
+// their noise.
+constexpr int kPcgAhead = 12;
+static_assert(kPcgAhead > kPcgPublish + 1, "the device publishes within what may be enqueued");
 
-// The iterations of one PCG solve, after its init kernels: enqueued in chunks until the done flag or maxIter. p holds
+// State of the current PCG run (iterations << 2 | done); `before` until the run has started
+static unsigned pcgState(ik_handle* h, unsigned before) {
+  const unsigned long long s = __atomic_load_n(&h->pcg->state, __ATOMIC_ACQUIRE);
+  if ((uint32_t)(s >> 32) != h->pcgRun) return before;
+  finishErrCheck(h);  // the element kernels' flags were copied ahead of this run
+  return (unsigned)s;
+}
+
+// waits for a state after `before`
+static unsigned pcgWait(ik_handle* h, unsigned before) {
+  bool idle = false;
+  for (unsigned spin = 1;; ++spin) {
+    const unsigned s = pcgState(h, before);
+    if (s != before) return s;
+    if (idle) throw Error{IK_EHIP, "internal error: the PCG run ended without a result"};
+    if (spin % 4096 == 0) {  // a launch or device that failed: an error here, not a wait without end
+      const hipError_t query = hipStreamQuery(h->stream);
+      idle                   = query == hipSuccess;
+      if (query == hipErrorNotReady)
+        (void)hipGetLastError();
+      else
+        IK_HIP(query);
+    }
+    __builtin_ia32_pause();
+  }
+}
+
+// The iterations of one PCG solve, after its init kernels: enqueued until the done flag or maxIter. p holds
 // the first direction, or zero with z = M^-1 r when z is given (the direction is then formed inside the SpMV,
 // alternating between p and p2). coarse: the two-level form's vector kernels instead of update and direction.
 template <typename T>
 static void pcgLoop(ik_handle* h, const T* K, T* x, T* r, T* p, T* p2, T* z, T* q, const T* pre, int64_t n,
                     int grid, int maxIter, bool coarse) {
   const unsigned sgrid = spmvGrid<T>(h->nn);
-  int enq              = 0;
-  for (;;) {
-    for (int c = 0, cn = pollChunk(enq); c < cn && enq < maxIter; ++c, ++enq) {
-      if (z) {
-        if (enq > 0) std::swap(p, p2);
-        ScopedKernelTimer t(h, KSPMV);
-        hipLaunchKernelGGL((pcgDirectionSpmv<T, kSplit>), dim3(sgrid), dim3(SPMV_BS), 0, h->stream, h->rowptr.p,
-                           h->sellStart.p, h->scol.p, K, z, p, p2, q, h->nn, h->partial.p, grid, pqPartials(h),
-                           h->sc.p, maxIter, c > 0 ? 1 : 0);
-      } else {
-        launchSpmv<T, T>(h, K, p, q, pqPartials(h), h->sc.p, enq & 1);
-      }
-      const double* pqSrc = pqPartials(h);
-      int npq             = (int)sgrid;
-      if (sgrid > (unsigned)kPqDirect) {
-        hipLaunchKernelGGL(pcgPqFold, dim3(kPqBlocks), dim3(256), 0, h->stream, pqPartials(h), (int)sgrid, pq2(h),
-                           h->sc.p);
-        pqSrc = pq2(h);
-        npq   = kPqBlocks;
-      }
-      if constexpr (std::is_same<T, float>::value)
-        if (coarse) {
-          coarseIteration(h, pqSrc, npq, x, r, p, q, pre, grid, h->partial.p, maxIter);
-          continue;
-        }
-      constexpr bool B = std::is_same<T, float>::value;  // FP64: diagonal preconditioner, FP32: 3x3 blocks
-      hipLaunchKernelGGL((pcgUpdateKernel<T, B>), dim3(grid), dim3(256), 0, h->stream, x, r, z ? p2 : p, q, pre, z, n,
-                         h->sc.p, pqSrc, npq, h->partial.p);
-      if (!z)
-        hipLaunchKernelGGL((pcgBetaPKernel<T, B>), dim3(grid), dim3(256), 0, h->stream, p, r, pre, n, h->partial.p,
-                           grid, h->sc.p, maxIter);
-    }
-    if (z)
+  unsigned state = 0;
+  for (int enq = 0;; ++enq) {
+    if (z && enq == maxIter)  // the last iteration's test, which no direction follows
       hipLaunchKernelGGL(pcgTestKernel, dim3(1), dim3(256), 0, h->stream, h->partial.p, grid, h->sc.p, maxIter);
-    IK_HIP(hipMemcpyAsync(h->hsc, h->sc.p, sizeof(PcgScalars), hipMemcpyDeviceToHost, h->stream));
-    IK_HIP(hipStreamSynchronize(h->stream));
-    finishErrCheck(h);
-    if (h->hsc->done || enq >= maxIter) break;
+    state = pcgState(h, state);
+    while (!(state & 3) && (enq == maxIter || enq - (int)(state >> 2) >= kPcgAhead)) state = pcgWait(h, state);
+    if (state & 3) break;
+    if (z) {
+      if (enq > 0) std::swap(p, p2);
+      ScopedKernelTimer t(h, KSPMV);
+      hipLaunchKernelGGL((pcgDirectionSpmv<T, kSplit>), dim3(sgrid), dim3(SPMV_BS), 0, h->stream, h->rowptr.p,
+                         h->sellStart.p, h->scol.p, K, z, p, p2, q, h->nn, h->partial.p, grid, pqPartials(h),
+                         h->sc.p, maxIter, enq > 0 ? 1 : 0);
+    } else {
+      launchSpmv<T, T>(h, K, p, q, pqPartials(h), h->sc.p, enq & 1);
+    }
+    const double* pqSrc = pqPartials(h);
+    int npq             = (int)sgrid;
+    if (sgrid > (unsigned)kPqDirect) {
+      hipLaunchKernelGGL(pcgPqFold, dim3(kPqBlocks), dim3(256), 0, h->stream, pqPartials(h), (int)sgrid, pq2(h),
+                         h->sc.p);
+      pqSrc = pq2(h);
+      npq   = kPqBlocks;
+    }
+    if constexpr (std::is_same<T, float>::value)
+      if (coarse) {
+        coarseIteration(h, pqSrc, npq, x, r, p, q, pre, grid, h->partial.p, maxIter);
+        continue;
+      }
+    constexpr bool B = std::is_same<T, float>::value;  // FP64: diagonal preconditioner, FP32: 3x3 blocks
+    hipLaunchKernelGGL((pcgUpdateKernel<T, B>), dim3(grid), dim3(256), 0, h->stream, x, r, z ? p2 : p, q, pre, z, n,
+                       h->sc.p, pqSrc, npq, h->partial.p);
+    if (!z)
+      hipLaunchKernelGGL((pcgBetaPKernel<T, B>), dim3(grid), dim3(256), 0, h->stream, p, r, pre, n, h->partial.p,
+                         grid, h->sc.p, maxIter);
   }
 }
 
@@ -865,11 +887,12 @@ void pcgJacobi64(ik_handle* h, const double* b, double* x, double rtol, int maxI
                      h->K64.p, h->nn, h->pdiag.p);
   hipLaunchKernelGGL(pcgInitKernel, dim3(g), dim3(256), 0, h->stream, b, h->pdiag.p, x, h->pr.p, h->pp.p, z, n,
                      h->partial.p);
-  hipLaunchKernelGGL(pcgInitFold, dim3(1), dim3(1024), 0, h->stream, h->partial.p, g, rtol * rtol, h->sc.p);
+  hipLaunchKernelGGL(pcgInitFold, dim3(1), dim3(1024), 0, h->stream, h->partial.p, g, rtol * rtol, h->sc.p,
+                     h->pcg, ++h->pcgRun);
   if (maxIter <= 0) maxIter = (int)(2 * n);
   pcgLoop<double>(h, h->K64.p, x, h->pr.p, h->pp.p, h->pb.p, z, h->pq.p, h->pdiag.p, n, g, maxIter, false);
-  *iters  = h->hsc->iters;
-  *relres = h->hsc->bb > 0 ? std::sqrt(h->hsc->rr / h->hsc->bb) : 0.0;
+  *iters  = (int)((unsigned)h->pcg->state >> 2);
+  *relres = h->pcg->bb > 0 ? std::sqrt(h->pcg->rr / h->pcg->bb) : 0.0;
 }
 
 void pcgMixed(ik_handle* h, const double* b, double* x, const ik_solver_opts* o, ik_solver_info* info,
@@ -925,9 +948,9 @@ void pcgMixed(ik_handle* h, const double* b, double* x, const ik_solver_opts* o,
                          h->fr.p, h->fp.p, z, h->nn, h->partial.p);
     }
     hipLaunchKernelGGL(pcgInitFold, dim3(1), dim3(1024), 0, h->stream, h->partial.p, gn, innerTol * innerTol,
-                       h->sc.p);
+                       h->sc.p, h->pcg, ++h->pcgRun);
     pcgLoop<float>(h, h->K32.p, h->fx.p, h->fr.p, h->fp.p, h->fp2.p, z, h->fq.p, h->fdiag.p, n, gn, maxIter, twoLevel);
-    info->iterations += h->hsc->iters + 1;
+    info->iterations += (int)((unsigned)h->pcg->state >> 2) + 1;
     info->refinements += 1;
     // x += ||r|| d ; r = b - K x in FP64
     hipLaunchKernelGGL(accumulateF32, dim3(g), dim3(256), 0, h->stream, x, h->fx.p, rnorm, n);
