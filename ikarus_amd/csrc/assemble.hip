@@ -26,6 +26,7 @@
 // apply the FULL Dirichlet treatment on the fly and write each block once. Large meshes are processed in chunks whose
 // gathers run behind them on the rows each chunk completes.
 #include "ik_internal.hh"
+#include "wave_reduce.hh"
 
 #include <type_traits>
 
@@ -53,7 +54,7 @@ __device__ inline double det3(const double A[3][3]) {
 }
 
 __device__ inline void inv3(const double A[3][3], double d, double I[3][3]) {
-  const double id = 1.0 / d;
+  const double id = reciprocal(d);
   I[0][0]         = (A[1][1] * A[2][2] - A[1][2] * A[2][1]) * id;
   I[0][1]         = (A[0][2] * A[2][1] - A[0][1] * A[2][2]) * id;
   I[0][2]         = (A[0][1] * A[1][2] - A[0][2] * A[1][1]) * id;
@@ -127,7 +128,7 @@ __device__ inline bool pointState(const double (*cf)[6], const double xi[3], dou
     const double detC = C[0] * (C[1] * C[2] - C[3] * C[3]) - C[5] * (C[5] * C[2] - C[3] * C[4]) +
                         C[4] * (C[5] * C[3] - C[1] * C[4]);
     const bool ok     = detC > 0.0;
-    const double lnJ  = log(sqrt(detC));
+    const double lnJ  = 0.5 * log(detC);
     s.w               = (mu - lam * lnJ) * s.dV;
     // P = mu (F - F^-T) + lambda ln J F^-T (zero to the last bit at u = 0)
     inv3(s.F, det3(s.F), s.Fi);
@@ -144,12 +145,13 @@ __device__ inline bool pointState(const double (*cf)[6], const double xi[3], dou
   }
 }
 
-// DPP lane moves within a row of 16 lanes (64-bit value as two 32-bit moves)
+// DPP lane moves within a row of 16 lanes (64-bit value as two 32-bit moves; bound control, although every source lane
+// exists: without it each move is preceded by one that clears its target)
 template <int CTRL>
 __device__ inline double dpp(double v) {
   const unsigned long long b = __builtin_bit_cast(unsigned long long, v);
-  const int lo = __builtin_amdgcn_update_dpp(0, (int)(unsigned)b, CTRL, 0xF, 0xF, false);
-  const int hi = __builtin_amdgcn_update_dpp(0, (int)(unsigned)(b >> 32), CTRL, 0xF, 0xF, false);
+  const int lo = __builtin_amdgcn_update_dpp(0, (int)(unsigned)b, CTRL, 0xF, 0xF, true);
+  const int hi = __builtin_amdgcn_update_dpp(0, (int)(unsigned)(b >> 32), CTRL, 0xF, 0xF, true);
   return __builtin_bit_cast(double, ((unsigned long long)(unsigned)hi << 32) | (unsigned long long)(unsigned)lo);
 }
 constexpr int DPP_XOR1 = 0xB1;   // quad_perm [1,0,3,2]
@@ -234,14 +236,15 @@ __device__ inline void cornerForces(const double Q[3][3], const double xi[3], in
     G[7][k] = Q[k][0] * x12 + Q[k][1] * x02 + Q[k][2] * x01;
   }
   // reduce-scatter over the element's eight lanes: keep the half of the monomials selected by this lane's
-  // bit, add the partner's partials of that half
+  // bit, add the partner's partials of that half (the first partner is lane 7 - q, one move, whose bit 2 differs; the
+  // lanes that keep one half then hold the sums of disjoint pairs)
   const bool b2 = (q >> 2) & 1, b1 = (q >> 1) & 1, b0 = q & 1;
   double n4[4][3];  // monomials j + 4 b2
 #pragma unroll
   for (int j = 0; j < 4; ++j)
 #pragma unroll
     for (int k = 0; k < 3; ++k)
-      n4[j][k] = (b2 ? G[j + 4][k] : G[j][k]) + laneXor<4>(b2 ? G[j][k] : G[j + 4][k]);
+      n4[j][k] = (b2 ? G[j + 4][k] : G[j][k]) + dpp<DPP_HALF_MIRROR>(b2 ? G[j][k] : G[j + 4][k]);
   double n2[2][3];  // monomials j + 2 b1 + 4 b2
 #pragma unroll
   for (int j = 0; j < 2; ++j)
@@ -347,7 +350,8 @@ __global__ __launch_bounds__(kTileThreads, KIND == IK_SVK ? 3 : 4) void hex8Tang
     gl = reinterpret_cast<uint32_t*>(gd + maxGroups);
     gm = reinterpret_cast<uint16_t*>(gl + maxGroups);
     const int4 m = tmeta[t];
-    g0 = m.x, m0 = m.y, nst = m.z & 0x3FF, n1 = (m.z >> 10) & 0x3FF, nm = m.z >> 20, nacc = m.w & 0xFFFF, most = m.w >> 16;
+    g0 = m.x, m0 = m.y, nst = m.z & 0x3FF, n1 = (m.z >> 10) & 0x3FF, nm = m.z >> 20;
+    nacc = m.w & 0xFFFF, most = m.w >> 16;
   }
   if (pw < PW) {
     const int el = pw * 8 + (lane >> 3), q = lane & 7;
@@ -642,6 +646,10 @@ __global__ __launch_bounds__(kTileThreads, KIND == IK_SVK ? 3 : 4) void hex8Tang
 // so with G_S = Q grad m_S summed over the element's points, R_a = sum_{S superset of a} (-1)^|S\a| G_S.
 // The eight Gauss-point lanes reduce-scatter their G_S (exchanges at lane distance 4, 2, 1, a fixed order),
 // which leaves G_q on lane q, and three more exchange steps turn G_q into corner q's three sums.
+// 128 x 128 x 64 elements, with the gather: 260 us a call against 291 (308 before the tangent's point form was shared):
+// 670 vector instructions per wavefront instead of 860 (no clearing before each lane move, one move instead of two in
+// the first exchange, short reciprocals) and stores to adjacent slots. Bound by the vector units (145 us) and the two
+// rounds of loads before them at four wavefronts per SIMD.
 template <int KIND>
 __global__ __launch_bounds__(64) void hex8Residual(const double* __restrict__ X, const double* __restrict__ U,
                                                    const int32_t* __restrict__ conn, int64_t e0, int64_t count,
@@ -649,13 +657,18 @@ __global__ __launch_bounds__(64) void hex8Residual(const double* __restrict__ X,
                                                    double* __restrict__ Rebe, const uint8_t* __restrict__ fbits,
                                                    double3 trac, unsigned long long* __restrict__ err) {
   __shared__ double CF[8][8][6];  // monomial coefficients of x (0..2) and u (3..5) per element
+  __shared__ int32_t slots[64];
   const int lane     = threadIdx.x;
   const int el       = lane >> 3, q = lane & 7;
   const int64_t base = (int64_t)blockIdx.x * 8;
   const int nvalid   = (int)(count - base < 8 ? count - base : 8);
   const bool valid   = el < nvalid;
   const int64_t e    = e0 + base + (valid ? el : nvalid - 1);
-  cornerCoefficients(X, U, conn[e * 8 + q], q, CF[el][q]);
+  const int32_t nd = conn[e * 8 + q];
+  int32_t slot     = rdest[e * 8 + q];
+  unsigned bits    = fbits ? fbits[e] : 0u;
+  cornerCoefficients(X, U, nd, q, CF[el][q]);
+  asm volatile("" : "+v"(slot), "+v"(bits));  // loaded here, not where they are used
   __syncthreads();
   double xi[3];
   gaussPoint(q, xi);
@@ -663,9 +676,20 @@ __global__ __launch_bounds__(64) void hex8Residual(const double* __restrict__ X,
   if (!pointState<KIND>(CF[el], xi, lam, mu, s) && valid) atomicMin(err, (unsigned long long)e);
   double r[3];
   cornerForces(s.Q, xi, q, r);
-  if (valid)
-    storeCorner(X, conn, e, q, r, fbits ? fbits[e] : 0u, trac,
-                Rebe + (rdest ? (int64_t)rdest[e * 8 + q] * 3 : e * 24 + 3 * q));
+  // through LDS, corner by corner over the eight elements: consecutive lanes then store to the adjacent slots that a
+  // row of elements has
+  __syncthreads();
+  double* out    = &CF[0][0][0];
+  const int from = q * 8 + el;
+  storeCorner(X, conn, e, q, r, bits, trac, out + from * 3);
+  slots[from] = valid ? slot : -1;
+  __syncthreads();
+#pragma unroll
+  for (int m = 0; m < 3; ++m) {
+    const int i = m * 64 + lane, c = i / 3;
+    const int32_t to = slots[c];
+    if (to >= 0) Rebe[(int64_t)to * 3 + (i - 3 * c)] = out[i];
+  }
 }
 
 // K gather: thread per (upper block, entry) over the gathered upper blocks [q0, q1) of one staging chunk (in
@@ -722,30 +746,27 @@ __global__ __launch_bounds__(256) void gatherK(const int32_t* __restrict__ segpt
   }
 }
 
-// R gather: thread per DOF over node rows [r0, r1); the node's staged corner contributions occupy the
-// contiguous slots [ncptr[n], ncptr[n+1]) (ordered by element) and are summed in that order.
+// R gather: thread per DOF over node rows [r0, r1); the node's staged corner contributions (see residualSlot; `tail`:
+// the first slot behind the slices) are summed in the order of their elements. 128 x 128 x 64 elements: 36 us against
+// 46 with each node's contributions side by side, of which a load read 24 bytes from each of 21 places (200 MB:
+// 6.2 TB/s).
 __global__ __launch_bounds__(256) void gatherR(const int32_t* __restrict__ ncptr, const uint8_t* __restrict__ fixed,
-                                               int maskDbc, const double* __restrict__ Rst, int64_t r0, int64_t r1,
-                                               double* __restrict__ R) {
+                                               int maskDbc, const double* __restrict__ Rst, int64_t tail, int64_t r0,
+                                               int64_t r1, double* __restrict__ R) {
   const int64_t d = r0 * 3 + (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (d >= r1 * 3) return;
-  if (maskDbc && fixed[d]) {
-    R[d] = 0.0;
-    return;
-  }
   const int64_t node = d / 3;
   const int k        = (int)(d - node * 3);
-  const int32_t c1   = ncptr[node + 1];
-  double acc         = 0.0;
-  for (int32_t c = ncptr[node]; c < c1; c += 8) {
-    double v[8];
+  const int32_t c0 = ncptr[node], n = ncptr[node + 1] - c0;
+  const double* src = Rst + residualSlot(node, 0) * 3 + k;
+  double v[kResidualRanks], acc = 0.0;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) v[j] = c + j < c1 ? Rst[(int64_t)(c + j) * 3 + k] : 0.0;
+  for (int j = 0; j < kResidualRanks; ++j) v[j] = j < n ? src[j * (64 * 3)] : 0.0;
 #pragma unroll
-    for (int j = 0; j < 8; ++j)
-      if (c + j < c1) acc += v[j];
-  }
-  R[d] = acc;
+  for (int j = 0; j < kResidualRanks; ++j)
+    if (j < n) acc += v[j];
+  for (int32_t j = kResidualRanks; j < n; ++j) acc += Rst[(tail + c0 + j) * 3 + k];
+  R[d] = maskDbc && fixed[d] ? 0.0 : acc;
 }
 
 __global__ void pointLoadKernel(const int64_t* __restrict__ dof, const double* __restrict__ coef, int64_t n,
@@ -784,8 +805,8 @@ inline unsigned gridFor(int64_t n, int bs) {
 template <typename T, int KIND, bool WR>
 void launchTiles(ik_handle* h, int64_t e0, int64_t count, T* Kebe, T* K, int mask) {
   const size_t lds = tangentLds<KIND>(h->maxAcc) + (size_t)h->maxGroups * kGroupTableBytes;
-  hipLaunchKernelGGL((hex8Tangent<KIND, T, WR, true>), dim3((unsigned)count), dim3(kTileThreads), lds, h->stream, h->X.p,
-                     h->u.p, h->conn.p, h->tileElem.p, h->tileNode.p, e0, count, h->lam, h->mu, (const int4*)h->tmeta.p,
+  hipLaunchKernelGGL((hex8Tangent<KIND, T, WR, true>), dim3((unsigned)count), dim3(kTileThreads), lds, h->stream,
+                     h->X.p, h->u.p, h->conn.p, h->tileElem.p, h->tileNode.p, e0, count, h->lam, h->mu, (const int4*)h->tmeta.p,
                      h->gdst.p, h->gpt.p, h->gmsk.p, h->epos.p, h->gmul.p, h->maxGroups, h->maxAcc, K, mask, h->rdest.p,
                      Kebe, h->ebeR.p, h->faceBits.p, loadedTraction(h), h->errFlag.p);
 }
@@ -795,7 +816,8 @@ void launchElements(ik_handle* h, int64_t e0, int64_t count, double* Kebe, doubl
   const unsigned grid = (unsigned)((count + kTileElems - 1) / kTileElems);
   hipLaunchKernelGGL((hex8Tangent<KIND, double, true, false>), dim3(grid), dim3(kTileThreads),
                      tangentLds<KIND>(kTileEntries), h->stream, h->X.p, h->u.p, h->conn.p, nullptr, nullptr, e0, count,
-                     h->lam, h->mu, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, 0, 0, (double*)nullptr, 0, nullptr,
+                     h->lam, h->mu, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, 0, 0, (double*)nullptr, 0,
+                     nullptr,
                      Kebe, Rebe, h->faceBits.p, loadedTraction(h), h->errFlag.p);
 }
 template <int KIND>
@@ -1141,7 +1163,7 @@ static void launchResidual(ik_handle* h, hipStream_t s) {
 }
 static void launchGatherR(ik_handle* h, int mask, int64_t r0, int64_t r1, hipStream_t s) {
   hipLaunchKernelGGL(gatherR, dim3((unsigned)(((r1 - r0) * 3 + 255) / 256)), dim3(256), 0, s, h->ncptr.p, h->fixed.p,
-                     mask, h->ebeR.p, r0, r1, h->R.p);
+                     mask, h->ebeR.p, residualTail(h->nn), r0, r1, h->R.p);
 }
 
 // Tangent assembly. Element chunks run on the main stream; each chunk's gathers run on the second stream,
@@ -1197,7 +1219,7 @@ static void runChunks(ik_handle* h, int dbc, bool wantR, bool fuseR, T* Kebe, T*
 
 void assembleKR(ik_handle* h, int dbc, int precision, bool wantK, bool wantR) {
   const int mask = dbc == IK_DBC_RAW ? 0 : 1;
-  h->ebeR.ensure((size_t)h->ne * 24);  // EAS elements always produce R_e
+  h->ebeR.ensure((size_t)h->rslots * 3);  // EAS elements always produce R_e
   if (h->neas) {
     // the EAS kernel computes the condensed R_e with K_e (in FP64; an FP32 matrix is gathered from the FP64
     // staging); both gathers run when K is wanted

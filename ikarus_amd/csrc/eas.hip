@@ -71,13 +71,6 @@ __device__ inline double readLane(double x, int lane) {
   return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
 }
 
-// 1/d by the hardware estimate and two Newton steps: within an ulp of the division, at a third of its instructions
-__device__ inline double reciprocal(double d) {
-  double r = __builtin_amdgcn_rcp(d);
-  r        = fma(fma(-d, r, 1.0), r, r);
-  return fma(fma(-d, r, 1.0), r, r);
-}
-
 // min(a, |b|); the compiler's fmin first quiets both operands, an instruction each
 __device__ inline double minAbs(double a, double b) {
   double m;

@@ -111,6 +111,15 @@ struct PcgScalars {
 
 enum KernelId { KASM_KR = 0, KASM_R = 1, KSPMV = 2, KMLP = 3, KGATHER = 4, KCOUNT = 5 };
 
+// Residual staging slots: in slices of 64 nodes, the incidence of rank j of all 64 side by side, so that elements along
+// a row of nodes write, and the gather's threads read, adjacent slots. Ranks that few nodes reach (more than 8 elements
+// around a node) lie behind all slices.
+constexpr int kResidualRanks = 8;
+__host__ __device__ constexpr int64_t residualSlot(int64_t node, int64_t rank) {
+  return (node >> 6) * (64 * kResidualRanks) + rank * 64 + (node & 63);
+}
+inline int64_t residualTail(int64_t nn) { return (nn + 63) / 64 * (64 * kResidualRanks); }
+
 // Reduction partials: one double per block, final fold in fixed order (deterministic).
 constexpr int kReduceBlocks = 1024;
 
@@ -206,11 +215,12 @@ struct ik_handle {
   //  << 20, accumulators | tmaxr << 16;
   //  tileNode[(16 t + s) 8 + q] = node of corner q of the element in slot s (padding: of slot 0).
   //  maxGroups, maxAcc = the largest numbers of groups and accumulators of a tile (they size the kernel's LDS).
-  // Residual staging: node by node, each node's (element, corner) incidences ordered by element;
-  // rdest[e*8+a] = slot, ncptr[n] = first slot of node n
+  // Residual staging: ncptr[n] = first (element, corner) incidence of node n, ordered by element; rdest[e*8+a] = slot
+  // of the incidence (residualSlot; ranks from kResidualRanks on at residualTail + incidence), rslots = number of slots
   ik::DevBuf<int32_t> bdest, segptr, ncptr, rdest;
   bool tiled = false;
   int64_t ntiles = 0, nstage = 0;  // tiles; staging slots of the tangent
+  int64_t rslots = 0;              // staging slots (3 doubles each) of the residual
   ik::DevBuf<int32_t> tileElem, tgptr, gdst, gpt;
   ik::DevBuf<uint16_t> epos, gmsk;
   ik::DevBuf<uint8_t> tmaxr;

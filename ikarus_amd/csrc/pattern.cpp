@@ -8,6 +8,7 @@
 // slot, and the maps from element blocks to staging slots in the gather order of their K blocks (per
 // element for EAS, per tile group for the plain element). The scalar CSC is re-derived from it on demand.
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstdlib>
 #include <thread>
@@ -447,7 +448,8 @@ void buildPattern(ik_handle* h) {
     std::vector<std::vector<int32_t>> gpart(chunkCount(ntiles, 256));
     std::vector<std::vector<uint32_t>> mpart(chunkCount(ntiles, 256));
     parallelChunks(ntiles, [&](int64_t t0, int64_t t1, int64_t ch) {
-      std::vector<int32_t> hkey(kHash), hval(kHash), touched, entQ(kTileEntries), cntQ(kTileEntries), accOf(kTileEntries);
+      std::vector<int32_t> hkey(kHash), hval(kHash), touched;
+      std::vector<int32_t> entQ(kTileEntries), cntQ(kTileEntries), accOf(kTileEntries);
       std::vector<int64_t> hstamp(kHash, -1);
       std::vector<uint16_t> entTr(kTileEntries);
       std::vector<int32_t>& out = gpart[ch];
@@ -735,11 +737,22 @@ void buildPattern(ik_handle* h) {
     for (int64_t i = 0; i < nn; ++i) dslot[i] = h->hpos[h->hdiag[i]];
     h->diagBlk.upload(dslot.data(), dslot.size(), h->stream);
   }
-  // residual staging slot of every element corner: its position in the node's incidence list
+  // residual staging slot of every element corner (residualSlot of its rank in the node's incidence list)
   HostVec<int32_t> rdest((size_t)ne * 8);
-  parallelChunks((int64_t)nlist.size(), [&](int64_t j0, int64_t j1, int64_t) {
-    for (int64_t j = j0; j < j1; ++j) rdest[nlist[j]] = (int32_t)j;
+  const int64_t tail = residualTail(nn);
+  std::atomic<bool> anyTail{false};
+  parallelChunks(nn, [&](int64_t i0, int64_t i1, int64_t) {
+    bool any = false;
+    for (int64_t i = i0; i < i1; ++i)
+      for (int64_t j = cnt[i]; j < cnt[i + 1]; ++j) {
+        const int64_t rank = j - cnt[i];
+        any |= rank >= kResidualRanks;
+        rdest[nlist[j]] = (int32_t)(rank < kResidualRanks ? residualSlot(i, rank) : tail + j);
+      }
+    if (any) anyTail = true;
   });
+  h->rslots = tail + (anyTail ? ne * 8 : 0);
+  require(h->rslots <= INT32_MAX, IK_EINVAL, "internal error: too many residual staging slots");
   h->ncptr.upload(ncnt.data(), ncnt.size(), h->stream);
   h->rdest.upload(rdest.data(), rdest.size(), h->stream);
   IK_HIP(hipStreamSynchronize(h->stream));

@@ -1,4 +1,4 @@
-// wave_reduce.hh — sums over the 64 lanes of a wavefront by DPP moves, and a wait for loads.
+// wave_reduce.hh — sums over the 64 lanes of a wavefront by DPP moves, a wait for loads, a short reciprocal.
 //
 // Shifts within rows of 16 lanes, then the row totals broadcast across rows; lane 63 ends with the total, read into a
 // scalar register. A shuffle-based tree goes through the LDS crossbar at every step: a double's six steps take about
@@ -51,6 +51,13 @@ template <typename T, int N>
 __device__ inline void arrived(T (&v)[N]) {
 #pragma unroll
   for (int i = 0; i < N; ++i) arrived(v[i]);
+}
+
+// 1/d by the hardware estimate and two Newton steps: within an ulp of the division, at a third of its instructions
+__device__ inline double reciprocal(double d) {
+  double r = __builtin_amdgcn_rcp(d);
+  r        = fma(fma(-d, r, 1.0), r, r);
+  return fma(fma(-d, r, 1.0), r, r);
 }
 
 }  // namespace ik
