@@ -18,17 +18,19 @@
 
 namespace ik {
 
-// elements per staging chunk; IKARUS_AMD_CHUNK_ELEMENTS overrides it. Splitting the 64^3 mesh into chunks
-// whose gathers overlap the next chunk's element work measured slower than one launch of each (the two
-// kernels contend for the same memory path), so the default takes meshes up to 1 M elements in one chunk.
-constexpr int64_t kChunkElements = 1 << 20;
+// elements per staging chunk; IKARUS_AMD_CHUNK_ELEMENTS overrides it. Plain element: splitting the 64^3 mesh into
+// chunks whose gathers overlap the next chunk's element work measured slower than one launch of each (the two kernels
+// contend for the same memory path), so the default takes meshes up to 1 M elements in one chunk. EAS: the element
+// kernel is bound by its arithmetic and leaves the memory to the gathers; 96 x 96 x 48 elements, assembly and update,
+// in chunks of 442,368 / 221,184 / 110,592 / 55,296 / 27,648 elements: 3,956 / 3,876 / 3,825 / 3,958 / 4,241 us.
+constexpr int64_t kChunkElements = 1 << 20, kChunkElementsEas = 1 << 17;
 
-static int64_t chunkElements() {
+static int64_t chunkElements(bool eas) {
   if (const char* v = std::getenv("IKARUS_AMD_CHUNK_ELEMENTS")) {
     const long long c = std::atoll(v);
     if (c >= 64) return (int64_t)c;
   }
-  return kChunkElements;
+  return eas ? kChunkElementsEas : kChunkElements;
 }
 
 // the low 21 bits of v spread to every third bit (bit i -> bit 3i)
@@ -343,7 +345,8 @@ void buildPattern(ik_handle* h) {
       for (int64_t k = cnt[i]; k < cnt[i + 1]; ++k) last[i] = std::max(last[i], unitOf[inc(k)]);
       if (i > 0) last[i] = std::max(last[i], last[i - 1]);
     }
-    const int64_t chunk = h->tiled ? (chunkElements() + kTileElems - 1) / kTileElems : chunkElements();
+    const int64_t chunk =
+        h->tiled ? (chunkElements(false) + kTileElems - 1) / kTileElems : chunkElements(h->neas > 0);
     h->chunkElem.assign(1, 0);
     h->chunkRow.assign(1, 0);
     int64_t r = 0;
