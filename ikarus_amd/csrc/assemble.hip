@@ -1169,10 +1169,9 @@ static void launchGatherR(ik_handle* h, int mask, int64_t r0, int64_t r1, hipStr
 // Tangent assembly. Element chunks run on the main stream; each chunk's gathers run on the second stream,
 // released by an event recorded behind the chunk, so the gathers of one chunk overlap the element work of
 // the next while its staged blocks are still cached. With one chunk the gather follows on the main stream.
-// wantR: the element kernel also stages R_e (EAS), gathered with K. fuseR: the residual pass of the plain
-// element follows the K gather on the main stream (run beside the gather on the second stream it slowed
-// both). In timing mode the chunks, the gathers and the residual pass run back to back on the main stream,
-// each group between one pair of events, giving stand-alone durations.
+// wantR: the element kernel also stages R_e (EAS), gathered with K chunk by chunk. fuseR: the plain element's tangent
+// kernel stages R_e too, gathered once behind all chunks. In timing mode the chunks and the gathers run back to back on
+// the main stream, each group between one pair of events, giving stand-alone durations.
 template <typename T>
 static void runChunks(ik_handle* h, int dbc, bool wantR, bool fuseR, T* Kebe, T* K) {
   const int mask = dbc == IK_DBC_RAW ? 0 : 1;
@@ -1225,9 +1224,7 @@ void assembleKR(ik_handle* h, int dbc, int precision, bool wantK, bool wantR) {
     // staging); both gathers run when K is wanted
     wantR = true;
   }
-  // EAS: one element pass yields K_e and R_e. Plain element: the register-bound tangent kernel and the
-  // residual kernel stay separate (R accumulated in the tangent kernel costs it more registers than the
-  // residual kernel takes time); with both wanted they share one launch sequence and one error check
+  // one element pass yields K_e and R_e; with both wanted, the plain element's tangent kernel forms R beside K
   const bool easBoth = h->neas && wantK;
   const bool fuseR   = !h->neas && wantK && wantR;
   if (wantK && precision == IK_FP64) {
