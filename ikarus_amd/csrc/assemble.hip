@@ -325,7 +325,7 @@ constexpr size_t kGroupTableBytes = 14;  // gdst, gpt, gmul, gmsk
 // alone 140 us. A tile's life is about 30,000 cycles, half of them the two rounds of loads and the point phase, so
 // tables are read in as few dependent rounds as possible. Persistent workgroups holding the next tile's loads in
 // registers spilled (405 us); mapping consecutive tiles to one XCD changed nothing.
-template <int KIND, typename TK, bool WANT_R, bool TILED>
+template <int KIND, typename TK, bool WANT_R, bool TILED, bool NT>
 __global__ __launch_bounds__(kTileThreads, KIND == IK_SVK ? 3 : 4) void hex8Tangent(
     const double* __restrict__ X, const double* __restrict__ U, const int32_t* __restrict__ conn,
     const int32_t* __restrict__ tileElem, const int32_t* __restrict__ tileNode, int64_t e0, int64_t count, double lam,
@@ -601,17 +601,21 @@ __global__ __launch_bounds__(kTileThreads, KIND == IK_SVK ? 3 : 4) void hex8Tang
     constexpr int kTeams = kTileThreads / 9;
     const int team = threadIdx.x / 9, tt = threadIdx.x % 9, k = tt / 3, l = tt - 3 * (tt / 3), tT = 3 * l + k;
     auto stage = [&](int d, double v) { Kebe[(int64_t)d * 9 + tt] = (TK)v; };
-    // complete K block: the FULL treatment as in the gather, then the block and its mirror, stored
-    // non-temporally (K is read back only by later passes, long after it has left the caches; the
-    // staged sums stay cached for the gather)
+    // complete K block: the FULL treatment as in the gather, then the block and its mirror, stored non-temporally if
+    // NT (see nonTemporalK; the staged sums always stay cached for the gather)
     auto direct = [&](int g, int2 d, double v) {
       if (maskDbc && d.y < 0) {
         const unsigned m = gm[g];
         if ((m >> tt) & 1u) v = (k == l && ((m >> (9 + k)) & 1u)) ? 1.0 : 0.0;
       }
       const int p = -d.x - 1, pt = d.y & INT32_MAX;
-      __builtin_nontemporal_store((TK)v, &K[(int64_t)p * 9 + tt]);
-      if (pt != p) __builtin_nontemporal_store((TK)v, &K[(int64_t)pt * 9 + tT]);
+      if constexpr (NT) {
+        __builtin_nontemporal_store((TK)v, &K[(int64_t)p * 9 + tt]);
+        if (pt != p) __builtin_nontemporal_store((TK)v, &K[(int64_t)pt * 9 + tT]);
+      } else {
+        K[(int64_t)p * 9 + tt] = (TK)v;
+        if (pt != p) K[(int64_t)pt * 9 + tT] = (TK)v;
+      }
     };
     // the larger groups first: their accumulators in entry order
     for (int m = team; m < nm; m += kTeams) {
@@ -802,23 +806,37 @@ inline unsigned gridFor(int64_t n, int bs) {
 }
 
 // tangent staging over tiles [e0, e0 + count), with the residual when WR
+// Whether the tangent kernel writes complete K blocks non-temporally. A K that fits the last-level cache (256 MB) is
+// written better through the caches, which put its 72-byte pieces together: Neo-Hooke FP64 in shuffled order, 48^3
+// elements, 278 us against 328. One somewhat larger would push out the staged sums that the gather reads next: 56^3 /
+// 64^3 in grid order 316 / 443 us non-temporally, 328 / 461 cached (shuffled 508 / 797 and 520 / 857). Far beyond it
+// the staging does not stay either: 68^3 / 72^3 / 80^3 / 96^3 in grid order 560 / 686 / 966 / 1,577 us non-temporally,
+// 562 / 664 / 901 / 1,477 cached. SVK, with more arithmetic per block, does not gain there (96^3: 1,604 and 1,634 us).
+template <int KIND>
+bool nonTemporalK(size_t bytes) {
+  return bytes > 256000000 && (KIND == IK_SVK || bytes <= 600000000);
+}
 template <typename T, int KIND, bool WR>
 void launchTiles(ik_handle* h, int64_t e0, int64_t count, T* Kebe, T* K, int mask) {
   const size_t lds = tangentLds<KIND>(h->maxAcc) + (size_t)h->maxGroups * kGroupTableBytes;
-  hipLaunchKernelGGL((hex8Tangent<KIND, T, WR, true>), dim3((unsigned)count), dim3(kTileThreads), lds, h->stream,
-                     h->X.p, h->u.p, h->conn.p, h->tileElem.p, h->tileNode.p, e0, count, h->lam, h->mu, (const int4*)h->tmeta.p,
-                     h->gdst.p, h->gpt.p, h->gmsk.p, h->epos.p, h->gmul.p, h->maxGroups, h->maxAcc, K, mask, h->rdest.p,
-                     Kebe, h->ebeR.p, h->faceBits.p, loadedTraction(h), h->errFlag.p);
+  auto launch = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3((unsigned)count), dim3(kTileThreads), lds, h->stream, h->X.p, h->u.p, h->conn.p,
+                       h->tileElem.p, h->tileNode.p, e0, count, h->lam, h->mu, (const int4*)h->tmeta.p, h->gdst.p,
+                       h->gpt.p, h->gmsk.p, h->epos.p, h->gmul.p, h->maxGroups, h->maxAcc, K, mask, h->rdest.p, Kebe,
+                       h->ebeR.p, h->faceBits.p, loadedTraction(h), h->errFlag.p);
+  };
+  if (nonTemporalK<KIND>((size_t)h->nsell * 9 * sizeof(T)))
+    launch(hex8Tangent<KIND, T, WR, true, true>);
+  else
+    launch(hex8Tangent<KIND, T, WR, true, false>);
 }
-// K_e and R_e of elements [e0, e0 + count) in element order
 template <int KIND>
 void launchElements(ik_handle* h, int64_t e0, int64_t count, double* Kebe, double* Rebe) {
   const unsigned grid = (unsigned)((count + kTileElems - 1) / kTileElems);
-  hipLaunchKernelGGL((hex8Tangent<KIND, double, true, false>), dim3(grid), dim3(kTileThreads),
+  hipLaunchKernelGGL((hex8Tangent<KIND, double, true, false, false>), dim3(grid), dim3(kTileThreads),
                      tangentLds<KIND>(kTileEntries), h->stream, h->X.p, h->u.p, h->conn.p, nullptr, nullptr, e0, count,
                      h->lam, h->mu, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, 0, 0, (double*)nullptr, 0,
-                     nullptr,
-                     Kebe, Rebe, h->faceBits.p, loadedTraction(h), h->errFlag.p);
+                     nullptr, Kebe, Rebe, h->faceBits.p, loadedTraction(h), h->errFlag.p);
 }
 template <int KIND>
 void launchResidualOnly(ik_handle* h, hipStream_t s) {
