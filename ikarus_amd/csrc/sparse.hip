@@ -733,12 +733,12 @@ static unsigned spmvGrid(int64_t nn) {
 static void ensureWork(ik_handle* h) {
   const int64_t spmvBlocks = std::max(spmvGrid<double>(h->nn), spmvGrid<float>(h->nn));
   h->partial.ensure((size_t)(2 * kReduceBlocks + spmvBlocks) + kPqBlocks + 8);
-  if (!h->sc.p) {
-    h->sc.ensure(1);
+  h->sc.ensure(1);
+  if (!h->pcg) {
     IK_HIP(hipHostMalloc((void**)&h->pcg, sizeof(PcgMirror), hipHostMallocCoherent));
     h->pcg->state = 0;
-    IK_HIP(hipHostMalloc((void**)&h->hred, sizeof(double) * 4, hipHostMallocDefault));
   }
+  if (!h->hred) IK_HIP(hipHostMalloc((void**)&h->hred, sizeof(double) * 4, hipHostMallocDefault));
 }
 
 // y = K x (partial: with x.y partials per block, and skipped once sc->done)
