@@ -484,24 +484,31 @@ __global__ __launch_bounds__(64, 2) void easElement(const double* __restrict__ X
     dmax = maxAbs(dmax, dppMove<0x142, 0xA>(dmax));
     dmax = maxAbs(dmax, dppMove<0x143, 0xC>(dmax));
     dmax = lane63(dmax);
+    // The diagonal blocks are inverted times a power of two that brings D's largest entry to about 1: D scales with
+    // mu h^-13 in the element's extent h, and the determinants with its square, which leaves the range of a double at
+    // extents where D does not (mu = 8e10: h of 1e-11; without the scaling such elements were called singular). Exact,
+    // so the results do not change: two multiplications per panel, the factor itself in scalar registers.
+    const int dexp     = (int)(__builtin_bit_cast(unsigned long long, dmax) >> 52);  // dmax >= 0
+    const double scale = __builtin_bit_cast(
+        double, (unsigned long long)(2046 - (dexp < 1 ? 1 : (dexp > 2045 ? 2045 : dexp))) << 52);
     // Pivots against the threshold, per 2 x 2 block its first entry and its determinant over that. One that is not
     // finite makes all later ones NaN (its reciprocal is), so the last one shows it.
-    const double limit = 1e-13 * dmax;
+    const double limit = 1e-13 * dmax, limitS = limit * scale;
     double least = INFINITY, gap = INFINITY;
     auto block2 = [&](double a, double b, double c) {  // 1 / determinant
       const double det = a * c - b * b;
       least            = minAbs(least, a);
-      gap              = minOf(gap, fma(-limit, fabs(a), fabs(det)));
+      gap              = minOf(gap, fma(-limitS, fabs(a), fabs(det)));
       return reciprocal(det);
     };
     double* cy = cache + e * kEasCache;
 #pragma unroll
     for (int p = 0; p < 5; ++p) {
       const double P0 = p < 4 ? t00[p & 3] : 0.0, P1 = p < 4 ? t01[p & 3] : t11[0], P2 = p < 4 ? t02[p & 3] : t12[0];
-      const double Pd = p < 4 ? P0 : P1;
+      const double Pd = (p < 4 ? P0 : P1) * scale;
       const int lc    = p < 4 ? 4 * p : 0;
       auto a = [&](int k, int l) { return readLane(Pd, 16 * k + lc + l); };
-      // D_pp = [A B; B^T C] by 2 x 2 blocks; x = column q of its inverse
+      // scale D_pp = [A B; B^T C] by 2 x 2 blocks; x = column q of its inverse
       const double a00 = a(0, 0), a01 = a(0, 1), a11 = a(1, 1);
       const double b00 = a(0, 2), b01 = a(0, 3), b10 = a(1, 2), b11 = a(1, 3);
       const double ra = block2(a00, a01, a11);
@@ -516,7 +523,7 @@ __global__ __launch_bounds__(64, 2) void easElement(const double* __restrict__ X
       const double x0 = i00 * unit[0] + i01 * unit[1] - (m00 * x2 + m01 * x3);
       const double x1 = i01 * unit[0] + i11 * unit[1] - (m10 * x2 + m11 * x3);
       asm("" : : "v"(x0), "v"(x1), "v"(x2), "v"(x3));  // all four before the selection: no branches around them
-      const double xr = (lane & 2) ? ((lane & 1) ? x3 : x2) : ((lane & 1) ? x1 : x0);
+      const double xr = ((lane & 2) ? ((lane & 1) ? x3 : x2) : ((lane & 1) ? x1 : x0)) * scale;
       const double W1 = __builtin_amdgcn_mfma_f64_4x4x4f64(xr, P1, 0.0, 0, 0, 0);
       const double W2 = __builtin_amdgcn_mfma_f64_4x4x4f64(xr, P2, 0.0, 0, 0, 0);
       if (p < 3) {
@@ -535,7 +542,7 @@ __global__ __launch_bounds__(64, 2) void easElement(const double* __restrict__ X
     }
     {  // row 20: register 1 of the tiles (1, J), lanes q = 0
       const double d20 = readLane(t11[1], 4), r20 = reciprocal(d20);
-      if (!(least > limit && gap > 0.0 && fabs(d20) > limit && fabs(d20) < INFINITY && dmax < INFINITY) && lane == 0)
+      if (!(least > limitS && gap > 0.0 && fabs(d20) > limit && fabs(d20) < INFINITY && dmax < INFINITY) && lane == 0)
         atomicMin(err + 1, (unsigned long long)e);
       const double P1 = q == 0 ? t11[1] : 0.0, P2 = q == 0 ? t12[1] : 0.0;
       const double W1 = P1 * r20, W2 = P2 * r20;
