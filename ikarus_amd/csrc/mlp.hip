@@ -502,7 +502,6 @@ inline unsigned g1(int64_t n) { return (unsigned)std::min<int64_t>(std::max<int6
 // ------------------------------------------------------------------------------------------------
 struct Mlp {
   hipStream_t s = nullptr;
-  int64_t maxBatch = 0;
   DevBuf<float> P, G, Mo, Vo;      // params (fp32 master), grads, Adam moments
   DevBuf<float> Aa[3], dZ[3], Y, dY, Xin, Tin;
   DevBuf<float> Gpart;  // per-slice partial gradients, folded in a fixed order
@@ -512,17 +511,22 @@ struct Mlp {
   int64_t step = 0;
   std::string err;
 
-  void ensure(int64_t n) {
-    if (n <= maxBatch) return;
-    maxBatch = n;
+  // Buffers of a batch of n rows, for the pass that uses them. Each one checks its own size, so one that could not be
+  // had is asked for again by the next call.
+  void ensureForward(int64_t n, bool host) {
+    Y.ensure(n * kOut);
+    if (host) Xin.ensure(n * kIn);
+  }
+  void ensureTraining(int64_t n, bool host) {
     for (int l = 0; l < 3; ++l) {
       Aa[l].ensure(n * kHid);
       dZ[l].ensure(n * kHid);
     }
-    Y.ensure(n * kOut);
     dY.ensure(n * kOut);
-    Xin.ensure(n * kIn);
-    Tin.ensure(n * kOut);
+    if (host) {
+      Xin.ensure(n * kIn);
+      Tin.ensure(n * kOut);
+    }
   }
 
   // y (n x 3) = the network on x (n x 14); nothing is kept and nothing is allocated
@@ -735,7 +739,7 @@ int ik_mlp_load(ik_mlp* m, const float* p, int where) {
 int ik_mlp_forward(ik_mlp* m, const float* x, int64_t n, float* y, int where) {
   return mguard(m, [&] {
     ik::require(n > 0, IK_EINVAL, "empty batch");
-    m->m->ensure(n);
+    m->m->ensureForward(n, where != IK_DEVICE);
     const float* xd = x;
     if (where != IK_DEVICE) {
       IK_HIP(hipMemcpyAsync(m->m->Xin.p, x, n * ik::kIn * sizeof(float), hipMemcpyHostToDevice, m->s));
@@ -767,7 +771,7 @@ int ik_mlp_forward_noalloc(ik_mlp* m, const float* x, int64_t n, float* y) {
 int ik_mlp_loss_grad(ik_mlp* m, const float* x, const float* t, int64_t n, double* loss, float* grad, int where) {
   return mguard(m, [&] {
     ik::require(n > 0, IK_EINVAL, "empty batch");
-    m->m->ensure(n);
+    m->m->ensureTraining(n, where != IK_DEVICE);
     const float *xd = x, *td = t;
     if (where != IK_DEVICE) {
       IK_HIP(hipMemcpyAsync(m->m->Xin.p, x, n * ik::kIn * sizeof(float), hipMemcpyHostToDevice, m->s));
@@ -788,7 +792,7 @@ int ik_mlp_loss_grad(ik_mlp* m, const float* x, const float* t, int64_t n, doubl
 int ik_mlp_train_step(ik_mlp* m, const float* x, const float* t, int64_t n, float lr, double* loss, int where) {
   return mguard(m, [&] {
     ik::require(n > 0, IK_EINVAL, "empty batch");
-    m->m->ensure(n);
+    m->m->ensureTraining(n, where != IK_DEVICE);
     const float *xd = x, *td = t;
     if (where != IK_DEVICE) {
       IK_HIP(hipMemcpyAsync(m->m->Xin.p, x, n * ik::kIn * sizeof(float), hipMemcpyHostToDevice, m->s));
