@@ -90,6 +90,7 @@ struct DevBuf {
 constexpr int kPcgPublish = 8;
 struct PcgMirror {
   double rr, bb;             // valid once done
+  unsigned long long err[2]; // the element kernels' error flag at the start of the run; valid with its first state
   unsigned long long state;  // run << 32 | iterations << 2 | done
 };
 

@@ -1,0 +1,30 @@
+// pcg_wait.hh — the host's side of a PCG run's progress in pinned memory: what a look at it says, and the wait for more.
+#pragma once
+#include <cstdint>
+
+#include "ik_internal.hh"
+
+namespace ik {
+
+// Whether run `run` has started, as the device's last store to the mirror says; then `state` is iterations << 2 | done
+// and `flagged` whether the element kernels ahead of the run found an invalid element. The device stores the flags
+// behind a fence before the run's first state, so they are there with any state of the run. (A copy of the flag enqueued
+// ahead of the run is not: only a synchronisation of its stream makes its target readable.)
+inline bool pcgLook(const PcgMirror& m, uint32_t run, unsigned& state, bool& flagged) {
+  const unsigned long long s = __atomic_load_n(&m.state, __ATOMIC_ACQUIRE);
+  if ((uint32_t)(s >> 32) != run) return false;
+  state   = (unsigned)s;
+  flagged = m.err[0] != ~0ull || m.err[1] != ~0ull;
+  return true;
+}
+
+// Looks until look() says true, with check() now and then for what would make it wait without end
+template <class Look, class Check>
+void pcgSpin(Look look, Check check) {
+  for (unsigned spin = 1; !look(); ++spin) {
+    if (spin % 4096 == 0) check();
+    __builtin_ia32_pause();
+  }
+}
+
+}  // namespace ik

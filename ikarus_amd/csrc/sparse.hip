@@ -10,6 +10,7 @@
 // iterations ahead of the test: the iterate after convergence is exactly the one Eigen's loop returns.
 #include "ik_internal.hh"
 #include "pcg_record.hh"
+#include "pcg_wait.hh"
 #include "wave_reduce.hh"
 
 namespace ik {
@@ -422,7 +423,8 @@ __global__ __launch_bounds__(256) void pcgInitKernel(const double* __restrict__ 
 }
 
 __global__ __launch_bounds__(1024) void pcgInitFold(const double* __restrict__ partial, int nb, double tol2,
-                                                    PcgScalars* __restrict__ sc, PcgMirror* mirror, uint32_t run) {
+                                                    PcgScalars* __restrict__ sc, PcgMirror* mirror, uint32_t run,
+                                                    const unsigned long long* __restrict__ err) {
   double rr = 0.0, rz = 0.0;
   for (int i = threadIdx.x; i < nb; i += 1024) {
     rr += partial[i];
@@ -443,6 +445,9 @@ __global__ __launch_bounds__(1024) void pcgInitFold(const double* __restrict__ p
     sc->alpha = sc->beta = 0.0;
     sc->mirror           = mirror;
     sc->run              = run;
+    mirror->err[0]       = err[0];
+    mirror->err[1]       = err[1];
+    __threadfence_system();
     pcgPublish(sc, rr, 0, sc->done);
   }
 }
@@ -797,31 +802,36 @@ void axpy(ik_handle* h, double a, const double* x, double* y, int64_t n) {
 constexpr int kPcgAhead = 12;
 static_assert(kPcgAhead > kPcgPublish + 1, "the device publishes within what may be enqueued");
 
-// State of the current PCG run (iterations << 2 | done); `before` until the run has started
+// State of the current PCG run (iterations << 2 | done); `before` until the run has started. An assembly whose error
+// flag is still to be read (errPending) is settled by the flag the run reports: if it is raised, here.
 static unsigned pcgState(ik_handle* h, unsigned before) {
-  const unsigned long long s = __atomic_load_n(&h->pcg->state, __ATOMIC_ACQUIRE);
-  if ((uint32_t)(s >> 32) != h->pcgRun) return before;
-  finishErrCheck(h);  // the element kernels' flags were copied ahead of this run
-  return (unsigned)s;
+  unsigned state = before;
+  bool flagged   = false;
+  if (!pcgLook(*h->pcg, h->pcgRun, state, flagged)) return before;
+  if (flagged) finishErrCheck(h, true);
+  h->errPending = false;
+  return state;
 }
 
 // waits for a state after `before`
 static unsigned pcgWait(ik_handle* h, unsigned before) {
-  bool idle = false;
-  for (unsigned spin = 1;; ++spin) {
-    const unsigned s = pcgState(h, before);
-    if (s != before) return s;
-    if (idle) throw Error{IK_EHIP, "internal error: the PCG run ended without a result"};
-    if (spin % 4096 == 0) {  // a launch or device that failed: an error here, not a wait without end
-      const hipError_t query = hipStreamQuery(h->stream);
-      idle                   = query == hipSuccess;
-      if (query == hipErrorNotReady)
-        (void)hipGetLastError();
-      else
-        IK_HIP(query);
-    }
-    __builtin_ia32_pause();
-  }
+  bool idle      = false;
+  unsigned state = before;
+  pcgSpin(
+      [&] {
+        state = pcgState(h, before);
+        if (state == before && idle) throw Error{IK_EHIP, "internal error: the PCG run ended without a result"};
+        return state != before;
+      },
+      [&] {  // a launch or device that failed: an error here, not a wait without end
+        const hipError_t query = hipStreamQuery(h->stream);
+        idle                   = query == hipSuccess;
+        if (query == hipErrorNotReady)
+          (void)hipGetLastError();
+        else
+          IK_HIP(query);
+      });
+  return state;
 }
 
 // The iterations of one PCG solve, after its init kernels: enqueued until the done flag or maxIter. p holds
@@ -888,7 +898,7 @@ void pcgJacobi64(ik_handle* h, const double* b, double* x, double rtol, int maxI
   hipLaunchKernelGGL(pcgInitKernel, dim3(g), dim3(256), 0, h->stream, b, h->pdiag.p, x, h->pr.p, h->pp.p, z, n,
                      h->partial.p);
   hipLaunchKernelGGL(pcgInitFold, dim3(1), dim3(1024), 0, h->stream, h->partial.p, g, rtol * rtol, h->sc.p,
-                     h->pcg, ++h->pcgRun);
+                     h->pcg, ++h->pcgRun, h->errFlag.p);
   if (maxIter <= 0) maxIter = (int)(2 * n);
   pcgLoop<double>(h, h->K64.p, x, h->pr.p, h->pp.p, h->pb.p, z, h->pq.p, h->pdiag.p, n, g, maxIter, false);
   *iters  = (int)((unsigned)h->pcg->state >> 2);
@@ -948,7 +958,7 @@ void pcgMixed(ik_handle* h, const double* b, double* x, const ik_solver_opts* o,
                          h->fr.p, h->fp.p, z, h->nn, h->partial.p);
     }
     hipLaunchKernelGGL(pcgInitFold, dim3(1), dim3(1024), 0, h->stream, h->partial.p, gn, innerTol * innerTol,
-                       h->sc.p, h->pcg, ++h->pcgRun);
+                       h->sc.p, h->pcg, ++h->pcgRun, h->errFlag.p);
     pcgLoop<float>(h, h->K32.p, h->fx.p, h->fr.p, h->fp.p, h->fp2.p, z, h->fq.p, h->fdiag.p, n, gn, maxIter, twoLevel);
     info->iterations += (int)((unsigned)h->pcg->state >> 2) + 1;
     info->refinements += 1;
