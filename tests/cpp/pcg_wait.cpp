@@ -1,7 +1,13 @@
 // pcg_wait.cpp — the host's side of a PCG run's progress (ikarus_amd/csrc/pcg_wait.hh) on the CPU: a plain struct stands
 // for the pinned mirror, threads for the device and for other solves.
+#include <pthread.h>
+#include <sched.h>
+
+#include <atomic>
+#include <chrono>
 #include <cstdio>
 #include <cstring>
+#include <thread>
 
 #include "../../ikarus_amd/csrc/pcg_wait.hh"
 
@@ -40,10 +46,50 @@ void flags() {
     }
 }
 
+// two waiting threads on one core hand a token to and fro: with a wait that keeps the core each of the 400 hand-overs
+// takes a time slice of the scheduler (a millisecond at least, 0.4 s in all), with one that gives it up microseconds
+void sharing() {
+  cpu_set_t one;
+  sched_getaffinity(0, sizeof(one), &one);
+  int cpu = 0;
+  while (!CPU_ISSET(cpu, &one)) ++cpu;
+  CPU_ZERO(&one);
+  CPU_SET(cpu, &one);
+  std::atomic<int> token{0};
+  int checks  = 0;
+  auto player = [&](int me) {
+    pthread_setaffinity_np(pthread_self(), sizeof(one), &one);
+    for (int turn = me; turn < 400; turn += 2) {
+      ik::pcgSpin([&] { return token.load() == turn; }, [] {});
+      token.store(turn + 1);
+    }
+  };
+  const auto t0 = std::chrono::steady_clock::now();
+  std::thread a(player, 0), b(player, 1);
+  a.join();
+  b.join();
+  const double s = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
+  std::printf("400 hand-overs on one core: %.4f s\n", s);
+  expect(token.load() == 400 && s < 0.2, "threads waiting on one core keep it from each other");
+}
+
+// the check for a wait without end is called while nothing arrives, and what it throws ends the wait
+void failure() {
+  int checks = 0;
+  try {
+    ik::pcgSpin([] { return false; }, [&] { if (++checks == 3) throw 1; });
+    expect(false, "the wait ended by itself");
+  } catch (int) {
+    expect(checks == 3, "check");
+  }
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
   if (argc > 1 && !std::strcmp(argv[1], "flags")) flags();
+  if (argc > 1 && !std::strcmp(argv[1], "sharing")) sharing();
+  if (argc > 1 && !std::strcmp(argv[1], "failure")) failure();
   std::printf(bad ? "FAILED\n" : "OK\n");
   return bad ? 1 : 0;
 }

@@ -16,3 +16,12 @@ def _run(tmp_path, what):
 def test_an_invalid_element_is_known_with_the_first_state(tmp_path):
     """The flag comes with the run's state, not from a copy that only a synchronisation makes readable."""
     _run(tmp_path, "flags")
+
+
+def test_waits_share_a_core(tmp_path):
+    """Threads that wait for their runs on one core give it to each other."""
+    _run(tmp_path, "sharing")
+
+
+def test_a_failed_run_ends_the_wait(tmp_path):
+    _run(tmp_path, "failure")
