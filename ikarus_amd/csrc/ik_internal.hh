@@ -222,9 +222,10 @@ struct ik_handle {
   bool tiled = false;
   int64_t ntiles = 0, nstage = 0;  // tiles; staging slots of the tangent
   int64_t rslots = 0;              // staging slots (3 doubles each) of the residual
-  ik::DevBuf<int32_t> tileElem, tgptr, gdst, gpt;
+  ik::DevBuf<int32_t> tileElem, gdst, gpt;
   ik::DevBuf<uint16_t> epos, gmsk;
-  ik::DevBuf<uint8_t> tmaxr;
+  std::vector<int32_t> tgptr;  // on the host: tmeta carries them to the kernel
+  std::vector<uint8_t> tmaxr;
   ik::DevBuf<int32_t> tmeta, tileNode;
   ik::DevBuf<uint32_t> gmul;
   int maxGroups = 0, maxAcc = 0;

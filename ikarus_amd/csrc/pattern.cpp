@@ -671,7 +671,6 @@ void buildPattern(ik_handle* h) {
     }
     h->ntiles = ntiles;
     h->tileElem.upload(tileElem.data(), tileElem.size(), h->stream);
-    h->tgptr.upload(tgptr.data(), tgptr.size(), h->stream);
     h->gdst.upload(gdst.data(), gdst.size(), h->stream);
     h->gpt.upload(gpt.data(), gpt.size(), h->stream);
     h->gmsk.upload(gmsk.data(), gmsk.size(), h->stream);
@@ -696,7 +695,8 @@ void buildPattern(ik_handle* h) {
     h->tmeta.upload(tmeta.data(), tmeta.size(), h->stream);
     h->tileNode.upload(tileNode.data(), tileNode.size(), h->stream);
     h->gmul.upload(gmul.data(), gmul.size(), h->stream);
-    h->tmaxr.upload(tmaxr.data(), tmaxr.size(), h->stream);
+    h->tgptr = std::move(tgptr);
+    h->tmaxr = std::move(tmaxr);
     h->maxGroups = maxGroups;
     h->maxAcc    = maxAcc;
   }

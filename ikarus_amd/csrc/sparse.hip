@@ -248,7 +248,7 @@ __global__ __launch_bounds__(SPMV_BS) void pcgDirectionSpmv(
   if (test) t.fetch(partial, nb, sc);
   double bt        = sc->beta;
   constexpr int NO = sizeof(TV) == 4 ? 3 : 1;  // outputs per lane
-  constexpr int DEPTH = 27 / G + 1 < 4 ? 27 / G + 1 : 4;
+  constexpr int DEPTH = 4;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, g = wave % G;
   const int rl      = sizeof(TV) == 4 ? lane : lane / 3;
   const int k       = sizeof(TV) == 4 ? 0 : lane - 3 * rl;
