@@ -21,16 +21,24 @@ namespace ik {
 // elements per staging chunk; IKARUS_AMD_CHUNK_ELEMENTS overrides it. Plain element: splitting the 64^3 mesh into
 // chunks whose gathers overlap the next chunk's element work measured slower than one launch of each (the two kernels
 // contend for the same memory path), so the default takes meshes up to 1 M elements in one chunk. EAS: the element
-// kernel is bound by its arithmetic and leaves the memory to the gathers; 96 x 96 x 48 elements, assembly and update,
-// in chunks of 442,368 / 221,184 / 110,592 / 55,296 / 27,648 elements: 3,956 / 3,876 / 3,825 / 3,958 / 4,241 us.
+// kernel is bound by its arithmetic and leaves the memory to the gathers, so the mesh is cut into equal chunks of about
+// kChunkElementsEas (a short last chunk leaves SIMDs idle), unless the numbering completes few rows before the last
+// chunk, which leaves nothing to overlap. Assembly and update, us, in one chunk / chunks of 131,072 and a rest / by
+// this rule, Neo-Hooke:
+//  grid order    141,987 elements 1,382 / 1,444 / 1,378, 198,476: 1,877 / 1,875 / 1,863, 238,328: 2,216 / 2,190 /
+//                2,196, 287,496: 2,645 / 2,606 / 2,604, 373,248: 3,387 / 3,307 / 3,308, 442,368: 3,986 / 3,879 /
+//                3,877, 806,400: 7,089 / 6,924 / 6,898
+//  random order  198,476: 1,990 / 2,033 / 1,991, 238,328: 2,350 / 2,399 / 2,349, 442,368: 4,324 / 4,401 / 4,329
+//  442,368 in grid order in chunks of 262,144 / 196,608 / 131,072 / 98,304 / 65,536: 4,040 / 3,891 / 3,862 / 3,879 /
+//                3,932
 constexpr int64_t kChunkElements = 1 << 20, kChunkElementsEas = 1 << 17;
 
-static int64_t chunkElements(bool eas) {
+static int64_t chunkOverride() {
   if (const char* v = std::getenv("IKARUS_AMD_CHUNK_ELEMENTS")) {
     const long long c = std::atoll(v);
     if (c >= 64) return (int64_t)c;
   }
-  return eas ? kChunkElementsEas : kChunkElements;
+  return 0;
 }
 
 // the low 21 bits of v spread to every third bit (bit i -> bit 3i)
@@ -345,19 +353,30 @@ void buildPattern(ik_handle* h) {
       for (int64_t k = cnt[i]; k < cnt[i + 1]; ++k) last[i] = std::max(last[i], unitOf[inc(k)]);
       if (i > 0) last[i] = std::max(last[i], last[i - 1]);
     }
-    const int64_t chunk =
-        h->tiled ? (chunkElements(false) + kTileElems - 1) / kTileElems : chunkElements(h->neas > 0);
-    h->chunkElem.assign(1, 0);
-    h->chunkRow.assign(1, 0);
-    int64_t r = 0;
-    for (int64_t u0 = 0; u0 < nunits; u0 += chunk) {
-      const int64_t u1 = std::min(nunits, u0 + chunk);
-      if (u1 == nunits)
-        r = nn;
-      else
-        while (r < nn && last[r] < u1) ++r;
-      h->chunkElem.push_back(u1);
-      h->chunkRow.push_back(r);
+    auto cut = [&](int64_t chunk) {
+      h->chunkElem.assign(1, 0);
+      h->chunkRow.assign(1, 0);
+      int64_t r = 0;
+      for (int64_t u0 = 0; u0 < nunits; u0 += chunk) {
+        const int64_t u1 = std::min(nunits, u0 + chunk);
+        if (u1 == nunits)
+          r = nn;
+        else
+          while (r < nn && last[r] < u1) ++r;
+        h->chunkElem.push_back(u1);
+        h->chunkRow.push_back(r);
+      }
+    };
+    const int64_t given = chunkOverride();
+    if (h->tiled) {
+      cut(((given ? given : kChunkElements) + kTileElems - 1) / kTileElems);
+    } else if (given) {
+      cut(given);
+    } else {
+      const int64_t nc = std::max<int64_t>(1, (ne + kChunkElementsEas / 2) / kChunkElementsEas);
+      cut((ne + nc - 1) / nc);
+      // in grid order the share of rows complete before the last chunk is close to (nc - 1) / nc, in random order to 0
+      if (nc > 1 && h->chunkRow[nc - 1] * 2 * nc < nn * (nc - 1)) cut(ne);
     }
   }
   const int64_t nchunks = (int64_t)h->chunkElem.size() - 1;

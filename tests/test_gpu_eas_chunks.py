@@ -1,6 +1,7 @@
-"""The EAS tangent where a wavefront takes four elements and the last one fewer, and where a mesh is staged in chunks that
-take different numbers of elements per wavefront (4, 2 or 1 by the size of the launch): each element's values must not
-depend on it, since a Newton solve mixes R of the R+K pass over chunks with R of the residual-only pass over the mesh."""
+"""The EAS tangent where a wavefront takes four elements and the last one fewer, and where a mesh is staged in chunks
+that take different numbers of elements per wavefront (4, 2 or 1 by the size of the launch): each element's values must
+not depend on it, since a Newton solve mixes R of the R+K pass over chunks with R of the residual-only pass over the
+mesh."""
 import numpy as np
 import pytest
 
@@ -74,9 +75,9 @@ def test_chunks_of_different_kinds(monkeypatch, nel, chunk, material):
 
 
 def test_default_chunks():
-    """More elements than one default chunk (131,072) holds: gathers beside the next chunk's elements, in both matrix
-    precisions; R of the R+K pass and of the residual-only pass, and the FP32 matrix as the FP64 one rounded."""
-    nel = (53, 51, 50)  # 135,150
+    """A mesh that is cut into chunks by default (two of 100,949 elements): gathers beside the next chunk's elements, in
+    both matrix precisions; R of the R+K pass and of the residual-only pass; the FP32 matrix as the FP64 one rounded."""
+    nel = (59, 58, 59)  # 201,898
     print(f"case: eas default chunks nel={nel}", flush=True)
     p, u, alpha, du = _state(nel, capi.NEOHOOKE)
     K, R, after, Ronly, afterOnly = _run(p, u, alpha, du)
