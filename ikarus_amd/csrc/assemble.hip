@@ -806,16 +806,6 @@ inline unsigned gridFor(int64_t n, int bs) {
 }
 
 // tangent staging over tiles [e0, e0 + count), with the residual when WR
-// Whether the tangent kernel writes complete K blocks non-temporally. A K that fits the last-level cache (256 MB) is
-// written better through the caches, which put its 72-byte pieces together: Neo-Hooke FP64 in shuffled order, 48^3
-// elements, 278 us against 328. One somewhat larger would push out the staged sums that the gather reads next: 56^3 /
-// 64^3 in grid order 316 / 443 us non-temporally, 328 / 461 cached (shuffled 508 / 797 and 520 / 857). Far beyond it
-// the staging does not stay either: 68^3 / 72^3 / 80^3 / 96^3 in grid order 560 / 686 / 966 / 1,577 us non-temporally,
-// 562 / 664 / 901 / 1,477 cached. SVK, with more arithmetic per block, does not gain there (96^3: 1,604 and 1,634 us).
-template <int KIND>
-bool nonTemporalK(size_t bytes) {
-  return bytes > 256000000 && (KIND == IK_SVK || bytes <= 600000000);
-}
 template <typename T, int KIND, bool WR>
 void launchTiles(ik_handle* h, int64_t e0, int64_t count, T* Kebe, T* K, int mask) {
   const size_t lds = tangentLds<KIND>(h->maxAcc) + (size_t)h->maxGroups * kGroupTableBytes;
@@ -825,11 +815,12 @@ void launchTiles(ik_handle* h, int64_t e0, int64_t count, T* Kebe, T* K, int mas
                        h->gpt.p, h->gmsk.p, h->epos.p, h->gmul.p, h->maxGroups, h->maxAcc, K, mask, h->rdest.p, Kebe,
                        h->ebeR.p, h->faceBits.p, loadedTraction(h), h->errFlag.p);
   };
-  if (nonTemporalK<KIND>((size_t)h->nsell * 9 * sizeof(T)))
+  if (nonTemporalK(KIND, (size_t)h->nsell * 9 * sizeof(T), h->adjacent))
     launch(hex8Tangent<KIND, T, WR, true, true>);
   else
     launch(hex8Tangent<KIND, T, WR, true, false>);
 }
+// K_e and R_e of elements [e0, e0 + count) in element order
 template <int KIND>
 void launchElements(ik_handle* h, int64_t e0, int64_t count, double* Kebe, double* Rebe) {
   const unsigned grid = (unsigned)((count + kTileElems - 1) / kTileElems);

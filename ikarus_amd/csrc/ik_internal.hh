@@ -121,6 +121,31 @@ __host__ __device__ constexpr int64_t residualSlot(int64_t node, int64_t rank) {
 }
 inline int64_t residualTail(int64_t nn) { return (nn + 63) / 64 * (64 * kResidualRanks); }
 
+// Whether the tangent kernel writes complete K blocks of a K of `bytes` non-temporally; `adjacent` as in ik_handle. A
+// K about as large as the last-level cache (256 MB) is written as well or better through the caches, which put its
+// 72-byte pieces together; a larger one written that way pushes out the staged sums that the gather reads next. Far
+// beyond it the staging does not stay either, and with Neo-Hooke, which has less arithmetic per block to hide the stores
+// behind, the putting together counts again, if there is something to put together: in a scattered numbering the pieces
+// of a tile have no neighbours. Assembly, us, non-temporally / through the caches:
+//  grid order (adjacent 0.6-0.7)
+//   NH FP64   174 MB 193 / 180, 225: 223 / 223, 284: 275 / 275, 354: 319 / 336, 526: 457 / 471, 629: 572 / 566, 745:
+//             697 / 671, 1,019: 976 / 908, 1,754: 1,573 / 1,483
+//   NH FP32   177 MB 276 / 281, 239: 359 / 368, 263: 389 / 394, 315: 469 / 466, 510: 727 / 720, 677: 931 / 916
+//   SVK FP64  174 MB 204 / 205, 225: 247 / 255, 354: 363 / 378, 526: 518 / 530, 745: 726 / 729, 1,754: 1,608 / 1,631
+//   SVK FP32  177 MB 331 / 334, 263: 470 / 475, 315: 562 / 559, 510: 876 / 862, 877: 1,436 / 1,433
+//  nodes in random order (adjacent 0)
+//   NH FP64   229 MB 332 / 283, 290: 413 / 387, 360: 515 / 527, 534: 801 / 865, 756: 1,218 / 1,296, 1,033: 1,741 /
+//             1,832
+//   NH FP32   180 MB 412 / 358, 267: 605 / 578, 319: 739 / 751, 517: 1,346 / 1,376, 685: 1,878 / 1,916
+//   SVK FP64  229 MB 346 / 307, 290: 421 / 389, 360: 527 / 531, 534: 808 / 869, 1,033: 1,751 / 1,830
+//   SVK FP32  180 MB 424 / 406, 267: 615 / 594, 319: 744 / 744, 517: 1,356 / 1,371, 685: 1,889 / 1,915
+//  nodes in random order by runs of 2 / 4 / 8 of the grid order (adjacent 0.19 / 0.33 / 0.44), NH FP64
+//   290 MB 392 / 362, 364 / 335, 347 / 320; 756 MB 1,159 / 1,180, 1,079 / 1,071, 942 / 912
+inline bool nonTemporalK(int material, size_t bytes, double adjacent) {
+  if (adjacent < 0.25) return bytes > 300000000;
+  return bytes > 256000000 && (material == IK_SVK || bytes <= 600000000);
+}
+
 // Reduction partials: one double per block, final fold in fixed order (deterministic).
 constexpr int kReduceBlocks = 1024;
 
@@ -229,6 +254,7 @@ struct ik_handle {
   ik::DevBuf<int32_t> tmeta, tileNode;
   ik::DevBuf<uint32_t> gmul;
   int maxGroups = 0, maxAcc = 0;
+  double adjacent = 0.0;  // share of the direct groups whose K slot follows that of the tile's previous direct group
   // staging chunks (tiles when tiled, elements otherwise) and the block rows complete after each chunk
   std::vector<int64_t> chunkElem, chunkRow;
   // element-by-element staging of K_e (36 upper 3x3 blocks) and R_e (24)

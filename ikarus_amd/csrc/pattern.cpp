@@ -695,8 +695,16 @@ void buildPattern(ik_handle* h) {
     h->gmsk.upload(gmsk.data(), gmsk.size(), h->stream);
     h->epos.upload(epos.data(), epos.size(), h->stream);
     HostVec<int32_t> tmeta(ntiles * 4), tileNode(ntiles * kTileElems * 8);
+    std::atomic<int64_t> direct{0}, adjacent{0};
     parallelChunks(ntiles, [&](int64_t t0, int64_t t1, int64_t) {
+      int64_t nd = 0, na = 0;
       for (int64_t t = t0; t < t1; ++t) {
+        for (int32_t g = tgptr[t], at = 1; g < tgptr[t + 1]; ++g)
+          if (gdst[g] < 0) {  // -(slot + 1)
+            ++nd;
+            na += gdst[g] + 1 == at;
+            at = gdst[g];
+          }
         const int32_t ng = tgptr[t + 1] - tgptr[t], nm = tmptr[t + 1] - tmptr[t];
         const uint32_t m = nm ? gmul[tmptr[t + 1] - 1] : (uint32_t)ng;  // the last accumulators
         tmeta[4 * t]     = tgptr[t];
@@ -710,7 +718,10 @@ void buildPattern(ik_handle* h) {
                       &tileNode[(t * kTileElems + s) * 8]);
         }
       }
+      direct += nd;
+      adjacent += na;
     });
+    h->adjacent = direct ? (double)adjacent / (double)direct : 0.0;
     h->tmeta.upload(tmeta.data(), tmeta.size(), h->stream);
     h->tileNode.upload(tileNode.data(), tileNode.size(), h->stream);
     h->gmul.upload(gmul.data(), gmul.size(), h->stream);

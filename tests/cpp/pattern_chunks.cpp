@@ -1,5 +1,5 @@
-// pattern_chunks.cpp — the staging chunks of the pattern build (ikarus_amd/csrc/pattern.cpp) on the CPU, with test
-// doubles in host memory for its calls into the HIP runtime.
+// pattern_chunks.cpp — what the pattern build (ikarus_amd/csrc/pattern.cpp) decides by the numbering of a mesh: staging
+// chunks and the stores of K, on the CPU, with test doubles in host memory for its calls into the HIP runtime.
 #include <algorithm>
 #include <cstdio>
 #include <cstdlib>
@@ -70,9 +70,53 @@ void check(const char* name, int n0, int n1, int n2, bool shuffled, const std::v
   bad += !ok;
 }
 
+// the share of a tile's complete blocks that follow each other in K, in grid order and with nodes in random order (the
+// numbering of the elements does not matter), and how K is then stored
+void checkStores(const char* name, bool shuffledNodes, double lo, double hi) {
+  ik_handle h;
+  const int n = 20, v = n + 1;
+  h.nn        = (int64_t)v * v * v;
+  h.ne        = (int64_t)n * n * n;
+  h.ndof      = h.nn * 3;
+  std::vector<int32_t> node(h.nn), elem(h.ne);
+  for (size_t i = 0; i < node.size(); ++i) node[i] = (int32_t)i;
+  for (size_t i = 0; i < elem.size(); ++i) elem[i] = (int32_t)i;
+  std::mt19937 rng(3);
+  if (shuffledNodes) std::shuffle(node.begin(), node.end(), rng);
+  std::shuffle(elem.begin(), elem.end(), rng);
+  h.hX.resize(h.nn * 3);
+  h.hfixed.assign(h.nn * 3, 0);
+  h.hconn.resize(h.ne * 8);
+  for (int64_t i = 0; i < h.nn; ++i) {
+    const int64_t x[3] = {i % v, i / v % v, i / v / v};
+    for (int d = 0; d < 3; ++d) h.hX[node[i] * 3 + d] = (double)x[d];
+  }
+  for (int64_t e = 0; e < h.ne; ++e) {
+    const int64_t i = elem[e] % n, j = elem[e] / n % n, k = elem[e] / n / n;
+    for (int a = 0; a < 8; ++a)
+      h.hconn[e * 8 + a] = node[(i + (a & 1)) + v * ((j + ((a >> 1) & 1)) + v * (k + ((a >> 2) & 1)))];
+  }
+  ik::buildPattern(&h);
+  bool ok = h.adjacent >= lo && h.adjacent <= hi;
+  for (int kind : {IK_NEOHOOKE, IK_SVK}) {
+    const size_t MB = 1000000;
+    ok &= !ik::nonTemporalK(kind, 200 * MB, h.adjacent) && ik::nonTemporalK(kind, 500 * MB, h.adjacent);
+    // beyond 600 MB a Neo-Hooke K goes through the caches where its blocks follow each other
+    ok &= ik::nonTemporalK(kind, 800 * MB, h.adjacent) == (kind == IK_SVK || shuffledNodes);
+  }
+  std::printf("%s: adjacent %.3f%s\n", name, h.adjacent, ok ? "" : " FAILED");
+  bad += !ok;
+}
+
 }  // namespace
 
-int main() {
+int main(int argc, char** argv) {
+  if (argc > 1 && !std::strcmp(argv[1], "stores")) {
+    checkStores("grid", false, 0.5, 0.8);
+    checkStores("random", true, 0.0, 0.05);
+    std::printf(bad ? "FAILED\n" : "OK\n");
+    return bad ? 1 : 0;
+  }
   unsetenv("IKARUS_AMD_CHUNK_ELEMENTS");
   check("141,987 grid", 57, 53, 47, false, {141987}, 0.0);
   check("201,898 grid", 59, 58, 59, false, {100949, 100949}, 0.45);
