@@ -754,7 +754,7 @@ int ik_assemble(ik_handle* h, int dbc, int precision, double* R, int where) {
     require(precision == IK_FP64 || precision == IK_FP32, IK_EINVAL, "bad precision");
     ensurePattern(h);
     const int d = dbc == IK_DBC_FULL ? IK_DBC_FULL : IK_DBC_RAW;
-    // FP64: one element pass produces K_e and R_e; FP32: the FP32 tangent and the FP64 residual are two passes
+    // one element pass produces K_e and R_e (in FP64; an FP32 matrix is rounded when its blocks are stored)
     ik::assembleKR(h, d, precision, true, true);
     h->kPrecision = precision;
     h->kDbc       = dbc;

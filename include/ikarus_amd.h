@@ -317,7 +317,10 @@ int ik_mlp_loss_grad(ik_mlp* m, const float* x, const float* t, int64_t n, doubl
 /* loss_grad followed by one Adam step (beta 0.9 / 0.999, eps 1e-8) with learning rate lr */
 int ik_mlp_train_step(ik_mlp* m, const float* x, const float* t, int64_t n, float lr, double* loss, int where);
 
-/* ---- timing of the hot kernels on the handle's stream (HIP events) ----------------------------- */
+/* ---- timing of the hot kernels on the handle's stream (HIP events) -----------------------------
+ * IK_KERNEL_ASSEMBLE_KR: the element kernel of a tangent, which forms R as well where both are asked for (ik_assemble,
+ * and every tangent of an EAS handle). IK_KERNEL_ASSEMBLE_R: residual-only element passes (ik_vector, the residual of a
+ * Newton iteration of the plain element); ik_assemble has none and adds nothing to it. The R gather is in neither. */
 enum { IK_KERNEL_ASSEMBLE_KR = 0, IK_KERNEL_ASSEMBLE_R = 1, IK_KERNEL_SPMV = 2, IK_KERNEL_MLP = 3,
        IK_KERNEL_GATHER_K = 4, IK_KERNEL_COUNT = 5 };
 int ik_timing_enable(ik_handle* h, int on);
